@@ -177,8 +177,7 @@ k_grid_rows_reg(SetDesc first, const SetDesc* __restrict__ sets, const int* __re
         for (int k = 1; k < RB; k++)
             if (rsr[k] <= e) r = k;
         float2* c = &tile[r * TS + pad_index(u_idx)];
-        atomicAdd(&c->x, v.x);
-        atomicAdd(&c->y, v.y);
+        lds_add(c, v.x, v.y);
         if constexpr (kUniform) atomicAdd(&cnt[r * N + u_idx], 1u);
         return ((edge >> r) & 1u) ? 1 : 2;
     };
@@ -808,8 +807,7 @@ k_grid_rows_wide(SetDesc first, const SetDesc* __restrict__ sets, const int* __r
         int r = 0;
         while (r + 1 < RB && rs[r + 1] <= e) r++;
         float2* c = &tile[r * TS + pad_index(u_idx)];
-        atomicAdd(&c->x, v.x);
-        atomicAdd(&c->y, v.y);
+        lds_add(c, v.x, v.y);
         if constexpr (kUniform) atomicAdd(&cnt[r * N + u_idx], 1u);
         const int row = r0 + r;
         return (row == 0 || row == H) ? 1 : 2;

@@ -155,6 +155,30 @@ __device__ __forceinline__ float2 select_pol2(float2 x0, float2 x1, int pol) {
     return make_float2((x0.x + x1.x) / 2.0f, (x0.y + x1.y) / 2.0f);  // I
 }
 
+// *p += (x, y) in LDS, atomically, in FP32.  gfx950 executes ds_add_f32 at
+// about 3 clocks per LANE, whatever the addresses (193 clocks per wavefront
+// instruction; ds_add_u32 9, ds_add_f64 21, measured with one 1024-thread
+// workgroup per CU), so two of them cost 389 clocks per wavefront.  A 64-bit
+// compare-and-swap of the whole cell costs 46 (79 with a third of the updates
+// in 128 cells) and rounds the same FP32 sums (768 channels x 256^2, 32896
+// baselines: 426 -> 355 us per batched call; 256 channels with 7 x 7
+// footprints 4.12 -> 1.34 ms).  The loop ends: a lane's swap
+// fails only when another lane's has succeeded in between.  p is 8-byte
+// aligned (float2).
+__device__ __forceinline__ void lds_add(float2* p, float x, float y) {
+    unsigned long long* q = (unsigned long long*)p;
+    unsigned long long old = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    for (;;) {
+        const float re = __uint_as_float((unsigned)old) + x;
+        const float im = __uint_as_float((unsigned)(old >> 32)) + y;
+        const unsigned long long sum =
+            ((unsigned long long)__float_as_uint(im) << 32) | __float_as_uint(re);
+        if (__hip_atomic_compare_exchange_strong(q, &old, sum, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP))
+            return;
+    }
+}
+
 __device__ __forceinline__ bool vis_ok(float2 v) {
     return !isnan(v.x) && !isnan(v.y) && (double)fabsf(v.x) < kMaxVis &&
            (double)fabsf(v.y) < kMaxVis;

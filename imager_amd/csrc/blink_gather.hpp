@@ -235,8 +235,7 @@ __device__ __forceinline__ int direct_walk(const SetDesc& sd, int64_t img, int c
                         *outside = true;
                         continue;
                     }
-                atomicAdd(&d->x, v.x);
-                atomicAdd(&d->y, v.y);
+                lds_add(d, v.x, v.y);
                 n_ok += (r == 0 || 2 * r == n) ? 1 : 2;
             }
             if (in2) {
@@ -246,8 +245,7 @@ __device__ __forceinline__ int direct_walk(const SetDesc& sd, int64_t img, int c
                         *outside = true;
                         continue;
                     }
-                atomicAdd(&d->x, v.x);
-                atomicAdd(&d->y, -v.y);
+                lds_add(d, v.x, -v.y);
                 n_ok += (r2 == 0 || 2 * r2 == n) ? 1 : 2;
             }
         }
@@ -327,8 +325,7 @@ __device__ __forceinline__ int kb_walk(const SetDesc& sd, int64_t img, int ch, i
                         continue;
                     }
                     const double w = yk[j] * wx;
-                    atomicAdd(&d->x, (float)((double)v.x * w));
-                    atomicAdd(&d->y, (float)((double)sgn * (double)v.y * w));
+                    lds_add(d, (float)((double)v.x * w), (float)((double)sgn * (double)v.y * w));
                 }
             }
         }

@@ -722,7 +722,7 @@ k_grid_tiles(GatherArgs g, const int* __restrict__ row_start, const uint32_t* __
              int overwrite, uint32_t* __restrict__ isums, int64_t img0) {
     extern __shared__ float4 tiles_lds4[];
     float2* tile = (float2*)tiles_lds4;                       // [rb][N]
-    float* cnt = (float*)(tile + (size_t)rb * n_pixels);      // [rb][N]
+    unsigned* cnt = (unsigned*)(tile + (size_t)rb * n_pixels);  // [rb][N]
     __shared__ int rs[kMaxTileRows + 1];
     __shared__ int red[kTileThreads / 64];
     const int n_rb = (n_pixels + rb - 1) / rb;
@@ -745,16 +745,15 @@ k_grid_tiles(GatherArgs g, const int* __restrict__ row_start, const uint32_t* __
     }
     for (int i = threadIdx.x; i < cells; i += blockDim.x) {
         tile[i] = make_float2(0.f, 0.f);
-        cnt[i] = 0.f;
+        cnt[i] = 0u;
     }
     __syncthreads();
     const int n_ok = gather_range<4>(g, img, ch, ent, rs[0], rs[nr], (int)threadIdx.x,
                                      (int)blockDim.x, [&](int e, int u_idx, float2 v) {
         const int r = row_of_entry(rs, nr, e);
         const int c = r * n_pixels + u_idx;
-        atomicAdd(&tile[c].x, v.x);
-        atomicAdd(&tile[c].y, v.y);
-        atomicAdd(&cnt[c], 1.0f);
+        lds_add(&tile[c], v.x, v.y);
+        atomicAdd(&cnt[c], 1u);
         return 1;
     });
     if (isums) {
@@ -766,7 +765,7 @@ k_grid_tiles(GatherArgs g, const int* __restrict__ row_start, const uint32_t* __
         const int r = i / n_pixels;
         if (overwrite) {
             grids[base + i] = tile[i];
-            if (counts) counts[base + i] = cnt[i];
+            if (counts) counts[base + i] = (float)cnt[i];
             continue;
         }
         if (rs[r + 1] == rs[r]) continue;  // empty row: nothing to add
@@ -775,7 +774,7 @@ k_grid_tiles(GatherArgs g, const int* __restrict__ row_start, const uint32_t* __
         o.x += t.x;
         o.y += t.y;
         grids[base + i] = o;
-        counts[base + i] += cnt[i];
+        counts[base + i] += (float)cnt[i];
     }
 }
 
@@ -839,8 +838,7 @@ k_grid_half_rows(GatherArgs g, const int* __restrict__ row_start,
     const int n_ok = gather_range<4>(g, img, ch, ent, rs[0], rs[nr], (int)threadIdx.x,
                                      (int)blockDim.x, [&](int e, int u_idx, float2 v) {
         const int r = row_of_entry(rs, nr, e);
-        atomicAdd(&tile[r * n + u_idx].x, v.x);
-        atomicAdd(&tile[r * n + u_idx].y, v.y);
+        lds_add(&tile[r * n + u_idx], v.x, v.y);
         if (uniform) atomicAdd(&cnt[r * n + u_idx], 1u);
         const int row = r0 + r;
         return (row == 0 || row == h) ? 1 : 2;
@@ -1185,8 +1183,7 @@ k_grid_rows_fft(SetDesc first, const SetDesc* __restrict__ sets, const int* __re
     const int n_ok = gather_range<4>(g, img, ch, ent, rs[0], rs[nr], (int)threadIdx.x,
                                      (int)blockDim.x, [&](int e, int u_idx, float2 v) {
         const int r = row_of_entry(rs, nr, e);
-        atomicAdd(&tile[r * n + u_idx].x, v.x);
-        atomicAdd(&tile[r * n + u_idx].y, v.y);
+        lds_add(&tile[r * n + u_idx], v.x, v.y);
         if (uniform) atomicAdd(&cnt[r * n + u_idx], 1u);
         // an entry stands for its mirror too, except in the self-conjugate rows
         // (0, and N/2 for even N), which list both
@@ -1649,8 +1646,8 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
                     int y;
                     if (!kb_cell(vp - mid + j, sgn, n, y)) continue;
                     const double w = yk[j] * wx;
-                    atomicAdd(&row[y].x, (float)((double)v.x * w));
-                    atomicAdd(&row[y].y, (float)((double)sgn * (double)v.y * w));
+                    lds_add(&row[y], (float)((double)v.x * w),
+                            (float)((double)sgn * (double)v.y * w));
                 }
             }
         }

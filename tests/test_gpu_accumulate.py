@@ -1,0 +1,69 @@
+"""LDS accumulation of gridded visibilities where many fall on one cell.
+
+The gridding kernels add complex values to LDS cells with a 64-bit
+compare-and-swap; every lane of a wavefront on one cell is its worst case.
+The FP32 sum of n values in any order lies within n 2^-24 sum |v| of the exact
+sum.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from imager_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _crowded(n_ant, n_pixels, cells, seed):
+    """An observation whose unflagged baselines share `cells` uv positions."""
+    o = synth.small(n_ant=n_ant, n_ch=1, n_t=1, n_pixels=n_pixels, seed=seed)
+    rng = np.random.Generator(np.random.PCG64(seed))
+    pick = rng.integers(0, cells, o.n_bl)
+    pos = rng.uniform(-0.2, 0.2, (2, cells)) * n_pixels
+    lam = synth.C_LIGHT / o.freq[0]
+    o.delta_u = o.delta_v = 1.0
+    o.u = (pos[0][pick] * lam).astype(np.float32)
+    o.v = (pos[1][pick] * lam).astype(np.float32)
+    return o
+
+
+@pytest.mark.parametrize("n_ant,n,cells", [(40, 64, 1), (65, 180, 2), (128, 128, 3), (256, 256, 1)])
+def test_crowded_cells(ctx, n_ant, n, cells):
+    import torch
+    from imager_amd import capi
+    o = _crowded(n_ant, n, cells, seed=n_ant + cells)
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.flags, o.freq)]
+    ref, cref, _ = oracle.gridding(o.vis.astype(np.complex64), o.n_ant, o.u, o.v, o.flags, o.freq,
+                                   1.0, 1.0, o.min_uv, n, "XX", precision="f64")
+    n_bl = o.n_bl
+    bound = n_bl * 2.0 ** -24 * np.abs(o.vis[0, 0, :, 0]).sum()
+    for algo in (capi.GRID_TILED, capi.GRID_ATOMIC):
+        grids = torch.zeros((1, 1, n, n), dtype=torch.complex64, device="cuda")
+        counts = torch.zeros((1, 1, n, n), dtype=torch.float32, device="cuda")
+        ctx.gridding(d[0], o.n_ant, 1, 1, d[1], d[2], d[3], d[4], 1.0, 1.0, o.min_uv, n, "XX", 0,
+                     grids, counts, algo=algo)
+        torch.cuda.synchronize()
+        assert np.array_equal(counts.cpu().numpy(), cref)
+        assert np.abs(grids.cpu().numpy() - ref).max() <= bound
+
+
+@pytest.mark.parametrize("n,transform", [(128, 0), (180, 0), (256, 0), (180, 2)])
+@pytest.mark.parametrize("direct", ["0", "1"])
+def test_crowded_cells_batched(ctx, monkeypatch, n, transform, direct):
+    import torch
+    from imager_amd import capi
+    monkeypatch.setenv("BLINK_DIRECT", direct)
+    o = _crowded(96, n, 2, seed=n)
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.w, o.flags, o.freq, o.cable)]
+    images = torch.empty((1, 1, n, n), dtype=torch.complex64, device="cuda")
+    ctx.image_batch([capi.make_set(d[0], o.n_ant, 1, 1, d[1], d[2], d[3], d[4], d[5], d[6], 3, 1.0,
+                                   1.0, o.min_uv, n, "XX", images, transform=transform)])
+    torch.cuda.synchronize()
+    ref, _ = oracle.run_f32(o.vis, o.n_ant, o.u, o.v, o.w, o.flags, o.freq, o.cable, True, True,
+                            1.0, 1.0, o.min_uv, n)
+    assert oracle.peak_normalised_error(images.cpu().numpy(), ref)[0] < 1e-5

@@ -324,31 +324,30 @@ int check_fft_size(blink_ctx* ctx, int n, FftPlan& plan) {
     return BLINK_OK;
 }
 
-// Rows then columns, optionally with the shift+scale epilogue on the column
-// store.  in -> out (in == out allowed).
-int fft2d(blink_ctx* ctx, const float* in, float* out, int n, int batch, int sign, bool shift,
-          const double* sums, hipStream_t stream) {
-    FftPlan plan;
-    int rc = check_fft_size(ctx, n, plan);
-    if (rc) return rc;
+// Images of one row / column launch pair of the stage transform: as many as
+// stay in the 256 MiB Infinity Cache between the two passes.
+constexpr int64_t kStageChunkBytes = 168ll << 20;
+int stage_chunk(int64_t n, int64_t batch) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>(batch, kStageChunkBytes / (8 * n * n)));
+}
+
+// Rows then columns of `batch` arrays, a chunk of them at a time.
+int fft2d(blink_ctx* ctx, StageFftArgs a, const FftPlan& plan, int batch, int sign,
+          hipStream_t stream) {
+    const int n = plan.n;
     const float* tw;
-    if ((rc = twiddles(ctx, n, &tw))) return rc;
-    LAUNCH("fft_rows", stream, launch_fft_rows(in, out, plan, (int64_t)batch * n, sign, tw, stream));
-    // The shifted store is fused into the in-place column pass when a
-    // workgroup can hold a column block and its shift partner; otherwise a
-    // separate shift+norm pass follows.
-    const bool fused = shift && cols_paired_fits(n);
-    ColArgs a{};
-    a.in = (const float2*)out;
-    a.out = (float2*)out;
-    a.in_img_stride = a.out_img_stride = (int64_t)n * n;
-    a.out_img_offset = 0;
-    a.paired = fused ? 1 : 0;
-    a.shift = fused ? 1 : 0;
-    a.sums = fused ? sums : nullptr;
-    a.n_ch = 1;
-    LAUNCH("fft_cols", stream, launch_fft_cols(a, plan, batch, sign, tw, stream));
-    if (shift && !fused) LAUNCH("shift_norm", stream, launch_shift_norm(out, n, n, batch, sums, batch, stream));
+    int rc = twiddles(ctx, n, &tw);
+    if (rc) return rc;
+    const int64_t gs = (int64_t)n * n;
+    const int chunk = stage_chunk(n, batch);
+    for (int i0 = 0; i0 < batch; i0 += chunk) {
+        const int cnt = std::min(chunk, batch - i0);
+        LAUNCH("fft_rows", stream, launch_stage_pass(true, a, plan, cnt, sign, tw, stream));
+        LAUNCH("fft_cols", stream, launch_stage_pass(false, a, plan, cnt, sign, tw, stream));
+        a.in += gs * cnt;
+        a.out += gs * cnt;
+        if (a.counts) a.grids += gs * cnt, a.counts += gs * cnt;
+    }
     return BLINK_OK;
 }
 
@@ -394,7 +393,7 @@ BLINK_API int blink_create(int device, blink_ctx** out) {
     g_lds_limit = std::min<int64_t>(lds, 160 * 1024) - 4 * 1024;
     g_lds_budget = g_lds_limit - 12 * 1024;
     if (set_kernel_attributes() != hipSuccess || set_batch_kernel_attributes() != hipSuccess ||
-        set_dft_kernel_attributes() != hipSuccess) {
+        set_dft_kernel_attributes() != hipSuccess || set_stage_kernel_attributes() != hipSuccess) {
         (void)hipGetLastError();
     }
     if (hipStreamCreateWithFlags(&ctx->capture_stream, hipStreamNonBlocking) != hipSuccess ||
@@ -717,7 +716,12 @@ BLINK_API int blink_fft2d_c2c(blink_ctx* ctx, const float* in, float* out, int n
     int rc = set_device(ctx);
     if (rc) return rc;
     if (batch == 0) return BLINK_OK;
-    return fft2d(ctx, in, out, n_pixels, batch, direction, false, nullptr, (hipStream_t)stream);
+    FftPlan plan;
+    if ((rc = check_fft_size(ctx, n_pixels, plan))) return rc;
+    StageFftArgs a{};
+    a.in = (const float2*)in;
+    a.out = (float2*)out;
+    return fft2d(ctx, a, plan, batch, direction, (hipStream_t)stream);
 }
 
 // ------------------------------------------------------------------ (d)
@@ -760,18 +764,19 @@ BLINK_API int blink_image(blink_ctx* ctx, float* grids, float* counts, int n_pix
     if ((rc = check_fft_size(ctx, n_pixels, plan))) return rc;
     if (n_images == 0) return BLINK_OK;
     hipStream_t s = (hipStream_t)stream;
+    // partial count sums and row marks of a chunk's images (the chunks follow
+    // one another on the stream; at most a partial and a mark per row)
+    const size_t rows = (size_t)n_pixels * stage_chunk(n_pixels, n_images);
     void* sums;
-    if ((rc = ctx_scratch(ctx, "image_sums", sizeof(double) * (size_t)n_images, &sums))) return rc;
-    const int64_t gs = (int64_t)n_pixels * n_pixels;
-    LAUNCH("vector_sum", s, launch_vector_sum(counts, gs, n_images, (double*)sums, s));
-    if ((rc = fft2d(ctx, grids, images, n_pixels, n_images, BLINK_FFT_BACKWARD, true,
-                    (const double*)sums, s)))
-        return rc;
-    if (zero_grids) {
-        LAUNCH("zero", s, launch_zero(grids, (int64_t)sizeof(float) * 2 * gs * n_images, s));
-        LAUNCH("zero", s, launch_zero(counts, (int64_t)sizeof(float) * gs * n_images, s));
-    }
-    return BLINK_OK;
+    if ((rc = ctx_scratch(ctx, "image_sums", (sizeof(double) + 1) * rows, &sums))) return rc;
+    StageFftArgs a{};
+    a.in = a.grids = (float2*)grids;
+    a.out = (float2*)images;
+    a.counts = counts;
+    a.part = (double*)sums;
+    a.used = (unsigned char*)sums + sizeof(double) * rows;
+    a.clear = zero_grids;
+    return fft2d(ctx, a, plan, n_images, BLINK_FFT_BACKWARD, s);
 }
 
 BLINK_API int blink_image_averaging(blink_ctx* ctx, const float* images, int64_t image_size,

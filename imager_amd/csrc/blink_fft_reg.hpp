@@ -74,7 +74,7 @@ struct TwSplit64 {  // two 64-entry tables: w(m) = lo[m % 64] * hi[m / 64], N <=
 // the same passes.
 template <int N, int L, bool kBlock = (L > 64)>
 struct RegFft {
-    static constexpr int V = N / L;
+    static constexpr int kN = N, kL = L, V = N / L;
     static constexpr RegRadices RAD = reg_radices(N, L);
     static_assert(RAD.n_pass > 0, "unsupported size / lane count");
 

@@ -43,40 +43,11 @@ __host__ __device__ constexpr size_t tw_lds_bytes(int n) {
 
 // ------------------------------------------------------------------ helpers
 
-__global__ void k_zero(float4* __restrict__ p, int64_t n_vec) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_vec; i += stride)
-        p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-}
-
-__global__ void k_zero_tail(float* __restrict__ p, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.f;
-}
-
 static unsigned grid_for(int64_t work, int block, int max_blocks) {
     int64_t b = (work + block - 1) / block;
     if (b < 1) b = 1;
     if (b > max_blocks) b = max_blocks;
     return (unsigned)b;
-}
-
-hipError_t launch_zero(void* ptr, int64_t bytes, hipStream_t stream) {
-    if (bytes <= 0) return hipSuccess;
-    float* f = (float*)ptr;
-    const int64_t n_float = bytes / 4;
-    const bool aligned = ((uintptr_t)ptr % 16) == 0;
-    const int64_t n_vec = aligned ? n_float / 4 : 0;
-    if (n_vec > 0) {
-        hipLaunchKernelGGL(k_zero, dim3(grid_for(n_vec, 256, 8192)), dim3(256), 0, stream,
-                           (float4*)f, n_vec);
-    }
-    const int64_t tail = n_float - n_vec * 4;
-    if (tail > 0) {
-        hipLaunchKernelGGL(k_zero_tail, dim3(grid_for(tail, 256, 1 << 20)), dim3(256), 0, stream,
-                           f + n_vec * 4, tail);
-    }
-    return hipGetLastError();
 }
 
 // ----------------------------------------------------- (a) phase corrections
@@ -933,114 +904,6 @@ hipError_t launch_uniform_weight(float* grids, const float* counts, int64_t n_ce
     return hipGetLastError();
 }
 
-// --------------------------------------------------------------- (c) FFT
-
-// Row pass: each team loads one row from global memory, transforms it in LDS
-// and writes it back (in == out allowed: a row is fully read before written).
-template <int S, bool kBlockTeam>
-__global__ void __launch_bounds__(kFftThreads)
-k_fft_rows(const float2* __restrict__ in, float2* __restrict__ out, FftPlan plan, int team,
-           int64_t n_rows, const float2* __restrict__ tw) {
-    extern __shared__ float4 rows_lds4[];
-    float2* lds = (float2*)rows_lds4;
-    const int n = plan.n;
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* buf = lds + (size_t)t_id * 2 * n;
-    float2* tmp = buf + n;
-    const int64_t row = (int64_t)blockIdx.x * teams + t_id;
-    const bool active = row < n_rows;
-    if (active) {
-        const float2* src = in + row * n;
-        for (int i = lane; i < n; i += team) buf[i] = src[i];
-    }
-    team_sync<kBlockTeam>();
-    if (kBlockTeam || active) {
-        const float2* res = fft_row<S, kBlockTeam>(buf, tmp, plan, tw, lane, team);
-        if (active) {
-            float2* dst = out + row * n;
-            for (int i = lane; i < n; i += team) dst[i] = res[i];
-        }
-    }
-}
-
-// Column pass.  A workgroup owns a set of columns: W contiguous columns
-// starting at c0 and, when `paired` is set, the W columns starting at
-// c0 + N/2 as well (then the fft_shift maps the set onto itself, which makes
-// an in-place shifted store safe).  The columns are loaded into an LDS tile
-// (transposed, one padded LDS row per column), transformed by the teams, and
-// stored row by row, optionally shifted and scaled.
-template <int S, bool kBlockTeam>
-__global__ void __launch_bounds__(kFftThreads)
-k_fft_cols(ColArgs a, FftPlan plan, int team, const float2* __restrict__ tw) {
-    extern __shared__ float4 cols_lds4[];
-    const int n = plan.n;
-    const int ld = n + 1;  // padded LDS row
-    const int wt = a.paired ? 2 * a.width : a.width;
-    float2* tile = (float2*)cols_lds4;                 // [wt][ld]
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* tmp = tile + (size_t)wt * ld + (size_t)t_id * n;
-    const int span = a.paired ? n / 2 : n;
-    const int n_cb = (span + a.width - 1) / a.width;
-    const int cb = blockIdx.x % n_cb;
-    const int64_t img = blockIdx.x / n_cb;
-    const int c0 = cb * a.width;
-    const int w_here = min(a.width, span - c0);
-    const float2* src = a.in + img * a.in_img_stride;
-    const int64_t oimg = a.out_img_offset + img;
-    float2* dst = a.out + img * a.out_img_stride;
-    const int* rs = a.row_start ? a.row_start + (oimg % a.n_ch) * (int64_t)(n + 1) : nullptr;
-    const uint32_t* isums = a.isums;
-
-    // load: element (r, w) of the set; columns c0+w and c0+N/2+w
-    const int total = n * wt;
-    for (int i = threadIdx.x; i < total; i += blockDim.x) {
-        const int r = i / wt;
-        const int wl = i % wt;
-        const int half = wl / a.width;  // 0 or 1
-        const int w = wl % a.width;
-        float2 v = make_float2(0.f, 0.f);
-        if (w < w_here && (!rs || rs[r + 1] != rs[r]))
-            v = src[(int64_t)r * n + c0 + half * (n / 2) + w];
-        tile[(size_t)wl * ld + r] = v;
-    }
-    __syncthreads();
-    const int ncols = a.paired ? 2 * w_here : w_here;
-    const int rounds = kBlockTeam ? ncols : (ncols + teams - 1) / teams;
-    for (int k = 0; k < rounds; k++) {
-        const int cidx = kBlockTeam ? k : k * teams + t_id;
-        if (!kBlockTeam && cidx >= ncols) break;
-        const int wl = a.paired ? (cidx < w_here ? cidx : a.width + (cidx - w_here)) : cidx;
-        float2* col = tile + (size_t)wl * ld;
-        const float2* res = fft_row<S, kBlockTeam>(col, tmp, plan, tw, lane, team);
-        if (res != col) {
-            for (int i = lane; i < n; i += team) col[i] = res[i];
-            team_sync<kBlockTeam>();
-        }
-    }
-    __syncthreads();
-    float scale = 1.0f;
-    if (a.sums) scale = (float)(1.0 / a.sums[oimg]);
-    else if (isums) scale = (float)(1.0 / (double)isums[oimg]);
-    const bool do_scale = a.sums || isums;
-    for (int i = threadIdx.x; i < total; i += blockDim.x) {
-        const int r = i / wt;
-        const int wl = i % wt;
-        const int half = wl / a.width;
-        const int w = wl % a.width;
-        if (w >= w_here) continue;
-        const int c = c0 + half * (n / 2) + w;
-        float2 v = tile[(size_t)wl * ld + r];
-        if (do_scale) v = cscale(v, scale);
-        const int orow = a.shift ? shift_index(r, n) : r;
-        const int ocol = a.shift ? shift_index(c, n) : c;
-        dst[(int64_t)orow * n + ocol] = v;
-    }
-}
-
 // ---------------------------------------------- (d) sums, shift+norm, averaging
 
 // sums[img] = sum of values of one image, in double.  One block per image.
@@ -1343,84 +1206,6 @@ bool make_fft_plan(int n, FftPlan& plan) {
         rem /= r;
     }
     return true;
-}
-
-template <int S>
-static hipError_t fft_rows_t(const float* in, float* out, const FftPlan& plan, int64_t n_rows,
-                             const float* tw, hipStream_t stream) {
-    const int n = plan.n;
-    const int team = fft_team_for(n);
-    if (team == kFftThreads) {
-        const size_t lds = sizeof(float2) * 2 * (size_t)n;
-        if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-        hipLaunchKernelGGL((k_fft_rows<S, true>), dim3((unsigned)n_rows), dim3(kFftThreads), lds,
-                           stream, (const float2*)in, (float2*)out, plan, team, n_rows,
-                           (const float2*)tw);
-    } else {
-        const int teams = kFftThreads / team;
-        const size_t lds = sizeof(float2) * 2 * (size_t)n * teams;
-        if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-        const unsigned blocks = (unsigned)((n_rows + teams - 1) / teams);
-        hipLaunchKernelGGL((k_fft_rows<S, false>), dim3(blocks), dim3(kFftThreads), lds, stream,
-                           (const float2*)in, (float2*)out, plan, team, n_rows, (const float2*)tw);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_fft_rows(const float* in, float* out, const FftPlan& plan, int64_t n_rows,
-                           int sign, const float* tw, hipStream_t stream) {
-    if (n_rows == 0) return hipSuccess;
-    return sign > 0 ? fft_rows_t<1>(in, out, plan, n_rows, tw, stream)
-                    : fft_rows_t<-1>(in, out, plan, n_rows, tw, stream);
-}
-
-// Column width: the largest divisor of the column span that fits in the LDS
-// budget next to the team scratch rows, at most kMaxColWidth.
-static int col_width_for(int n, int teams, bool paired) {
-    const int64_t budget = g_lds_budget - (int64_t)teams * n * 8;
-    int w = (int)(budget / ((int64_t)(n + 1) * 8 * (paired ? 2 : 1)));
-    w = std::min(w, kMaxColWidth);
-    const int span = paired ? n / 2 : n;
-    w = std::max(1, std::min(w, span));
-    while (span % w) w--;
-    return w;
-}
-
-bool cols_paired_fits(int n) {
-    const int team = fft_team_for(n);
-    const int teams = team == kFftThreads ? 1 : kFftThreads / team;
-    const size_t lds = sizeof(float2) * (2 * (size_t)(n + 1) + (size_t)teams * n);
-    return n % 2 == 0 && lds_fits(lds);
-}
-
-template <int S>
-static hipError_t fft_cols_t(ColArgs a, const FftPlan& plan, int n_images, const float* tw,
-                             hipStream_t stream) {
-    const int n = plan.n;
-    const int team = fft_team_for(n);
-    const bool block_team = team == kFftThreads;
-    const int teams = block_team ? 1 : kFftThreads / team;
-    a.width = col_width_for(n, teams, a.paired != 0);
-    const int span = a.paired ? n / 2 : n;
-    const int n_cb = (span + a.width - 1) / a.width;
-    const int wt = a.paired ? 2 * a.width : a.width;
-    const size_t lds = sizeof(float2) * ((size_t)wt * (n + 1) + (size_t)teams * n);
-    if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-    const dim3 grid((unsigned)((int64_t)n_cb * n_images));
-    if (block_team)
-        hipLaunchKernelGGL((k_fft_cols<S, true>), grid, dim3(kFftThreads), lds, stream, a, plan,
-                           team, (const float2*)tw);
-    else
-        hipLaunchKernelGGL((k_fft_cols<S, false>), grid, dim3(kFftThreads), lds, stream, a, plan,
-                           team, (const float2*)tw);
-    return hipGetLastError();
-}
-
-hipError_t launch_fft_cols(const ColArgs& a, const FftPlan& plan, int n_images, int sign,
-                           const float* tw, hipStream_t stream) {
-    if (n_images == 0) return hipSuccess;
-    return sign > 0 ? fft_cols_t<1>(a, plan, n_images, tw, stream)
-                    : fft_cols_t<-1>(a, plan, n_images, tw, stream);
 }
 
 int grid_rows_tile_rows(int n) {
@@ -1888,14 +1673,6 @@ hipError_t set_kernel_attributes() {
         hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
         if (r != hipSuccess && e == hipSuccess) e = r;
     };
-    set((const void*)k_fft_rows<1, true>);
-    set((const void*)k_fft_rows<1, false>);
-    set((const void*)k_fft_rows<-1, true>);
-    set((const void*)k_fft_rows<-1, false>);
-    set((const void*)k_fft_cols<1, true>);
-    set((const void*)k_fft_cols<1, false>);
-    set((const void*)k_fft_cols<-1, true>);
-    set((const void*)k_fft_cols<-1, false>);
     set((const void*)k_grid_rows_kb<1, true, false>);
     set((const void*)k_grid_rows_kb<1, false, false>);
     set((const void*)k_grid_rows_kb<1, true, true>);

@@ -116,19 +116,18 @@ __device__ __forceinline__ SetDesc set_of(const SetDesc& first, const SetDesc* _
     else return sets[img_set[gi]];
 }
 
-struct ColArgs {
-    const float2* in;          // [img][N][N], images of this launch
-    float2* out;               // [img][N][N], images of this launch
-    int64_t in_img_stride;     // elements
-    int64_t out_img_stride;
-    int64_t out_img_offset;    // global index of the launch's first image (sums, plan)
-    int width;                 // W, set by the launcher
-    int paired;                // also load columns c0 + N/2 .. (+W)
-    int shift;                 // fft_shift on store
-    const double* sums;        // scale (float)(1/sums[img]) on store, or null
-    const uint32_t* isums;     // integer sums alternative, or null
-    const int* row_start;      // plan rows: skip empty rows on load, or null
-    int n_ch;
+// Operands of the stage path's 2-D transform (blink_image.hip), for the images
+// of one launch.  counts == nullptr: a plain transform in -> out.  Otherwise
+// in = grids, the columns and rows are shifted, the images are scaled by
+// 1 / (sum of the counts), and with `clear` grids and counts are zeroed.
+struct StageFftArgs {
+    const float2* in;          // [img][N][N]
+    float2* out;               // [img][N][N] (== in allowed for a plain transform)
+    float2* grids;             // [img][N][N]
+    float* counts;             // [img][N][N]
+    double* part;              // [img][stage_fft_parts] partial count sums
+    unsigned char* used;       // [img][N] rows that hold a non-zero cell
+    int clear;
 };
 
 // Compute units of the current device (queried once per process: every device
@@ -136,12 +135,9 @@ struct ColArgs {
 int device_cu_count();
 
 bool make_fft_plan(int n, FftPlan& plan);
-// Whether the in-place (paired) shifted column pass fits in LDS for side n.
-bool cols_paired_fits(int n);
 int grid_rows_tile_rows(int n);
 hipError_t set_kernel_attributes();
 
-hipError_t launch_zero(void* ptr, int64_t bytes, hipStream_t stream);
 hipError_t launch_phase_correct(float* vis, int n_ant, int n_ch, int n_t, const float* w_m,
                                 const double* cable_m, const double* freq_hz, unsigned which,
                                 hipStream_t stream);
@@ -176,10 +172,12 @@ hipError_t launch_grid_tiles(const GatherArgs& g, const int* row_start, const ui
                              int64_t img0 = 0);
 hipError_t launch_uniform_weight(float* grids, const float* counts, int64_t n_cells,
                                  hipStream_t stream);
-hipError_t launch_fft_rows(const float* in, float* out, const FftPlan& plan, int64_t n_rows,
-                           int sign, const float* tw, hipStream_t stream);
-hipError_t launch_fft_cols(const ColArgs& a, const FftPlan& plan, int n_images, int sign,
-                           const float* tw, hipStream_t stream);
+// One pass (rows, then columns) of the 2-D transform of n_img images;
+// stage_fft_parts(n, n_img) partial count sums per image.
+hipError_t launch_stage_pass(bool rows, const StageFftArgs& a, const FftPlan& plan, int64_t n_img,
+                             int sign, const float* tw, hipStream_t stream);
+int stage_fft_parts(int n, int64_t n_img);
+hipError_t set_stage_kernel_attributes();
 hipError_t launch_vector_sum(const float* values, int64_t image_size, int n_images, double* sums,
                              hipStream_t stream);
 hipError_t launch_shift_norm(float* images, int nx, int ny, int n_images, const double* sums,

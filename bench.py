@@ -89,7 +89,7 @@ def algorithmic_bytes(kernel: str, n_bl: int, n_pix: int, n_img: int) -> float |
     reported as an effective bandwidth, not as a roofline fraction."""
     g = 16.0 * n_bl + 12.0 * n_pix * n_pix
     f = 16.0 * n_pix * n_pix
-    if kernel in ("grid_rows_fft", "grid_tiles"):
+    if kernel == "grid_rows_fft":
         return g * n_img
     if kernel == "grid_half_rows":   # DFT transform: half plane, complex only
         return (16.0 * n_bl + 8.0 * (n_pix // 2 + 1) * n_pix) * n_img
@@ -557,12 +557,12 @@ def main():
     direct = "direct_prep" in prof   # the direct row pass ran (no plan)
     if N is not None:
         stats = plan_stats(obs, transposed=args.transform == "fft")
-        n_launch = max(prof.get("grid_rows_fft", (0, 0))[0], prof.get("grid_tiles", (0, 0))[0],
+        n_launch = max(prof.get("grid_rows_fft", (0, 0))[0],
                        prof.get("grid_half_rows", (0, 0))[0],
                        prof.get("grid_rows_kb", (0, 0))[0]) // args.steps
         chunk = -(-job["images_per_step"] // max(n_launch, 1))
         imgs_per_launch = chunk if dom in ("grid_rows_fft", "grid_rows_kb", "fft_cols",
-                                           "grid_tiles", "grid_half_rows", "dft_rows",
+                                           "grid_half_rows", "dft_rows",
                                            "dft_cols") \
             else job["images_per_step"]
         avg_s = kernels[dom]["avg_ms"] * 1e-3

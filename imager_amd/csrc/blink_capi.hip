@@ -516,25 +516,6 @@ BLINK_API int blink_uv_cells(blink_ctx* ctx, const float* u_m, const float* v_m,
     return BLINK_OK;
 }
 
-// Builds the per-channel row plan into context scratch.
-static int build_plan(blink_ctx* ctx, const float* u_m, const float* v_m, const int* flags,
-                      int n_bl, const double* freq_hz, int n_ch, double du, double dv,
-                      double min_uv, int n_pixels, int** row_start, uint32_t** entries,
-                      hipStream_t stream, const char* tag) {
-    void *rs, *en;
-    int rc;
-    std::string a = std::string("plan_rows") + tag, b = std::string("plan_entries") + tag;
-    if ((rc = ctx_scratch(ctx, a.c_str(), sizeof(int) * (size_t)n_ch * (n_pixels + 1), &rs))) return rc;
-    if ((rc = ctx_scratch(ctx, b.c_str(), sizeof(uint32_t) * 2 * (size_t)n_ch * std::max(n_bl, 1), &en)))
-        return rc;
-    LAUNCH("plan_rows", stream,
-           launch_plan_rows(u_m, v_m, flags, n_bl, freq_hz, n_ch, du, dv, min_uv, n_pixels,
-                            (int*)rs, (uint32_t*)en, stream));
-    *row_start = (int*)rs;
-    *entries = (uint32_t*)en;
-    return BLINK_OK;
-}
-
 BLINK_API int blink_gridding(blink_ctx* ctx, const float* vis, int n_ant, int n_ch, int n_t,
                              const float* u_m, const float* v_m, const int* bl_flags,
                              const double* freq_hz, double delta_u, double delta_v, double min_uv,
@@ -553,26 +534,15 @@ BLINK_API int blink_gridding(blink_ctx* ctx, const float* vis, int n_ant, int n_
     if ((rc = set_device(ctx))) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int n_bl = n_ant * (n_ant + 1) / 2;
-    const int n_img = n_ch * n_t;
-    if (algo == BLINK_GRID_ATOMIC) {
-        LAUNCH("grid_atomic", s,
-               launch_grid_atomic(vis, n_ant, n_ch, n_t, u_m, v_m, bl_flags, freq_hz, delta_u,
-                                  delta_v, min_uv, n_pixels, pol, grids, counts, s));
-    } else {
-        int* rs;
-        uint32_t* en;
-        if ((rc = build_plan(ctx, u_m, v_m, bl_flags, n_bl, freq_hz, n_ch, delta_u, delta_v, min_uv,
-                             n_pixels, &rs, &en, s, "")))
-            return rc;
-        GatherArgs g{};
-        g.vis = (const float4*)vis;
-        g.freq_hz = freq_hz;
-        g.corrections = 0;
-        g.pol = pol;
-        g.n_bl = n_bl;
-        g.n_ch = n_ch;
-        LAUNCH("grid_tiles", s, launch_grid_tiles(g, rs, en, n_img, n_pixels, grids, counts, s));
-    }
+    const int64_t n_img = (int64_t)n_ch * n_t;
+    const bool slabs = algo == BLINK_GRID_TILED && stage_grid_slabs(n_pixels, n_bl, n_img);
+    void* cells = nullptr;
+    if (slabs && (rc = ctx_scratch(ctx, "grid_cells",
+                                   sizeof(uint32_t) * (size_t)n_ch * stage_cell_stride(n_bl), &cells)))
+        return rc;
+    LAUNCH(slabs ? "grid_slabs" : "grid_atomic", s,
+           launch_stage_grid(vis, n_ant, n_ch, n_t, u_m, v_m, bl_flags, freq_hz, delta_u, delta_v,
+                             min_uv, n_pixels, pol, (uint32_t*)cells, grids, counts, s));
     if (weighting == BLINK_WEIGHTING_UNIFORM)
         LAUNCH("uniform_weight", s,
                launch_uniform_weight(grids, counts, (int64_t)n_img * n_pixels * n_pixels, s));

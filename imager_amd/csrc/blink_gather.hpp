@@ -93,7 +93,8 @@ struct GatherBatch {
 struct CellUnit {
     double wl, r_wl, r_du, r_dv, ku, kv;
     bool fast;
-    __device__ __forceinline__ CellUnit(double freq_hz, const SetDesc& sd) {
+    template <class Set>  // (SetDesc, or any holder of du and dv)
+    __device__ __forceinline__ CellUnit(double freq_hz, const Set& sd) {
 #pragma clang fp contract(off)
         wl = wavelength_of(freq_hz);
         r_wl = 1.0 / wl;
@@ -112,8 +113,9 @@ struct CellUnit {
 // zero, huge, infinite or NaN coordinate or cell size) take the IEEE division.
 // Almost every cell is decided first by one product per coordinate
 // (round_quotient_fast), which gives the same integers.
-__device__ __forceinline__ bool plan_cell(float u_m, float v_m, const CellUnit& cu,
-                                          const SetDesc& sd, int& up, int& vp) {
+template <class Set>  // (SetDesc, or any holder of du, dv, min_uv and n_pixels)
+__device__ __forceinline__ bool plan_cell(float u_m, float v_m, const CellUnit& cu, const Set& sd,
+                                          int& up, int& vp) {
 #pragma clang fp contract(off)
     if (sd.min_uv == -INFINITY) {
         const double um = (double)u_m, vm = (double)v_m;

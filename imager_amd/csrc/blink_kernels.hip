@@ -204,47 +204,251 @@ hipError_t launch_uv_max(const float* u_m, const float* v_m, const int* flags, i
 
 // ------------------------------------------------ (b) gridding, plain atomic
 
-// One thread per (t, ch, bl), FP32 global atomics (the plain path, in the
-// shape of gridding_kernel, src/gpu/gridding_gpu.cpp:58-124, with per-image
-// counts as the CPU path keeps them, src/pacer_imager.cpp:387,408).
-__global__ void k_grid_atomic(const float4* __restrict__ vis, int n_bl, int n_ch, int64_t n_rec,
-                              const float* __restrict__ u_m, const float* __restrict__ v_m,
-                              const int* __restrict__ flags, const double* __restrict__ freq_hz,
-                              double du, double dv, double min_uv, int n_pixels, int pol,
-                              float* __restrict__ grids, float* __restrict__ counts) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t gs = (int64_t)n_pixels * n_pixels;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_rec; i += stride) {
-        const int bl = (int)(i % n_bl);
-        const int64_t img = i / n_bl;
-        const int ch = (int)(img % n_ch);
-        if (flags[bl]) continue;
-        const float2 val = select_pol(vis[2 * i], vis[2 * i + 1], pol);
-        if (!vis_ok(val)) continue;
-        int up, vp;
-        if (!cell_of(u_m[bl], v_m[bl], wavelength_of(freq_hz[ch]), du, dv, min_uv, n_pixels, up, vp))
-            continue;
-        const int64_t p = img * gs + (int64_t)wrap_index(vp, n_pixels) * n_pixels + wrap_index(up, n_pixels);
-        const int64_t q = img * gs + (int64_t)wrap_index(-vp, n_pixels) * n_pixels + wrap_index(-up, n_pixels);
-        unsafeAtomicAdd(&grids[2 * p], val.x);
-        unsafeAtomicAdd(&grids[2 * p + 1], val.y);
-        unsafeAtomicAdd(&counts[p], 1.0f);
-        unsafeAtomicAdd(&grids[2 * q], val.x);
-        unsafeAtomicAdd(&grids[2 * q + 1], -val.y);
-        unsafeAtomicAdd(&counts[q], 1.0f);
+// Inputs of the stage gridding kernels.
+struct StageGrid {
+    const float2* vis;  // [img][bl][4]
+    const float* u_m;
+    const float* v_m;
+    const int* flags;
+    const double* freq_hz;
+    double du, dv, min_uv;
+    int n_bl, n_ch, n_pixels, pol;
+    float2* grids;
+    float* counts;
+};
+
+// The selected polarisation of record (img, bl).
+__device__ __forceinline__ float2 stage_value(const StageGrid& g, int64_t img, int bl) {
+    const float2* rec = g.vis + 4 * (img * g.n_bl + bl);
+    const int p0 = g.pol == 1 ? 3 : (g.pol == 3 ? 1 : 0);
+    const float2 x0 = rec[p0];
+    const float2 x1 = g.pol >= 2 ? rec[g.pol == 3 ? 2 : 3] : make_float2(0.f, 0.f);
+    return select_pol2(x0, x1, g.pol);
+}
+
+// FP32 global atomics, one baseline per thread and image blockIdx.y (per-image
+// counts as the CPU path keeps them, src/pacer_imager.cpp:387,408).  The
+// two components of a cell are added by neighbouring lanes of one instruction,
+// so that a cell is one request of the memory side that performs the atomics.
+__global__ void __launch_bounds__(256)
+k_grid_atomic(StageGrid g, int64_t n_img) {
+    const int bl = (int)(blockIdx.x * 256 + threadIdx.x), n = g.n_pixels;
+    const int lane = threadIdx.x & 63;
+    for (int64_t img = blockIdx.y; img < n_img; img += gridDim.y) {
+        const double nu = g.freq_hz[img % g.n_ch];
+        float2 val = make_float2(0.f, 0.f);
+        int64_t p = -1, q = -1;
+        if (bl < g.n_bl && !g.flags[bl]) {
+            val = stage_value(g, img, bl);
+            int up, vp;
+            if (vis_ok(val) && plan_cell(g.u_m[bl], g.v_m[bl], CellUnit(nu, g), g, up, vp)) {
+                const int64_t base = img * (int64_t)n * n;
+                p = base + (int64_t)wrap_index(vp, n) * n + wrap_index(up, n);
+                q = base + (int64_t)wrap_index(-vp, n) * n + wrap_index(-up, n);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {  // lanes 2 j, 2 j + 1 add cell j + 32 k of the wave
+            const int from = (lane >> 1) + 32 * k;
+            const float re = __shfl(val.x, from, 64), im = __shfl(val.y, from, 64);
+            const int64_t pc = __shfl(p, from, 64), qc = __shfl(q, from, 64);
+            if (pc < 0) continue;
+            const int odd = lane & 1;
+            unsafeAtomicAdd((float*)g.grids + 2 * pc + odd, odd ? im : re);
+            unsafeAtomicAdd((float*)g.grids + 2 * qc + odd, odd ? -im : re);
+        }
+        if (p >= 0) {
+            unsafeAtomicAdd(&g.counts[p], 1.0f);
+            unsafeAtomicAdd(&g.counts[q], 1.0f);
+        }
     }
 }
 
-hipError_t launch_grid_atomic(const float* vis, int n_ant, int n_ch, int n_t, const float* u_m,
-                              const float* v_m, const int* flags, const double* freq_hz, double du,
-                              double dv, double min_uv, int n_pixels, int pol, float* grids,
-                              float* counts, hipStream_t stream) {
+// Cells of every (channel, baseline), packed row << 16 | column (kNoCell where
+// not gridded), channels `stride` apart (a multiple of 4; the tail is kNoCell).
+__global__ void __launch_bounds__(256)
+k_stage_cells(StageGrid g, int stride, uint32_t* __restrict__ cells) {
+    const int bl = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (bl >= stride) return;
+    for (int ch = blockIdx.y; ch < g.n_ch; ch += gridDim.y) {
+        uint32_t packed = kNoCell;
+        int up, vp;
+        if (bl < g.n_bl && !g.flags[bl] &&
+            plan_cell(g.u_m[bl], g.v_m[bl], CellUnit(g.freq_hz[ch], g), g, up, vp))
+            packed = ((uint32_t)wrap_index(vp, g.n_pixels) << 16) |
+                     (uint32_t)wrap_index(up, g.n_pixels);
+        cells[(int64_t)ch * stride + bl] = packed;
+    }
+}
+
+// Slabs of the Hermitian half plane in LDS.  Workgroup (slab, image) owns the
+// rows r = slab, slab + S, .. of 0 .. N/2 (interleaved, so that the rows the
+// array reaches are spread evenly).  It walks the cells of
+// its channel, kSlabChunk at a time, and queues in LDS the baselines whose
+// cell or mirrored cell falls in its rows; then the queue is gridded with full
+// wavefronts (a slab's records are 1 / S of all: reading them where they are
+// found left most lanes waiting for a few).  At the end it adds its non-empty
+// cells, and their conjugates at the mirrored cells, to the global grid (no
+// other workgroup touches either).
+constexpr int kSlabThreads = 1024, kSlabVec = 3;
+constexpr int kSlabChunk = kSlabThreads * 4 * kSlabVec;  // (256 antennas: 3 chunks)
+static_assert(kSlabChunk <= 65536, "queue entries are 16-bit offsets");
+__global__ void __launch_bounds__(kSlabThreads)
+k_grid_slabs(StageGrid g, int S, int rows, int stride, const uint32_t* __restrict__ cells) {
+    extern __shared__ float4 slabs_lds4[];
+    const int n = g.n_pixels, h = n / 2;
+    float2* tile = (float2*)slabs_lds4;                      // [rows][n]
+    unsigned* cnt = (unsigned*)(tile + (size_t)rows * n);    // [rows][n]
+    unsigned short* queue = (unsigned short*)(cnt + (size_t)rows * n);  // [kSlabChunk]
+    __shared__ int n_queued;
+    const int slab = (int)(blockIdx.x % (unsigned)S);
+    const int64_t img = blockIdx.x / (unsigned)S;
+    // r / S of a row r < 2^13 (exact: r and S are below 2^13)
+    const unsigned inv = ((1u << 26) + (unsigned)S - 1) / (unsigned)S;
+    auto div_s = [&](int r) { return (int)(((uint64_t)r * inv) >> 26); };
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t* cl = cells + (img % g.n_ch) * stride;
+    auto load = [&](int base, uint4(&p)[kSlabVec]) {
+#pragma unroll
+        for (int k = 0; k < kSlabVec; k++) {
+            const int b = base + 4 * (tid + k * kSlabThreads);
+            p[k] = b < stride ? *(const uint4*)&cl[b]
+                              : make_uint4(kNoCell, kNoCell, kNoCell, kNoCell);
+        }
+    };
+    uint4 p[kSlabVec];
+    load(0, p);
+    for (int i = tid; i < rows * n; i += kSlabThreads) {
+        tile[i] = make_float2(0.f, 0.f);
+        cnt[i] = 0u;
+    }
+    for (int base = 0; base < stride; base += kSlabChunk) {
+        if (tid == 0) n_queued = 0;
+        __syncthreads();
+        unsigned keep = 0;
+#pragma unroll
+        for (int k = 0; k < kSlabVec; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t c = j == 0 ? p[k].x : j == 1 ? p[k].y : j == 2 ? p[k].z : p[k].w;
+                const int r0 = (int)(c >> 16), r = r0 <= h ? r0 : n - r0;
+                if (c != kNoCell && r - S * div_s(r) == slab) keep |= 1u << (4 * k + j);
+            }
+        int before = __popc(keep);
+        const int own = before;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(before, o, 64);
+            if (lane >= o) before += t;
+        }
+        int at = 0;
+        if (lane == 63) at = atomicAdd(&n_queued, before);
+        at = __shfl(at, 63, 64) + before - own;
+#pragma unroll
+        for (int k = 0; k < kSlabVec; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if ((keep >> (4 * k + j)) & 1u)
+                    queue[at++] = (unsigned short)(4 * (tid + k * kSlabThreads) + j);
+        __syncthreads();
+        load(base + kSlabChunk, p);  // the next chunk, while the queue is gridded
+        const int nq = n_queued;
+        for (int i = tid; i < nq; i += kSlabThreads) {
+            const int bl = base + queue[i];
+            const uint32_t cell = cl[bl];
+            const float2 v = stage_value(g, img, bl);
+            if (!vis_ok(v)) continue;
+            const int r = (int)(cell >> 16), c = (int)(cell & 0xffffu);
+            const int r2 = r == 0 ? 0 : n - r, c2 = c == 0 ? 0 : n - c;
+            if (r <= h) {
+                const int j = div_s(r) * n + c;
+                lds_add(&tile[j], v.x, v.y);
+                atomicAdd(&cnt[j], 1u);
+            }
+            if (r2 <= h) {  // both in the self-conjugate rows 0 and N/2
+                const int j = div_s(r2) * n + c2;
+                lds_add(&tile[j], v.x, -v.y);
+                atomicAdd(&cnt[j], 1u);
+            }
+        }
+        __syncthreads();
+    }
+    float2* grid = g.grids + img * (int64_t)n * n;
+    float* counts = g.counts + img * (int64_t)n * n;
+    for (int i = tid; i < rows * n; i += kSlabThreads) {
+        const unsigned k = cnt[i];
+        if (!k) continue;  // (rows past N/2 hold nothing)
+        const int lr = i / n, c = i - lr * n, r = lr * S + slab;
+        const float2 t = tile[i];
+        // the cell and its mirror (the same twice over in rows 0 and N/2: one write)
+        const bool twice = r != 0 && 2 * r != n;
+        const int64_t p = (int64_t)r * n + c;
+        const int64_t q = twice ? (int64_t)(n - r) * n + (c == 0 ? 0 : n - c) : p;
+        const float2 o = grid[p], oq = grid[q];
+        const float kp = counts[p], kq = counts[q];
+        grid[p] = make_float2(o.x + t.x, o.y + t.y);
+        counts[p] = kp + (float)k;
+        if (twice) {
+            grid[q] = make_float2(oq.x + t.x, oq.y - t.y);
+            counts[q] = kq + (float)k;
+        }
+    }
+}
+
+static size_t slab_lds(int n, int rows) { return (size_t)12 * n * rows + 2 * kSlabChunk; }
+
+// Slabs per image: as few as leave two workgroups per CU in LDS (one row at
+// the least), more while the images do not give every CU a workgroup.
+static int stage_slabs(int n, int64_t n_img) {
+    const int h1 = n / 2 + 1;
+    const int64_t room = (g_lds_limit / 2 - 2 * kSlabChunk) / (12 * (int64_t)n);
+    const int rows = (int)std::max<int64_t>(1, std::min<int64_t>(room, h1));
+    const int64_t fill = (device_cu_count() + n_img - 1) / n_img;
+    return (int)std::min<int64_t>(h1, std::max<int64_t>((h1 + rows - 1) / rows, fill));
+}
+
+// Slabs pay a pass over the channel's cells per slab, atomics pay per
+// visibility; slabs win on dense grids of small sides, atomics on sparse or
+// large ones and on a single image.  The line compares the two costs fitted to
+// measurements (us): slabs 13 + rounds of two workgroups per CU x (2.7 +
+// 0.44 per 1000 baselines), atomics 7 + 0.18 per 1000 visibilities.  Measured,
+// slabs / atomics, 32896 baselines: 1 x 180^2 18 / 15.5, 3 x 256^2 17 / 26,
+// 32 x 225^2 41 / 239, 32 x 512^2 52 / 204, 16 x 1024^2 80 / 102, 16 x 2048^2
+// 245 / 102; 8256 baselines: 24 x 512^2 21 / 40, 32 x 800^2 42 / 54, 24 x
+// 1024^2 49 / 40, 4 x 4096^2 94 / 9.3.  (Row plans and row tiles before, which
+// both replace: 188, -, 224, 327, -, -; 124, -, 170, 381.)
+bool stage_grid_slabs(int n, int n_bl, int64_t n_img) {
+    if (n > kMaxPixels || n_img == 0) return false;
+    const double rounds = (double)n_img * stage_slabs(n, n_img) / (2.0 * device_cu_count());
+    return 13.0 + rounds * (2.7 + 0.44e-3 * n_bl) < 7.0 + 0.18e-3 * (double)n_img * n_bl;
+}
+
+hipError_t launch_stage_grid(const float* vis, int n_ant, int n_ch, int n_t, const float* u_m,
+                             const float* v_m, const int* flags, const double* freq_hz, double du,
+                             double dv, double min_uv, int n_pixels, int pol, uint32_t* cells,
+                             float* grids, float* counts, hipStream_t stream) {
     const int n_bl = n_ant * (n_ant + 1) / 2;
-    const int64_t n_rec = (int64_t)n_bl * n_ch * n_t;
-    if (n_rec == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_grid_atomic, dim3(grid_for(n_rec, 256, 65536)), dim3(256), 0, stream,
-                       (const float4*)vis, n_bl, n_ch, n_rec, u_m, v_m, flags, freq_hz, du, dv,
-                       min_uv, n_pixels, pol, grids, counts);
+    const int64_t n_img = (int64_t)n_ch * n_t;
+    if (n_img == 0 || n_bl == 0) return hipSuccess;
+    const StageGrid g{(const float2*)vis, u_m, v_m, flags, freq_hz, du, dv, min_uv,
+                      n_bl, n_ch, n_pixels, pol, (float2*)grids, counts};
+    if (!cells) {
+        hipLaunchKernelGGL(k_grid_atomic,
+                           dim3((unsigned)((n_bl + 255) / 256), (unsigned)std::min<int64_t>(n_img, 65535)),
+                           dim3(256), 0, stream, g, n_img);
+        return hipGetLastError();
+    }
+    const int S = stage_slabs(n_pixels, n_img), rows = (n_pixels / 2 + S) / S;
+    const size_t lds = slab_lds(n_pixels, rows);
+    const int64_t blocks = n_img * S;
+    if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    const int stride = (int)stage_cell_stride(n_bl);
+    if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL(k_stage_cells, dim3((unsigned)((stride + 255) / 256), (unsigned)std::min(n_ch, 65535)),
+                       dim3(256), 0, stream, g, stride, cells);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_grid_slabs, dim3((unsigned)blocks), dim3(kSlabThreads), lds, stream, g, S,
+                       rows, stride, cells);
     return hipGetLastError();
 }
 
@@ -321,95 +525,10 @@ hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const 
     return hipGetLastError();
 }
 
-// --------------------------------------------- (b) gridding plan (row CSR)
-
-// Per channel: every gridded (baseline, conjugate) pair becomes two entries,
-// counting-sorted by grid row.  row_start[ch][0..N] (exclusive prefix sum of
-// the row histogram) and entries[ch][0..2*n_bl) packed as
-// u | conj << 13 | bl << 14.  One workgroup per channel.
-__global__ void __launch_bounds__(kPlanThreads)
-k_plan_rows(const float* __restrict__ u_m, const float* __restrict__ v_m,
-            const int* __restrict__ flags, int n_bl, const double* __restrict__ freq_hz,
-            double du, double dv, double min_uv, int n_pixels, int* __restrict__ row_start,
-            uint32_t* __restrict__ entries) {
-    extern __shared__ int plan_lds[];
-    int* hist = plan_lds;                 // [n_pixels]
-    int* cursor = plan_lds + n_pixels;    // [n_pixels]
-    __shared__ int warp_tot[kPlanThreads / 64];
-    const int ch = blockIdx.x;
-    const int tid = threadIdx.x;
-    const double wl = wavelength_of(freq_hz[ch]);
-    int* rs = row_start + (int64_t)ch * (n_pixels + 1);
-    uint32_t* ent = entries + (int64_t)ch * 2 * n_bl;
-
-    for (int i = tid; i < n_pixels; i += kPlanThreads) hist[i] = 0;
-    __syncthreads();
-    for (int bl = tid; bl < n_bl; bl += kPlanThreads) {
-        int up, vp;
-        if (flags[bl] || !cell_of(u_m[bl], v_m[bl], wl, du, dv, min_uv, n_pixels, up, vp)) continue;
-        atomicAdd(&hist[wrap_index(vp, n_pixels)], 1);
-        atomicAdd(&hist[wrap_index(-vp, n_pixels)], 1);
-    }
-    __syncthreads();
-    // Exclusive scan: each thread sums a contiguous chunk, the chunk totals
-    // are scanned across the block, then each chunk is rewritten.
-    const int chunk = (n_pixels + kPlanThreads - 1) / kPlanThreads;
-    const int c0 = min(tid * chunk, n_pixels), c1 = min(c0 + chunk, n_pixels);
-    int local = 0;
-    for (int i = c0; i < c1; i++) local += hist[i];
-    // inclusive scan of `local` across the block
-    const int lane = tid & 63, wid = tid >> 6;
-    int x = local;
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) warp_tot[wid] = x;
-    __syncthreads();
-    if (wid == 0) {
-        int t = (lane < kPlanThreads / 64) ? warp_tot[lane] : 0;
-        for (int o = 1; o < 64; o <<= 1) {
-            int y = __shfl_up(t, o, 64);
-            if (lane >= o) t += y;
-        }
-        if (lane < kPlanThreads / 64) warp_tot[lane] = t;
-    }
-    __syncthreads();
-    int run = x - local + (wid > 0 ? warp_tot[wid - 1] : 0);
-    for (int i = c0; i < c1; i++) {
-        const int h = hist[i];
-        rs[i] = run;
-        cursor[i] = run;
-        run += h;
-    }
-    if (tid == kPlanThreads - 1) rs[n_pixels] = warp_tot[kPlanThreads / 64 - 1];
-    __syncthreads();
-    for (int bl = tid; bl < n_bl; bl += kPlanThreads) {
-        int up, vp;
-        if (flags[bl] || !cell_of(u_m[bl], v_m[bl], wl, du, dv, min_uv, n_pixels, up, vp)) continue;
-        const int p = atomicAdd(&cursor[wrap_index(vp, n_pixels)], 1);
-        ent[p] = (uint32_t)wrap_index(up, n_pixels) | ((uint32_t)bl << 14);
-        const int q = atomicAdd(&cursor[wrap_index(-vp, n_pixels)], 1);
-        ent[q] = (uint32_t)wrap_index(-up, n_pixels) | (1u << 13) | ((uint32_t)bl << 14);
-    }
-}
-
-hipError_t launch_plan_rows(const float* u_m, const float* v_m, const int* flags, int n_bl,
-                            const double* freq_hz, int n_ch, double du, double dv, double min_uv,
-                            int n_pixels, int* row_start, uint32_t* entries, hipStream_t stream) {
-    if (n_ch == 0) return hipSuccess;
-    const size_t lds = sizeof(int) * 2 * (size_t)n_pixels;
-    if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k_plan_rows, dim3(n_ch), dim3(kPlanThreads), lds, stream, u_m, v_m, flags,
-                       n_bl, freq_hz, du, dv, min_uv, n_pixels, row_start, entries);
-    return hipGetLastError();
-}
-
 // ------------------------------------------ (b) gridding plans of a batched call
 //
 // One plan unit per (set, channel): the counting sort of the channel's 2 n_bl
-// cells by grid row, the same result k_plan_rows gives.  `parts` workgroups
-// per unit share its baselines.
+// cells by grid row; `parts` workgroups per unit share its baselines.
 //   count    the cell of every baseline of the part (FP64, bit-exact), kept
 //            packed for the scatter, and the part's histogram by row;
 //   scan     per unit: row starts, and each part's first slot in every row;
@@ -679,90 +798,6 @@ __device__ __forceinline__ int row_of_entry(const int* rs, int nr, int e) {
     int r = 0;
     while (r + 1 < nr && rs[r + 1] <= e) r++;
     return r;
-}
-
-// ------------------------------- (b) gridding, LDS-privatised row tiles
-
-// Workgroup = (row tile of RB rows, image).  The tile's plan entries are
-// accumulated with LDS atomics (complex grid and counts), then the tile is
-// added to the global grids/counts (each cell is owned by one workgroup, so
-// the flush needs no atomics).
-__global__ void __launch_bounds__(kTileThreads)
-k_grid_tiles(GatherArgs g, const int* __restrict__ row_start, const uint32_t* __restrict__ entries,
-             int n_pixels, int rb, float2* __restrict__ grids, float* __restrict__ counts,
-             int overwrite, uint32_t* __restrict__ isums, int64_t img0) {
-    extern __shared__ float4 tiles_lds4[];
-    float2* tile = (float2*)tiles_lds4;                       // [rb][N]
-    unsigned* cnt = (unsigned*)(tile + (size_t)rb * n_pixels);  // [rb][N]
-    __shared__ int rs[kMaxTileRows + 1];
-    __shared__ int red[kTileThreads / 64];
-    const int n_rb = (n_pixels + rb - 1) / rb;
-    const int tile_id = blockIdx.x % n_rb;
-    const int64_t li = blockIdx.x / n_rb;       // image within the launch
-    const int64_t img = img0 + li;              // image within the set
-    const int ch = (int)(img % g.n_ch);
-    const int r0 = tile_id * rb;
-    const int nr = min(rb, n_pixels - r0);
-    const int* rsg = row_start + (int64_t)ch * (n_pixels + 1);
-    const uint32_t* ent = entries + (int64_t)ch * 2 * g.n_bl;
-    if (threadIdx.x <= nr) rs[threadIdx.x] = rsg[r0 + threadIdx.x];
-    __syncthreads();
-    const int64_t base = li * (int64_t)n_pixels * n_pixels + (int64_t)r0 * n_pixels;
-    const int cells = nr * n_pixels;
-    if (rs[nr] == rs[0]) {  // nothing lands in this tile
-        if (overwrite)
-            for (int i = threadIdx.x; i < cells; i += blockDim.x) grids[base + i] = make_float2(0.f, 0.f);
-        return;
-    }
-    for (int i = threadIdx.x; i < cells; i += blockDim.x) {
-        tile[i] = make_float2(0.f, 0.f);
-        cnt[i] = 0u;
-    }
-    __syncthreads();
-    const int n_ok = gather_range<4>(g, img, ch, ent, rs[0], rs[nr], (int)threadIdx.x,
-                                     (int)blockDim.x, [&](int e, int u_idx, float2 v) {
-        const int r = row_of_entry(rs, nr, e);
-        const int c = r * n_pixels + u_idx;
-        lds_add(&tile[c], v.x, v.y);
-        atomicAdd(&cnt[c], 1u);
-        return 1;
-    });
-    if (isums) {
-        const int tot = block_sum_int(n_ok, red);
-        if (threadIdx.x == 0 && tot) atomicAdd(&isums[img], (uint32_t)tot);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < cells; i += blockDim.x) {
-        const int r = i / n_pixels;
-        if (overwrite) {
-            grids[base + i] = tile[i];
-            if (counts) counts[base + i] = (float)cnt[i];
-            continue;
-        }
-        if (rs[r + 1] == rs[r]) continue;  // empty row: nothing to add
-        const float2 t = tile[i];
-        float2 o = grids[base + i];
-        o.x += t.x;
-        o.y += t.y;
-        grids[base + i] = o;
-        counts[base + i] += (float)cnt[i];
-    }
-}
-
-hipError_t launch_grid_tiles(const GatherArgs& g, const int* row_start, const uint32_t* entries,
-                             int n_images, int n_pixels, float* grids, float* counts,
-                             hipStream_t stream, int overwrite, uint32_t* isums, int64_t img0) {
-    if (n_images == 0) return hipSuccess;
-    // 12 bytes per cell (complex + count) within the LDS budget.
-    int rb = (int)(g_lds_budget / (12 * (int64_t)n_pixels));
-    rb = std::max(1, std::min(rb, kMaxTileRows));
-    const int n_rb = (n_pixels + rb - 1) / rb;
-    const size_t lds = (size_t)rb * n_pixels * 12;
-    if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k_grid_tiles, dim3((unsigned)((int64_t)n_rb * n_images)), dim3(kTileThreads),
-                       lds, stream, g, row_start, entries, n_pixels, rb, (float2*)grids, counts,
-                       overwrite, isums, img0);
-    return hipGetLastError();
 }
 
 // Hermitian half plane for the DFT transform: rows v = 0 .. N/2 of each image
@@ -1692,9 +1727,8 @@ hipError_t set_kernel_attributes() {
     set((const void*)k_cols_half_odd<1, false, false>);
     set((const void*)k_cols_half_odd<1, true, true>);
     set((const void*)k_cols_half_odd<1, false, true>);
-    set((const void*)k_grid_tiles);
+    set((const void*)k_grid_slabs);
     set((const void*)k_grid_half_rows);
-    set((const void*)k_plan_rows);
     set((const void*)k_plan_count);
     set((const void*)k_plan_scatter);
     return e;

@@ -13,7 +13,6 @@ namespace blink {
 
 constexpr int kMaxPixels = 8192;      // largest grid side (plan entries pack positions in 13 bits)
 constexpr int kMaxBaselines = 1 << 18;  // plan packs the baseline in 18 bits
-constexpr int kPlanThreads = 1024;
 constexpr int kTileThreads = 256;
 constexpr int kFftThreads = 256;
 // Columns per block of the register kernels' column-blocked row-pass buffer.
@@ -144,10 +143,16 @@ hipError_t launch_phase_correct(float* vis, int n_ant, int n_ch, int n_t, const 
 hipError_t launch_uv_cells(const float* u_m, const float* v_m, const int* flags, int n_bl,
                            const double* freq_hz, int n_ch, double du, double dv, double min_uv,
                            int n_pixels, int* cells, hipStream_t stream);
-hipError_t launch_grid_atomic(const float* vis, int n_ant, int n_ch, int n_t, const float* u_m,
-                              const float* v_m, const int* flags, const double* freq_hz, double du,
-                              double dv, double min_uv, int n_pixels, int pol, float* grids,
-                              float* counts, hipStream_t stream);
+// Nearest-cell gridding of the stage path, accumulating into grids and counts:
+// global atomics, or, with `cells` (scratch of stage_cell_stride(n_bl) words
+// per channel), slabs of the half plane in LDS (n_pixels <= kMaxPixels).
+// stage_grid_slabs says which is faster.
+bool stage_grid_slabs(int n_pixels, int n_bl, int64_t n_img);
+constexpr int64_t stage_cell_stride(int64_t n_bl) { return (n_bl + 3) & ~(int64_t)3; }
+hipError_t launch_stage_grid(const float* vis, int n_ant, int n_ch, int n_t, const float* u_m,
+                             const float* v_m, const int* flags, const double* freq_hz, double du,
+                             double dv, double min_uv, int n_pixels, int pol, uint32_t* cells,
+                             float* grids, float* counts, hipStream_t stream);
 hipError_t launch_zenith_uvw(const double* x, const double* y, const double* z, int n_ant,
                              float* u_m, float* v_m, float* w_m, hipStream_t stream);
 hipError_t launch_baseline_flags(const int* ant_flags, int n_ant, int* bl_flags,
@@ -160,16 +165,6 @@ hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const 
                           const float* v_m, const int* flags, const double* freq_hz, double du,
                           double dv, double min_uv, int n_pixels, int pol, int kernel_size,
                           const double* table, float* grids, float* counts, hipStream_t stream);
-hipError_t launch_plan_rows(const float* u_m, const float* v_m, const int* flags, int n_bl,
-                            const double* freq_hz, int n_ch, double du, double dv, double min_uv,
-                            int n_pixels, int* row_start, uint32_t* entries, hipStream_t stream);
-// Row-tile gridding.  Accumulates into grids/counts, or with overwrite != 0
-// writes every cell of the n_images grids (counts may then be null); valid
-// visibilities are added to isums[img0 + image] when isums is given.
-hipError_t launch_grid_tiles(const GatherArgs& g, const int* row_start, const uint32_t* entries,
-                             int n_images, int n_pixels, float* grids, float* counts,
-                             hipStream_t stream, int overwrite = 0, uint32_t* isums = nullptr,
-                             int64_t img0 = 0);
 hipError_t launch_uniform_weight(float* grids, const float* counts, int64_t n_cells,
                                  hipStream_t stream);
 // One pass (rows, then columns) of the 2-D transform of n_img images;

@@ -90,7 +90,8 @@ enum blink_transform {
 
 /* Gridding algorithm for blink_gridding. */
 enum blink_grid_algo {
-    BLINK_GRID_TILED = 0,  /* per-channel row plan + LDS-privatised row tiles (default) */
+    BLINK_GRID_TILED = 0,  /* slabs of the plane privatised in LDS, or atomics where they are
+                              faster (default) */
     BLINK_GRID_ATOMIC = 1  /* one thread per visibility, global atomics (plain path) */
 };
 

@@ -67,3 +67,32 @@ def test_crowded_cells_batched(ctx, monkeypatch, n, transform, direct):
     ref, _ = oracle.run_f32(o.vis, o.n_ant, o.u, o.v, o.w, o.flags, o.freq, o.cable, True, True,
                             1.0, 1.0, o.min_uv, n)
     assert oracle.peak_normalised_error(images.cpu().numpy(), ref)[0] < 1e-5
+
+
+@pytest.mark.parametrize("n_ant,n_ch,n_t,n", [(96, 3, 2, 128), (256, 3, 1, 225), (128, 9, 1, 512), (64, 40, 1, 45),
+                                              (256, 17, 1, 1024), (160, 1, 1, 2), (33, 300, 1, 16)])
+@pytest.mark.parametrize("pol,min_uv", [("XX", -np.inf), ("V", 2.0)])
+def test_stage_gridding_adds_to_what_is_there(ctx, n_ant, n_ch, n_t, n, pol, min_uv):
+    """blink_gridding accumulates: twice over the same cells of non-empty grids, odd and even
+    sides, both sides of the choice between slabs and atomics.  Counts exact; sums within the
+    bound of an FP32 sum of the cell's values and what was there."""
+    import torch
+    from imager_amd import capi
+    o = synth.small(n_ant=n_ant, n_ch=n_ch, n_t=n_t, n_pixels=n, seed=n_ant + n, bl_flag_fraction=0.2)
+    o.vis[0, 0, 3, :] = np.nan
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.flags, o.freq)]
+    ref, cref, _ = oracle.gridding(o.vis, o.n_ant, o.u, o.v, o.flags, o.freq, o.delta_u, o.delta_v,
+                                   min_uv, n, pol, precision="f64")
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    start = torch.randn((n_t, n_ch, n, n, 2), device="cuda", generator=gen)
+    grids = torch.view_as_complex(start.clone())
+    counts = torch.full((n_t, n_ch, n, n), 5.0, device="cuda")
+    for _ in range(2):
+        ctx.gridding(d[0], o.n_ant, n_ch, n_t, d[1], d[2], d[3], d[4], o.delta_u, o.delta_v, min_uv, n,
+                     pol, 0, grids, counts)
+    torch.cuda.synchronize()
+    assert np.array_equal(counts.cpu().numpy(), 5.0 + 2.0 * cref)
+    want = torch.view_as_complex(start.double()).cpu().numpy() + 2.0 * ref
+    big = float(np.nanmax(np.abs(o.vis))) * 2.0
+    terms = 2.0 * cref.max() + 2.0
+    assert np.abs(grids.cpu().numpy() - want).max() <= terms * 2.0 ** -24 * (terms * big + 10.0)

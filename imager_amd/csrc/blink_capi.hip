@@ -665,9 +665,16 @@ BLINK_API int blink_gridding_kernel(blink_ctx* ctx, const float* vis, int n_ant,
     const double* table;
     if ((rc = kb_table(ctx, kernel_size, kernel_mode, &table))) return rc;
     hipStream_t s = (hipStream_t)stream;
+    const int n_bl = n_ant * (n_ant + 1) / 2;
+    void* cells = nullptr;
+    if (kb_grid_slabs(n_pixels, n_bl, (int64_t)n_ch * n_t, kernel_size) &&
+        (rc = ctx_scratch(ctx, "grid_cells",
+                          sizeof(uint32_t) * (size_t)n_ch * stage_cell_stride(n_bl), &cells)))
+        return rc;
     LAUNCH("grid_kernel", s,
            launch_grid_kb(vis, n_ant, n_ch, n_t, u_m, v_m, bl_flags, freq_hz, delta_u, delta_v,
-                          min_uv, n_pixels, pol, kernel_size, table, grids, counts, s));
+                          min_uv, n_pixels, pol, kernel_size, table, (uint32_t*)cells, grids,
+                          counts, s));
     if (weighting == BLINK_WEIGHTING_UNIFORM)
         LAUNCH("uniform_weight", s,
                launch_uniform_weight(grids, counts, (int64_t)n_ch * n_t * n_pixels * n_pixels, s));

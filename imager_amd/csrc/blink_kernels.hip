@@ -454,74 +454,269 @@ hipError_t launch_stage_grid(const float* vis, int n_ant, int n_ch, int n_t, con
 
 // --------------------------------------- (b) convolutional (Kaiser-Bessel) gridding
 
-// One thread per (t, ch, bl).  The visibility and its conjugate are spread
-// over K x K cells with weights kt[ky][j] * kt[kx][i] (double), the kernel
-// row chosen from the 1023-times oversampled fractional cell position as
-// convolve_with_kernel does (src/pacer_imager.cpp:654-714); counts go to the
-// nearest cells (:387,408).  FP32 global atomics.
-__global__ void k_grid_kb(const float4* __restrict__ vis, int n_bl, int n_ch, int64_t n_rec,
-                          const float* __restrict__ u_m, const float* __restrict__ v_m,
-                          const int* __restrict__ flags, const double* __restrict__ freq_hz,
-                          double du, double dv, double min_uv, int n_pixels, int pol, int K,
-                          const double* __restrict__ kt, float* __restrict__ grids,
-                          float* __restrict__ counts) {
+// Nearest cell and kernel rows of one visibility, as convolve_with_kernel
+// chooses them from the 1023-times oversampled fractional cell position
+// (src/pacer_imager.cpp:654-714).
+struct KbSpot {
+    int up, vp;        // nearest cell
+    const double* xk;  // K weights along u
+    const double* yk;  // K weights along v
+};
+__device__ __forceinline__ bool kb_spot(const StageGrid& g, double wl, int bl, int K,
+                                        const double* __restrict__ kt, KbSpot& sp) {
 #pragma clang fp contract(off)
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t gs = (int64_t)n_pixels * n_pixels;
-    const int mid = K / 2;
+    if (!cell_of(g.u_m[bl], g.v_m[bl], wl, g.du, g.dv, g.min_uv, g.n_pixels, sp.up, sp.vp)) return false;
+    const double ue = (double)g.u_m[bl] / wl / g.du;
+    const double ve = (double)g.v_m[bl] / wl / g.dv;
+    int kx = (int)round((ue - (double)sp.up) * 1023.0);
+    int ky = (int)round((ve - (double)sp.vp) * 1023.0);
+    kx = (kx + 1534) % 1023;
+    ky = (ky + 1534) % 1023;
+    sp.xk = kt + (int64_t)kx * K;
+    sp.yk = kt + (int64_t)ky * K;
+    return true;
+}
+
+// Sparse grids of large sides (see kb_grid_slabs): one thread per (image,
+// baseline), FP32 global atomics.  The visibility and its conjugate
+// are spread over K x K cells with weights kt[ky][j] * kt[kx][i] in FP64; counts
+// go to the nearest cells (:387,408).
+__global__ void __launch_bounds__(256)
+k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
+#pragma clang fp contract(off)
+    const int n = g.n_pixels, mid = K / 2;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, gs = (int64_t)n * n;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_rec; i += stride) {
-        const int bl = (int)(i % n_bl);
-        const int64_t img = i / n_bl;
-        const int ch = (int)(img % n_ch);
-        if (flags[bl]) continue;
-        const float2 val = select_pol(vis[2 * i], vis[2 * i + 1], pol);
-        if (!vis_ok(val)) continue;
-        const double wl = wavelength_of(freq_hz[ch]);
-        int up, vp;
-        if (!cell_of(u_m[bl], v_m[bl], wl, du, dv, min_uv, n_pixels, up, vp)) continue;
-        const double ue = (double)u_m[bl] / wl / du;
-        const double ve = (double)v_m[bl] / wl / dv;
-        int kx = (int)round((ue - (double)up) * 1023.0);
-        int ky = (int)round((ve - (double)vp) * 1023.0);
-        kx = (kx + 1534) % 1023;
-        ky = (ky + 1534) % 1023;
-        const double* xk = kt + (int64_t)kx * K;
-        const double* yk = kt + (int64_t)ky * K;
-        float* g = grids + 2 * img * gs;
+        const int bl = (int)(i % g.n_bl);
+        const int64_t img = i / g.n_bl;
+        if (g.flags[bl]) continue;
+        const float2 val = stage_value(g, img, bl);
+        KbSpot sp;
+        if (!vis_ok(val) || !kb_spot(g, wavelength_of(g.freq_hz[img % g.n_ch]), bl, K, kt, sp)) continue;
+        float* grid = (float*)(g.grids + img * gs);
         for (int s = 1; s >= -1; s -= 2) {
             for (int j = 0; j < K; j++) {
                 int y;
-                if (!kb_cell(vp - mid + j, s, n_pixels, y)) continue;
-                const double wy = yk[j];
+                if (!kb_cell(sp.vp - mid + j, s, n, y)) continue;
+                const double wy = sp.yk[j];
                 for (int c = 0; c < K; c++) {
                     int x;
-                    if (!kb_cell(up - mid + c, s, n_pixels, x)) continue;
-                    const double w = wy * xk[c];
-                    const double re = (double)val.x * w;
-                    const double im = (double)s * (double)val.y * w;
-                    const int64_t p = (int64_t)y * n_pixels + x;
-                    unsafeAtomicAdd(&g[2 * p], (float)re);
-                    unsafeAtomicAdd(&g[2 * p + 1], (float)im);
+                    if (!kb_cell(sp.up - mid + c, s, n, x)) continue;
+                    const double w = wy * sp.xk[c];
+                    const int64_t p = (int64_t)y * n + x;
+                    unsafeAtomicAdd(&grid[2 * p], (float)((double)val.x * w));
+                    unsafeAtomicAdd(&grid[2 * p + 1], (float)((double)s * (double)val.y * w));
+                }
+            }
+            unsafeAtomicAdd(&g.counts[img * gs + (int64_t)wrap_index(s * sp.vp, n) * n +
+                                      wrap_index(s * sp.up, n)], 1.0f);
+        }
+    }
+}
+
+// Row slabs in LDS.  Workgroup (slab, image) owns the consecutive grid rows
+// slab * rows .. + rows - 1.  It walks the cells of its channel (k_stage_cells)
+// a chunk at a time, queues (baseline, sign) wherever the nearest row of that
+// footprint lies within K / 2 rows (cyclically: a superset of the footprints
+// that reach the slab), and each thread then spreads one queued footprint over
+// the slab's rows, only those it reaches (a mask), so that the lanes of a
+// wavefront take at most `rows` turns.  At the end the
+// non-zero cells are added to the global grid; no other workgroup touches them.
+// The work is the K x K updates of every footprint.  The cells are FP64 planes:
+// ds_add_f64 costs 21 clocks per wavefront instruction whatever collides, where
+// the footprints of a dense core make compare-and-swaps of FP32 cells retry.
+// kX: largest K whose weights along u stay in registers; each weight read in
+// the inner loop would be a gather of 64 cache lines per wavefront.
+constexpr int kKbThreads = 512, kKbVec = 3;
+constexpr int kKbChunk = kKbThreads * 4 * kKbVec;
+static_assert(2 * kKbChunk <= 32768, "queue entries: 15-bit offset and a sign");
+template <int kX>
+__global__ void __launch_bounds__(kKbThreads)
+k_grid_kb_slabs(StageGrid g, int rows, int stride, const uint32_t* __restrict__ cells, int K,
+                const double* __restrict__ kt) {
+#pragma clang fp contract(off)
+    extern __shared__ float4 kb_slabs_lds4[];
+    const int n = g.n_pixels, mid = K / 2;
+    double* re = (double*)kb_slabs_lds4;                     // [rows][n]
+    double* im = re + (size_t)rows * n;                      // [rows][n]
+    unsigned* cnt = (unsigned*)(im + (size_t)rows * n);      // [rows][n]
+    unsigned short* queue = (unsigned short*)(cnt + (size_t)rows * n);  // [2 kKbChunk]
+    __shared__ int n_queued;
+    const int n_slab = (n + rows - 1) / rows;
+    const int r0 = (int)(blockIdx.x % (unsigned)n_slab) * rows, nr = min(rows, n - r0);
+    const int64_t img = blockIdx.x / (unsigned)n_slab;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t* cl = cells + (img % g.n_ch) * stride;
+    const double wl = wavelength_of(g.freq_hz[img % g.n_ch]);
+    for (int i = tid; i < rows * n; i += kKbThreads) {
+        re[i] = im[i] = 0.0;
+        cnt[i] = 0u;
+    }
+    // rows r0 - reach .. r0 + nr - 1 + reach (kb_cell places the negative rows of
+    // an odd side one lower than wrap_index does)
+    const int reach = mid + (n & 1), span = nr + 2 * reach;
+    auto near = [&](int r) {
+        int d = r - (r0 - reach);
+        d = d < 0 ? d + n : (d >= n ? d - n : d);
+        return d < span || span >= n;
+    };
+    for (int base = 0; base < stride; base += kKbChunk) {
+        if (tid == 0) n_queued = 0;
+        __syncthreads();
+        uint4 p[kKbVec];
+#pragma unroll
+        for (int k = 0; k < kKbVec; k++) {
+            const int b = base + 4 * (tid + k * kKbThreads);
+            p[k] = b < stride ? *(const uint4*)&cl[b]
+                              : make_uint4(kNoCell, kNoCell, kNoCell, kNoCell);
+        }
+        unsigned keep = 0;  // two bits per baseline: its own footprint, its conjugate's
+#pragma unroll
+        for (int k = 0; k < kKbVec; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t c = j == 0 ? p[k].x : j == 1 ? p[k].y : j == 2 ? p[k].z : p[k].w;
+                if (c == kNoCell) continue;
+                const int r = (int)(c >> 16);
+                if (near(r)) keep |= 1u << (8 * k + 2 * j);
+                if (near(r == 0 ? 0 : n - r)) keep |= 2u << (8 * k + 2 * j);
+            }
+        int before = __popc(keep);
+        const int own = before;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(before, o, 64);
+            if (lane >= o) before += t;
+        }
+        int at = 0;
+        if (lane == 63) at = atomicAdd(&n_queued, before);
+        at = __shfl(at, 63, 64) + before - own;
+        while (keep) {
+            const int bit = __ffs(keep) - 1;
+            keep &= keep - 1;
+            queue[at++] = (unsigned short)((4 * (tid + (bit >> 3) * kKbThreads) + ((bit >> 1) & 3)) * 2 +
+                                           (bit & 1));
+        }
+        __syncthreads();
+        const int nq = n_queued;
+        for (int i = tid; i < nq; i += kKbThreads) {
+            const int q = queue[i], bl = base + (q >> 1), s = (q & 1) ? -1 : 1;
+            const float2 v = stage_value(g, img, bl);
+            KbSpot sp;
+            if (!vis_ok(v) || !kb_spot(g, wl, bl, K, kt, sp)) continue;
+            const int rn = wrap_index(s * sp.vp, n) - r0;
+            if ((unsigned)rn < (unsigned)nr) atomicAdd(&cnt[rn * n + wrap_index(s * sp.up, n)], 1u);
+            double xw[kX > 0 ? kX : 1];
+            int xc[kX > 0 ? kX : 1];
+            if constexpr (kX > 0) {
+#pragma unroll
+                for (int c = 0; c < kX; c++) {
+                    xc[c] = -1;
+                    if (c >= K) continue;
+                    xw[c] = sp.xk[c];
+                    int x;
+                    if (kb_cell(sp.up - mid + c, s, n, x)) xc[c] = x;
+                }
+            }
+            unsigned hit = 0;  // rows j of the footprint in this slab
+            for (int j = 0; j < K; j++) {
+                int y;
+                if (kb_cell(sp.vp - mid + j, s, n, y) && (unsigned)(y - r0) < (unsigned)nr) hit |= 1u << j;
+            }
+            for (; hit; hit &= hit - 1) {
+                const int j = __ffs(hit) - 1;
+                int y = 0;
+                kb_cell(sp.vp - mid + j, s, n, y);
+                const double wy = sp.yk[j];
+                const int row = (y - r0) * n;
+                auto put = [&](int x, double wx) {
+                    const double w = wy * wx;
+                    atomicAdd(&re[row + x], (double)v.x * w);
+                    atomicAdd(&im[row + x], (double)s * (double)v.y * w);
+                };
+                if constexpr (kX > 0) {
+#pragma unroll
+                    for (int c = 0; c < kX; c++)
+                        if (xc[c] >= 0) put(xc[c], xw[c]);
+                } else {
+                    for (int c = 0; c < K; c++) {
+                        int x;
+                        if (kb_cell(sp.up - mid + c, s, n, x)) put(x, sp.xk[c]);
+                    }
                 }
             }
         }
-        unsafeAtomicAdd(&counts[img * gs + (int64_t)wrap_index(vp, n_pixels) * n_pixels +
-                                wrap_index(up, n_pixels)], 1.0f);
-        unsafeAtomicAdd(&counts[img * gs + (int64_t)wrap_index(-vp, n_pixels) * n_pixels +
-                                wrap_index(-up, n_pixels)], 1.0f);
+        __syncthreads();
     }
+    float2* grid = g.grids + img * (int64_t)n * n + (int64_t)r0 * n;
+    float* counts = g.counts + img * (int64_t)n * n + (int64_t)r0 * n;
+    for (int i = tid; i < nr * n; i += kKbThreads) {
+        const double x = re[i], y = im[i];
+        const unsigned k = cnt[i];
+        if (!(x == 0.0 && y == 0.0)) {
+            const float2 o = grid[i];
+            grid[i] = make_float2((float)((double)o.x + x), (float)((double)o.y + y));
+        }
+        if (k) counts[i] += (float)k;
+    }
+}
+
+static size_t kb_slab_lds(int n, int rows) { return (size_t)20 * n * rows + 4 * kKbChunk; }
+
+// Rows per slab: up to 8 (the wider, the fewer slabs compute a footprint's
+// weights again), fewer while that leaves under four workgroups per CU or
+// fills more than a third of a CU's LDS.
+static int kb_slab_rows(int n, int64_t n_img) {
+    int rows = 8;
+    while (rows > 1 && (3 * (int64_t)kb_slab_lds(n, rows) > g_lds_limit ||
+                        n_img * ((n + rows - 1) / rows) < 4 * device_cu_count()))
+        rows /= 2;
+    return rows;
+}
+
+// Slabs pay their set-up (clearing, walking the channel's cells, the flush) per
+// workgroup, global atomics 4 K^2 round trips per visibility.  Costs fitted to
+// measurements (us): slabs 20 + 0.022 per workgroup (0.035 where one fills a CU's
+// LDS) + 1.1e-5 per footprint cell, atomics 2.3e-4 per footprint cell.  Measured,
+// atomics -> slabs: 16 x 256^2, 32896 baselines, K 7 4914 -> 287; 1 x 180^2 803 ->
+// 74; 2 x 225^2, K 15 5926 -> 232; 8256 baselines: 4 x 1024^2 349 -> 85, 2 x 4096^2
+// 187 -> 285.
+bool kb_grid_slabs(int n, int n_bl, int64_t n_img, int K) {
+    if (n > kMaxPixels || n_img == 0) return false;
+    const int rows = kb_slab_rows(n, n_img);
+    const double wgs = (double)n_img * ((n + rows - 1) / rows);
+    const double cells = (double)n_img * n_bl * K * K;
+    const double per = 2 * (int64_t)kb_slab_lds(n, rows) > g_lds_limit ? 0.035 : 0.022;
+    return 20.0 + per * wgs + 1.1e-5 * cells < 2.3e-4 * cells;
 }
 
 hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const float* u_m,
                           const float* v_m, const int* flags, const double* freq_hz, double du,
                           double dv, double min_uv, int n_pixels, int pol, int kernel_size,
-                          const double* table, float* grids, float* counts, hipStream_t stream) {
+                          const double* table, uint32_t* cells, float* grids, float* counts,
+                          hipStream_t stream) {
     const int n_bl = n_ant * (n_ant + 1) / 2;
-    const int64_t n_rec = (int64_t)n_bl * n_ch * n_t;
-    if (n_rec == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_grid_kb, dim3(grid_for(n_rec, 256, 65536)), dim3(256), 0, stream,
-                       (const float4*)vis, n_bl, n_ch, n_rec, u_m, v_m, flags, freq_hz, du, dv,
-                       min_uv, n_pixels, pol, kernel_size, table, grids, counts);
+    const int64_t n_img = (int64_t)n_ch * n_t;
+    if (n_img == 0 || n_bl == 0) return hipSuccess;
+    const StageGrid g{(const float2*)vis, u_m, v_m, flags, freq_hz, du, dv, min_uv,
+                      n_bl, n_ch, n_pixels, pol, (float2*)grids, counts};
+    if (!cells) {
+        const int64_t n_rec = n_bl * n_img;
+        hipLaunchKernelGGL(k_grid_kb, dim3(grid_for(n_rec, 256, 65536)), dim3(256), 0, stream, g,
+                           n_rec, kernel_size, table);
+        return hipGetLastError();
+    }
+    const int rows = kb_slab_rows(n_pixels, n_img);
+    const size_t lds = kb_slab_lds(n_pixels, rows);
+    const int64_t blocks = n_img * ((n_pixels + rows - 1) / rows);
+    if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    const int stride = (int)stage_cell_stride(n_bl);
+    hipLaunchKernelGGL(k_stage_cells, dim3((unsigned)((stride + 255) / 256), (unsigned)std::min(n_ch, 65535)),
+                       dim3(256), 0, stream, g, stride, cells);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const auto k = kernel_size <= 8 ? k_grid_kb_slabs<8> : k_grid_kb_slabs<0>;
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kKbThreads), lds, stream, g, rows, stride,
+                       cells, kernel_size, table);
     return hipGetLastError();
 }
 
@@ -1728,6 +1923,8 @@ hipError_t set_kernel_attributes() {
     set((const void*)k_cols_half_odd<1, true, true>);
     set((const void*)k_cols_half_odd<1, false, true>);
     set((const void*)k_grid_slabs);
+    set((const void*)k_grid_kb_slabs<8>);
+    set((const void*)k_grid_kb_slabs<0>);
     set((const void*)k_grid_half_rows);
     set((const void*)k_plan_count);
     set((const void*)k_plan_scatter);

@@ -160,11 +160,15 @@ hipError_t launch_baseline_flags(const int* ant_flags, int n_ant, int* bl_flags,
 hipError_t launch_uv_max(const float* u_m, const float* v_m, const int* flags, int n_bl,
                          double* uv_max, hipStream_t stream);
 // Convolutional gridding with a kernel table of 1023 rows of kernel_size
-// doubles (row = oversampled fractional cell position).
+// doubles (row = oversampled fractional cell position); `cells`: scratch of
+// stage_cell_stride(n_bl) words per channel for slabs in LDS, null for global
+// atomics; kb_grid_slabs says which is faster.
+bool kb_grid_slabs(int n_pixels, int n_bl, int64_t n_img, int kernel_size);
 hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const float* u_m,
                           const float* v_m, const int* flags, const double* freq_hz, double du,
                           double dv, double min_uv, int n_pixels, int pol, int kernel_size,
-                          const double* table, float* grids, float* counts, hipStream_t stream);
+                          const double* table, uint32_t* cells, float* grids, float* counts,
+                          hipStream_t stream);
 hipError_t launch_uniform_weight(float* grids, const float* counts, int64_t n_cells,
                                  hipStream_t stream);
 // One pass (rows, then columns) of the 2-D transform of n_img images;

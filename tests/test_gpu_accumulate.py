@@ -96,3 +96,33 @@ def test_stage_gridding_adds_to_what_is_there(ctx, n_ant, n_ch, n_t, n, pol, min
     big = float(np.nanmax(np.abs(o.vis))) * 2.0
     terms = 2.0 * cref.max() + 2.0
     assert np.abs(grids.cpu().numpy() - want).max() <= terms * 2.0 ** -24 * (terms * big + 10.0)
+
+
+@pytest.mark.parametrize("n_ant,n_ch,n,K", [(48, 2, 64, 1), (40, 3, 45, 7), (64, 1, 180, 8), (64, 2, 225, 9),
+                                            (96, 5, 256, 7), (24, 1, 16, 31), (200, 1, 61, 16), (10, 1, 1024, 7),
+                                            (128, 2, 1001, 4)])
+@pytest.mark.parametrize("pol,min_uv", [("XX", -np.inf), ("I", 2.0)])
+def test_stage_footprints_add_to_what_is_there(ctx, n_ant, n_ch, n, K, pol, min_uv):
+    """blink_gridding_kernel over its slabs and its atomics (the smallest and sparsest sets), odd and
+    even sides and footprints, footprints wider than a slab or cut by the plane's edge, twice
+    over non-empty grids.  Counts exact; sums within the bound of an FP32 sum."""
+    import torch
+    o = synth.small(n_ant=n_ant, n_ch=n_ch, n_t=1, n_pixels=n, seed=n_ant + n + K, bl_flag_fraction=0.2)
+    o.vis[0, 0, 5, :] = np.nan
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.flags, o.freq)]
+    ref, cref, _ = oracle.gridding(o.vis, o.n_ant, o.u, o.v, o.flags, o.freq, o.delta_u, o.delta_v,
+                                   min_uv, n, pol, precision="f64", kernel_size=K, with_sinc=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    start = torch.randn((1, n_ch, n, n, 2), device="cuda", generator=gen)
+    grids = torch.view_as_complex(start.clone())
+    counts = torch.full((1, n_ch, n, n), 3.0, device="cuda")
+    for _ in range(2):
+        ctx.gridding_kernel(d[0], o.n_ant, n_ch, 1, d[1], d[2], d[3], d[4], o.delta_u, o.delta_v,
+                            min_uv, n, pol, 0, K, grids, counts)
+    torch.cuda.synchronize()
+    assert np.array_equal(counts.cpu().numpy(), 3.0 + 2.0 * cref)
+    want = torch.view_as_complex(start.double()).cpu().numpy() + 2.0 * ref
+    weight = float(np.abs(oracle.kb_kernels(K)).max()) ** 2
+    big = float(np.nanmax(np.abs(o.vis))) * max(weight, 1.0)
+    terms = 4.0 * o.n_bl
+    assert np.abs(grids.cpu().numpy() - want).max() <= terms * 2.0 ** -24 * (big + 10.0)

@@ -358,10 +358,8 @@ __device__ __forceinline__ void win_transform_rows(float2* tile, int r0, int nr,
 // channel, whose images share their row starts) the workgroup only sets
 // start[N] = -1, which the second pass never reads, and leaves the image to
 // k_grid_rows_direct_blocks, launched next.  A cell outside the window (not
-// expected: the bound is exact) does the same.  kKb: convolutional gridding
-// (kb_walk), the window widened by K/2 on every side for the footprints.
-// `cap`: tile elements in LDS.
-template <int N, int NT, bool kMulti, bool kKb>
+// expected: the bound is exact) does the same.  `cap`: tile elements in LDS.
+template <int N, int NT, bool kMulti>
 __global__ void __launch_bounds__(NT)
 k_grid_rows_direct_win(SetDesc first, const SetDesc* __restrict__ sets,
                        const int* __restrict__ img_set, int64_t gi0, float2* __restrict__ inter,
@@ -392,9 +390,8 @@ k_grid_rows_direct_win(SetDesc first, const SetDesc* __restrict__ sets,
         const double wl = wavelength_of(sd.g.freq_hz[ch]);
         const double eu = fabs(round(((double)mu / wl) / sd.du));
         const double ev = fabs(round(((double)mv / wl) / sd.dv));
-        const double margin = kKb ? (double)(sd.kb_size / 2) : 0.0;
-        er = (sd.uv_swap ? eu : ev) + margin;
-        ec = (sd.uv_swap ? ev : eu) + margin;
+        er = sd.uv_swap ? eu : ev;
+        ec = sd.uv_swap ? ev : eu;
     }
     const bool fits = sd.n_img == sd.g.n_ch && er < H && ec < H &&
                       (((int)er + 2) & ~1) * (int64_t)max(2 * (int)ec + 1, kMinStride) <= cap;
@@ -412,11 +409,7 @@ k_grid_rows_direct_win(SetDesc first, const SetDesc* __restrict__ sets,
         const int j = c <= e_c ? c : (c >= N - e_c ? c - c_shift : -1);
         return j >= 0 ? &tile[r * s + j] : nullptr;
     };
-    int n_ok;
-    if constexpr (kKb)
-        n_ok = kb_walk<true>(sd, img, ch, N, 0, n_win, tid, NT, at, &outside);
-    else
-        n_ok = direct_walk<2, true>(sd, img, ch, N, 0, n_win, tid, NT, at, &outside);
+    const int n_ok = direct_walk<2, true>(sd, img, ch, N, 0, n_win, tid, NT, at, &outside);
     if (__syncthreads_or(outside ? 1 : 0)) {
         if (tid == 0) rsg[N] = -1;
         return;
@@ -435,8 +428,7 @@ k_grid_rows_direct_win(SetDesc first, const SetDesc* __restrict__ sets,
 // images of a channel with several timesteps see it too).  Workgroups take
 // the chunk's images in turn and return at once for the windowed ones.
 // (NT = 512: the walk and two-row transforms in one loop fit its registers.)
-// kKb: convolutional gridding (kb_walk).
-template <int N, int NT, bool kMulti, bool kKb>
+template <int N, int NT, bool kMulti>
 __global__ void __launch_bounds__(NT)
 k_grid_rows_direct_blocks(SetDesc first, const SetDesc* __restrict__ sets,
                           const int* __restrict__ img_set, int64_t gi0, int n_img,
@@ -467,10 +459,7 @@ k_grid_rows_direct_blocks(SetDesc first, const SetDesc* __restrict__ sets,
             for (int i = tid; i < ((nr + 1) & ~1) * N; i += NT) tile[i] = make_float2(0.f, 0.f);
             __syncthreads();
             auto at = [&](int r, int c) { return &tile[r * N + c]; };
-            if constexpr (kKb)
-                n_ok += kb_walk<false>(sd, img, ch, N, r0, nr, tid, NT, at, nullptr);
-            else
-                n_ok += direct_walk<2>(sd, img, ch, N, r0, nr, tid, NT, at);
+            n_ok += direct_walk<2>(sd, img, ch, N, r0, nr, tid, NT, at);
             __syncthreads();
             win_transform_rows<N, NT, true>(tile, r0, nr, N, 0, li, inter, twl,
                                             sd.cached_inter != 0);
@@ -1140,7 +1129,7 @@ bool batch_direct_supported(int n) {
 
 bool direct_uses_window(int n) { return n == kDirectWinSide; }
 
-template <int N, int NT, bool kKb>
+template <int N, int NT>
 static hipError_t launch_rows_direct_win_t(const SetDesc& first, const SetDesc* sets,
                                            const int* img_set, int n_sets, int64_t gi0,
                                            int n_img, float* inter, const float* tw,
@@ -1150,15 +1139,15 @@ static hipError_t launch_rows_direct_win_t(const SetDesc& first, const SetDesc* 
     const int64_t cap = g_lds_limit / (int64_t)sizeof(float2) - N;
     if (((cap / N) & ~1) < 2) return hipErrorInvalidConfiguration;
     const size_t lds = sizeof(float2) * (size_t)(cap + N);
-    auto k = n_sets == 1 ? k_grid_rows_direct_win<N, NT, false, kKb>
-                         : k_grid_rows_direct_win<N, NT, true, kKb>;
+    auto k = n_sets == 1 ? k_grid_rows_direct_win<N, NT, false>
+                         : k_grid_rows_direct_win<N, NT, true>;
     hipLaunchKernelGGL(k, dim3((unsigned)n_img), dim3(NT), lds, stream, first, sets, img_set, gi0,
                        (float2*)inter, (const float2*)tw, (int)cap);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // the images the window does not hold: a workgroup per CU takes them in turn
-    auto kb = n_sets == 1 ? k_grid_rows_direct_blocks<N, kDirectBlockThreads, false, kKb>
-                          : k_grid_rows_direct_blocks<N, kDirectBlockThreads, true, kKb>;
+    auto kb = n_sets == 1 ? k_grid_rows_direct_blocks<N, kDirectBlockThreads, false>
+                          : k_grid_rows_direct_blocks<N, kDirectBlockThreads, true>;
     const int blocks = (int)std::min<int64_t>(n_img, std::max(1, device_cu_count()));
     hipLaunchKernelGGL(kb, dim3((unsigned)blocks), dim3(kDirectBlockThreads), lds, stream, first,
                        sets, img_set,
@@ -1170,13 +1159,10 @@ hipError_t launch_grid_rows_direct(const SetDesc& first, const SetDesc* sets, co
                                    int n_sets, int n, int64_t gi0, int n_img, float* inter,
                                    const float* tw, hipStream_t stream) {
     if (n_img == 0) return hipSuccess;
+    if (first.kb_size > 0) return hipErrorNotSupported;
     if (n == kDirectWinSide)
-        return first.kb_size > 0
-                   ? launch_rows_direct_win_t<kDirectWinSide, kDirectWinThreads, true>(
-                         first, sets, img_set, n_sets, gi0, n_img, inter, tw, stream)
-                   : launch_rows_direct_win_t<kDirectWinSide, kDirectWinThreads, false>(
-                         first, sets, img_set, n_sets, gi0, n_img, inter, tw, stream);
-    if (first.kb_size > 0) return hipErrorNotSupported;  // convolutional: the window side only
+        return launch_rows_direct_win_t<kDirectWinSide, kDirectWinThreads>(
+            first, sets, img_set, n_sets, gi0, n_img, inter, tw, stream);
 #define X(NN, T) \
     if (n == NN) \
         return launch_rows_direct_t<NN, T>(first, sets, img_set, n_sets, gi0, n_img, inter, tw, \
@@ -1218,14 +1204,10 @@ hipError_t set_batch_kernel_attributes() {
     BLINK_DIRECT_VARIANTS(X)
 #undef X
     for (const void* f :
-         {(const void*)k_grid_rows_direct_win<kDirectWinSide, kDirectWinThreads, false, false>,
-          (const void*)k_grid_rows_direct_win<kDirectWinSide, kDirectWinThreads, true, false>,
-          (const void*)k_grid_rows_direct_win<kDirectWinSide, kDirectWinThreads, false, true>,
-          (const void*)k_grid_rows_direct_win<kDirectWinSide, kDirectWinThreads, true, true>,
-          (const void*)k_grid_rows_direct_blocks<kDirectWinSide, kDirectBlockThreads, false, false>,
-          (const void*)k_grid_rows_direct_blocks<kDirectWinSide, kDirectBlockThreads, true, false>,
-          (const void*)k_grid_rows_direct_blocks<kDirectWinSide, kDirectBlockThreads, false, true>,
-          (const void*)k_grid_rows_direct_blocks<kDirectWinSide, kDirectBlockThreads, true, true>})
+         {(const void*)k_grid_rows_direct_win<kDirectWinSide, kDirectWinThreads, false>,
+          (const void*)k_grid_rows_direct_win<kDirectWinSide, kDirectWinThreads, true>,
+          (const void*)k_grid_rows_direct_blocks<kDirectWinSide, kDirectBlockThreads, false>,
+          (const void*)k_grid_rows_direct_blocks<kDirectWinSide, kDirectBlockThreads, true>})
         set(f);
 #define X(NN, T)                                  \
     set((const void*)k_cols_reg<NN, T, false>);   \

@@ -815,6 +815,7 @@ struct BatchGroup {
     // direct row pass (no plan): dense sets with a plan per image
     bool direct = false;
     int direct_work = 0;  // the largest n_img or n_bl of its sets (launch_direct_prep)
+    int kb_max_bl = 0, kb_max_ch = 0;  // convolutional gridding (launch_kb_cells)
 };
 
 struct BatchPlan {
@@ -999,6 +1000,18 @@ static int build_batch(blink_ctx* ctx, const blink_image_set* sets, int n_sets, 
         g.direct_work = work;
         for (int i : g.sets) set_direct[i] = 1;
     }
+    // convolutional gridding needs no plan: its row pass finds a slab's
+    // footprints in the cells of each channel (launch_kb_cells)
+    for (BatchGroup& g : bp.groups) {
+        if (!g.kb_size) continue;
+        for (int i : g.sets) {
+            const int n_bl = sets[i].n_ant * (sets[i].n_ant + 1) / 2;
+            g.direct_work = std::max<int>({g.direct_work, n_bl, sets[i].n_ch * sets[i].n_t});
+            g.kb_max_bl = std::max(g.kb_max_bl, n_bl);
+            g.kb_max_ch = std::max(g.kb_max_ch, sets[i].n_ch);
+            set_direct[i] = 1;
+        }
+    }
     // scratch sizes of the plans
     size_t rs_bytes = 0, en_bytes = 0;
     std::vector<size_t> rs_off(n_sets), en_off(n_sets), is_off(n_sets), co_off(n_sets);
@@ -1016,6 +1029,8 @@ static int build_batch(blink_ctx* ctx, const blink_image_set* sets, int n_sets, 
         co_off[i] = (size_t)n_bl_all;
         n_bl_all += n_bl;
         en_off[i] = en_bytes;
+        if (st.kernel_size > 0)
+            en_bytes += align16(sizeof(uint32_t) * (size_t)st.n_ch * kb_cell_stride(n_bl));
         if (set_direct[i]) continue;  // no plan
         en_bytes += align16(sizeof(uint32_t) * 2 * (size_t)st.n_ch * std::max(n_bl, 1));
         n_units += st.n_ch;
@@ -1250,13 +1265,11 @@ static int build_batch(blink_ctx* ctx, const blink_image_set* sets, int n_sets, 
             d.kb_size = st.kernel_size;
             d.kb_table = bp.sc[i].kb_table;
             // (the FFT groups' direct row passes write the row starts instead)
-            d.all_rows = (st.kernel_size > 0 && !g.direct) || (g.direct && is_dft(g.transform))
-                             ? 1
-                             : 0;
+            d.all_rows = st.kernel_size > 0 || (g.direct && is_dft(g.transform)) ? 1 : 0;
             d.cached_inter = g.cached_inter ? 1 : 0;
             // the windowed direct row pass's |u|, |v| maxima: in the row
             // lists, which no direct set uses (n_ch (N + 3) >= 2 kUvMaxParts)
-            d.uv_max = g.direct && !is_dft(g.transform) && direct_uses_window(g.n)
+            d.uv_max = g.direct && !g.kb_size && !is_dft(g.transform) && direct_uses_window(g.n)
                            ? (float*)bp.sc[i].row_list
                            : nullptr;
             base += d.n_img;
@@ -1564,7 +1577,9 @@ static int enqueue_chunks(blink_ctx* ctx, const blink_image_set* sets, const Bat
     make_fft_plan(n, plan);
     const std::pair<int, int> tl = tiles_for(ctx, g);
     // the direct row pass's count sums and phase coefficients
-    if (g.direct) LAUNCH("direct_prep", s, launch_direct_prep(sd, ns, g.direct_work, s));
+    if (g.direct || g.kb_size)
+        LAUNCH(g.direct ? "direct_prep" : "plan", s, launch_direct_prep(sd, ns, g.direct_work, s));
+    if (g.kb_size) LAUNCH("kb_cells", s, launch_kb_cells(sd, ns, g.kb_max_bl, g.kb_max_ch, s));
     // the second pass is skipped when no set of the group forms its images
     bool any_images = false;
     for (int i : g.sets) any_images |= sets[i].images != nullptr;
@@ -1583,9 +1598,9 @@ static int enqueue_chunks(blink_ctx* ctx, const blink_image_set* sets, const Bat
         // the buffer's previous chunk (k - 2) must have been read
         if (two && k >= 2)
             HIP_TRY(hipStreamWaitEvent(s, ctx->pass_ev[2 * ((k - 2) % kPassEvents) + 1], 0));
-        if (g.direct && g.kb_size)
+        if (g.kb_size)
             LAUNCH("grid_rows_kb", s,
-                   launch_grid_rows_direct(first, sd, is, ns, n, gi0, cnt, buf, tw, s));
+                   launch_grid_rows_kb(first, sd, is, ns, plan, gi0, cnt, buf, tw, g.kb_blocked, s));
         else if (g.direct && g.reg)
             LAUNCH("grid_rows_fft", s,
                    launch_grid_rows_direct(first, sd, is, ns, n, gi0, cnt, buf, tw, s));
@@ -1596,10 +1611,6 @@ static int enqueue_chunks(blink_ctx* ctx, const blink_image_set* sets, const Bat
             LAUNCH("grid_rows_fft", s,
                    launch_grid_rows_reg(first, sd, is, ns, n, tl.first, gi0, cnt, buf, tw, s,
                                         g.uniform));
-        else if (g.kb_size)
-            LAUNCH("grid_rows_kb", s,
-                   launch_grid_rows_kb(first, sd, is, ns, plan, gi0, cnt, buf, tw, g.kb_blocked,
-                                       s));
         else
             LAUNCH("grid_rows_fft", s,
                    launch_grid_rows_fft(first, sd, is, ns, plan, gi0, cnt, buf, tw, s));

@@ -5,6 +5,7 @@
 #include "blink_gather.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace blink {
 
@@ -514,44 +515,35 @@ k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
     }
 }
 
-// Row slabs in LDS.  Workgroup (slab, image) owns the consecutive grid rows
-// slab * rows .. + rows - 1.  It walks the cells of its channel (k_stage_cells)
-// a chunk at a time, queues (baseline, sign) wherever the nearest row of that
-// footprint lies within K / 2 rows (cyclically: a superset of the footprints
-// that reach the slab), and each thread then spreads one queued footprint over
-// the slab's rows, only those it reaches (a mask), so that the lanes of a
-// wavefront take at most `rows` turns.  At the end the
-// non-zero cells are added to the global grid; no other workgroup touches them.
+// Footprints of the rows r0 .. r0 + nr - 1 (grid rows v, or with kSwap grid columns
+// u) accumulated in LDS planes re, im [nr][n].  The workgroup walks the cells
+// of a channel (packed row << 16 | position, `stride` of them) a chunk at a time,
+// queues (baseline, sign) wherever the nearest row of that footprint lies
+// within K / 2 rows (cyclically: a superset of the footprints that reach the
+// rows), and each thread then spreads one queued footprint over those of its
+// rows that are here (a mask, so that the lanes of a wavefront take few
+// turns).  value(bl) gives the visibility; count(row, position) is called once
+// per gridded nearest cell in the rows.
 // The work is the K x K updates of every footprint.  The cells are FP64 planes:
 // ds_add_f64 costs 21 clocks per wavefront instruction whatever collides, where
 // the footprints of a dense core make compare-and-swaps of FP32 cells retry.
-// kX: largest K whose weights along u stay in registers; each weight read in
+// kX: largest K whose weights along a row stay in registers; each weight read in
 // the inner loop would be a gather of 64 cache lines per wavefront.
-constexpr int kKbThreads = 512, kKbVec = 3;
-constexpr int kKbChunk = kKbThreads * 4 * kKbVec;
-static_assert(2 * kKbChunk <= 32768, "queue entries: 15-bit offset and a sign");
-template <int kX>
-__global__ void __launch_bounds__(kKbThreads)
-k_grid_kb_slabs(StageGrid g, int rows, int stride, const uint32_t* __restrict__ cells, int K,
-                const double* __restrict__ kt) {
+// Returns the number of footprints queued.
+constexpr int kb_chunk(int nt, int vec) { return nt * 4 * vec; }  // baselines per chunk
+constexpr size_t kb_queue_bytes(int nt, int vec) {
+    return 2 * sizeof(unsigned short) * (size_t)kb_chunk(nt, vec);
+}
+template <int NT, int kVec, int kX, bool kSwap, class Value, class Count>
+__device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int K,
+                                              const double* __restrict__ kt,
+                                              const uint32_t* __restrict__ cl, int stride, int r0,
+                                              int nr, double* re, double* im,
+                                              unsigned short* queue, int* n_queued, Value value,
+                                              Count count) {
 #pragma clang fp contract(off)
-    extern __shared__ float4 kb_slabs_lds4[];
-    const int n = g.n_pixels, mid = K / 2;
-    double* re = (double*)kb_slabs_lds4;                     // [rows][n]
-    double* im = re + (size_t)rows * n;                      // [rows][n]
-    unsigned* cnt = (unsigned*)(im + (size_t)rows * n);      // [rows][n]
-    unsigned short* queue = (unsigned short*)(cnt + (size_t)rows * n);  // [2 kKbChunk]
-    __shared__ int n_queued;
-    const int n_slab = (n + rows - 1) / rows;
-    const int r0 = (int)(blockIdx.x % (unsigned)n_slab) * rows, nr = min(rows, n - r0);
-    const int64_t img = blockIdx.x / (unsigned)n_slab;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const uint32_t* cl = cells + (img % g.n_ch) * stride;
-    const double wl = wavelength_of(g.freq_hz[img % g.n_ch]);
-    for (int i = tid; i < rows * n; i += kKbThreads) {
-        re[i] = im[i] = 0.0;
-        cnt[i] = 0u;
-    }
+    static_assert(kVec <= 4 && 2 * kb_chunk(NT, kVec) <= 65536, "queue entries: 15-bit offset and a sign");
+    const int n = g.n_pixels, mid = K / 2, tid = threadIdx.x, lane = tid & 63;
     // rows r0 - reach .. r0 + nr - 1 + reach (kb_cell places the negative rows of
     // an odd side one lower than wrap_index does)
     const int reach = mid + (n & 1), span = nr + 2 * reach;
@@ -560,27 +552,25 @@ k_grid_kb_slabs(StageGrid g, int rows, int stride, const uint32_t* __restrict__ 
         d = d < 0 ? d + n : (d >= n ? d - n : d);
         return d < span || span >= n;
     };
-    for (int base = 0; base < stride; base += kKbChunk) {
-        if (tid == 0) n_queued = 0;
+    int total = 0;
+    for (int base = 0; base < stride; base += kb_chunk(NT, kVec)) {
+        if (tid == 0) *n_queued = 0;
         __syncthreads();
-        uint4 p[kKbVec];
-#pragma unroll
-        for (int k = 0; k < kKbVec; k++) {
-            const int b = base + 4 * (tid + k * kKbThreads);
-            p[k] = b < stride ? *(const uint4*)&cl[b]
-                              : make_uint4(kNoCell, kNoCell, kNoCell, kNoCell);
-        }
         unsigned keep = 0;  // two bits per baseline: its own footprint, its conjugate's
 #pragma unroll
-        for (int k = 0; k < kKbVec; k++)
+        for (int k = 0; k < kVec; k++) {
+            const int b = base + 4 * (tid + k * NT);
+            const uint4 p = b < stride ? *(const uint4*)&cl[b]
+                                       : make_uint4(kNoCell, kNoCell, kNoCell, kNoCell);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const uint32_t c = j == 0 ? p[k].x : j == 1 ? p[k].y : j == 2 ? p[k].z : p[k].w;
+                const uint32_t c = j == 0 ? p.x : j == 1 ? p.y : j == 2 ? p.z : p.w;
                 if (c == kNoCell) continue;
                 const int r = (int)(c >> 16);
                 if (near(r)) keep |= 1u << (8 * k + 2 * j);
                 if (near(r == 0 ? 0 : n - r)) keep |= 2u << (8 * k + 2 * j);
             }
+        }
         int before = __popc(keep);
         const int own = before;
         for (int o = 1; o < 64; o <<= 1) {
@@ -588,65 +578,99 @@ k_grid_kb_slabs(StageGrid g, int rows, int stride, const uint32_t* __restrict__ 
             if (lane >= o) before += t;
         }
         int at = 0;
-        if (lane == 63) at = atomicAdd(&n_queued, before);
+        if (lane == 63) at = atomicAdd(n_queued, before);
         at = __shfl(at, 63, 64) + before - own;
         while (keep) {
             const int bit = __ffs(keep) - 1;
             keep &= keep - 1;
-            queue[at++] = (unsigned short)((4 * (tid + (bit >> 3) * kKbThreads) + ((bit >> 1) & 3)) * 2 +
+            queue[at++] = (unsigned short)((4 * (tid + (bit >> 3) * NT) + ((bit >> 1) & 3)) * 2 +
                                            (bit & 1));
         }
         __syncthreads();
-        const int nq = n_queued;
-        for (int i = tid; i < nq; i += kKbThreads) {
+        const int nq = *n_queued;
+        total += nq;
+        for (int i = tid; i < nq; i += NT) {
             const int q = queue[i], bl = base + (q >> 1), s = (q & 1) ? -1 : 1;
-            const float2 v = stage_value(g, img, bl);
+            const float2 v = value(bl);
             KbSpot sp;
             if (!vis_ok(v) || !kb_spot(g, wl, bl, K, kt, sp)) continue;
-            const int rn = wrap_index(s * sp.vp, n) - r0;
-            if ((unsigned)rn < (unsigned)nr) atomicAdd(&cnt[rn * n + wrap_index(s * sp.up, n)], 1u);
-            double xw[kX > 0 ? kX : 1];
-            int xc[kX > 0 ? kX : 1];
+            const int rp = kSwap ? sp.up : sp.vp, cp = kSwap ? sp.vp : sp.up;
+            const double* rk = kSwap ? sp.xk : sp.yk;
+            const double* ck = kSwap ? sp.yk : sp.xk;
+            const int rn = wrap_index(s * rp, n) - r0;
+            if ((unsigned)rn < (unsigned)nr) count(rn, wrap_index(s * cp, n));
+            double cw[kX > 0 ? kX : 1];
+            int cx[kX > 0 ? kX : 1];
             if constexpr (kX > 0) {
 #pragma unroll
                 for (int c = 0; c < kX; c++) {
-                    xc[c] = -1;
+                    cx[c] = -1;
                     if (c >= K) continue;
-                    xw[c] = sp.xk[c];
+                    cw[c] = ck[c];
                     int x;
-                    if (kb_cell(sp.up - mid + c, s, n, x)) xc[c] = x;
+                    if (kb_cell(cp - mid + c, s, n, x)) cx[c] = x;
                 }
             }
-            unsigned hit = 0;  // rows j of the footprint in this slab
+            unsigned hit = 0;  // rows j of the footprint that are here
             for (int j = 0; j < K; j++) {
                 int y;
-                if (kb_cell(sp.vp - mid + j, s, n, y) && (unsigned)(y - r0) < (unsigned)nr) hit |= 1u << j;
+                if (kb_cell(rp - mid + j, s, n, y) && (unsigned)(y - r0) < (unsigned)nr) hit |= 1u << j;
             }
             for (; hit; hit &= hit - 1) {
                 const int j = __ffs(hit) - 1;
                 int y = 0;
-                kb_cell(sp.vp - mid + j, s, n, y);
-                const double wy = sp.yk[j];
+                kb_cell(rp - mid + j, s, n, y);
+                const double wr = rk[j];
                 const int row = (y - r0) * n;
-                auto put = [&](int x, double wx) {
-                    const double w = wy * wx;
+                auto put = [&](int x, double wc) {
+                    const double w = wr * wc;
                     atomicAdd(&re[row + x], (double)v.x * w);
                     atomicAdd(&im[row + x], (double)s * (double)v.y * w);
                 };
                 if constexpr (kX > 0) {
 #pragma unroll
                     for (int c = 0; c < kX; c++)
-                        if (xc[c] >= 0) put(xc[c], xw[c]);
+                        if (cx[c] >= 0) put(cx[c], cw[c]);
                 } else {
                     for (int c = 0; c < K; c++) {
                         int x;
-                        if (kb_cell(sp.up - mid + c, s, n, x)) put(x, sp.xk[c]);
+                        if (kb_cell(cp - mid + c, s, n, x)) put(x, ck[c]);
                     }
                 }
             }
         }
         __syncthreads();
     }
+    return total;
+}
+
+// Stage path: workgroup (slab, image) owns `rows` consecutive grid rows; at the
+// end the non-zero cells are added to the global grid (no other workgroup
+// touches them).
+constexpr int kKbThreads = 512, kKbVec = 2;
+template <int kX>
+__global__ void __launch_bounds__(kKbThreads)
+k_grid_kb_slabs(StageGrid g, int rows, int stride, const uint32_t* __restrict__ cells, int K,
+                const double* __restrict__ kt) {
+    extern __shared__ float4 kb_slabs_lds4[];
+    const int n = g.n_pixels;
+    double* re = (double*)kb_slabs_lds4;                     // [rows][n]
+    double* im = re + (size_t)rows * n;                      // [rows][n]
+    unsigned* cnt = (unsigned*)(im + (size_t)rows * n);      // [rows][n]
+    unsigned short* queue = (unsigned short*)(cnt + (size_t)rows * n);
+    __shared__ int n_queued;
+    const int n_slab = (n + rows - 1) / rows;
+    const int r0 = (int)(blockIdx.x % (unsigned)n_slab) * rows, nr = min(rows, n - r0);
+    const int64_t img = blockIdx.x / (unsigned)n_slab;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < rows * n; i += kKbThreads) {
+        re[i] = im[i] = 0.0;
+        cnt[i] = 0u;
+    }
+    kb_accumulate<kKbThreads, kKbVec, kX, false>(
+        g, wavelength_of(g.freq_hz[img % g.n_ch]), K, kt, cells + (img % g.n_ch) * stride, stride,
+        r0, nr, re, im, queue, &n_queued, [&](int bl) { return stage_value(g, img, bl); },
+        [&](int r, int c) { atomicAdd(&cnt[r * n + c], 1u); });
     float2* grid = g.grids + img * (int64_t)n * n + (int64_t)r0 * n;
     float* counts = g.counts + img * (int64_t)n * n + (int64_t)r0 * n;
     for (int i = tid; i < nr * n; i += kKbThreads) {
@@ -660,7 +684,9 @@ k_grid_kb_slabs(StageGrid g, int rows, int stride, const uint32_t* __restrict__ 
     }
 }
 
-static size_t kb_slab_lds(int n, int rows) { return (size_t)20 * n * rows + 4 * kKbChunk; }
+static size_t kb_slab_lds(int n, int rows) {
+    return (size_t)20 * n * rows + kb_queue_bytes(kKbThreads, kKbVec);
+}
 
 // Rows per slab: up to 8 (the wider, the fewer slabs compute a footprint's
 // weights again), fewer while that leaves under four workgroups per CU or
@@ -1565,118 +1591,102 @@ hipError_t launch_grid_rows_direct_fft(const SetDesc& first, const SetDesc* sets
     return hipGetLastError();
 }
 
-// Convolutional gridding fused with the row FFT (generic kernels, transposed
-// plan: plan rows are grid columns x, positions rows y).  Workgroup = (tile of
-// rb consecutive plan rows r0 .. r1 of 0 .. N/2, image).  Every visibility
-// that is gridded adds its K x K footprint around its nearest cell (u, v) with
-// value V and, mirrored, around (-u, -v) with conj(V) (convolve_with_kernel,
-// src/pacer_imager.cpp:654-714, placed as calc_xy_grid2 places it, :716-750).
-// The plan lists, per visibility, the one of its two nearest cells that falls
-// in rows 1 .. N/2-1 (its partner is in row N - p), or both when they fall in
-// rows 0 and N/2.  A footprint around row p covers rows p - K/2 .. p + K/2,
-// so a tile gathers the entries of rows r0 - K/2 .. r1 + K/2 and, when r1 +
-// K/2 reaches N/2, of rows N - r1 - K/2 .. N/2 (their partners' footprints
-// reach back below N/2); each entry adds its own footprint and, for rows 1 ..
-// N/2-1, its partner's, keeping the cells in rows r0 .. r1.  Counts stay at
-// the nearest cells, as the reference keeps them.  Every row of the tile is
-// transformed and written, row-major or, for the register sides, in the
-// column-blocked layout of the register second pass.
-template <int S, bool kBlockTeam, bool kMulti>
-__global__ void __launch_bounds__(kFftThreads)
-k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __restrict__ img_set,
-               FftPlan plan, int team, int rb, int64_t gi0, float2* __restrict__ inter,
-               const float2* __restrict__ tw, int blocked) {
-#pragma clang fp contract(off)
-    extern __shared__ float4 grk_lds4[];
-    const int n = plan.n;
-    float2* tile = (float2*)grk_lds4;  // [rb][n]
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* tmp = tile + (size_t)rb * n + (size_t)t_id * n;
-    __shared__ int red[kFftThreads / 64];
+// Cells of a group's sets for the row pass below, as the plan's count pass packs
+// them: SetDesc::entries holds kb_cell_stride(n_bl) words per channel.
+__global__ void __launch_bounds__(256)
+k_kb_cells(const SetDesc* __restrict__ sets) {
+    const SetDesc sd = sets[blockIdx.z];
+    const int n_bl = sd.g.n_bl, n = sd.n_pixels, stride = kb_cell_stride(n_bl);
+    const int bl = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (bl >= stride) return;
+    for (int ch = blockIdx.y; ch < sd.g.n_ch; ch += gridDim.y) {
+        uint32_t packed = kNoCell;
+        int up, vp;
+        if (bl < n_bl && !sd.flags[bl] &&
+            plan_cell(sd.u_m[bl], sd.v_m[bl], CellUnit(sd.g.freq_hz[ch], sd), sd, up, vp))
+            packed = ((uint32_t)wrap_index(up, n) << 16) | (uint32_t)wrap_index(vp, n);
+        sd.entries[(int64_t)ch * stride + bl] = packed;
+    }
+}
 
-    const int h = n / 2;
-    const int n_rb = (h + 1 + rb - 1) / rb;
-    const unsigned nwg = gridDim.x;
-    unsigned bid = blockIdx.x;
-    if ((nwg & 7u) == 0) bid = (bid & 7u) * (nwg >> 3) + (bid >> 3);
-    const int tile_id = (int)(bid % n_rb);
-    const int li = (int)(bid / n_rb);
+hipError_t launch_kb_cells(const SetDesc* sets, int n_sets, int max_bl, int max_ch,
+                           hipStream_t stream) {
+    if (n_sets == 0 || max_bl == 0 || max_ch == 0) return hipSuccess;
+    if (n_sets > 65535) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL(k_kb_cells,
+                       dim3((unsigned)((kb_cell_stride(max_bl) + 255) / 256),
+                            (unsigned)std::min(max_ch, 65535), (unsigned)n_sets),
+                       dim3(256), 0, stream, sets);
+    return hipGetLastError();
+}
+
+// Row pass of convolutional gridding, any side: workgroup (slab, image) owns
+// `rb` consecutive plan rows (grid columns u) of 0 .. N/2, accumulates their
+// footprints in FP64 (kb_accumulate), transforms each row (the planes become
+// the row and its Stockham partner) and writes it, row-major or in the
+// column-blocked layout of the register second pass.  The slabs nearest u = 0,
+// the dense core, are launched first.  It measured, against a gather of plan
+// entries with FP32 cells (and a window of the plane at 256^2) before: 256
+// channels x 256^2, K = 7, 1336 -> see launch_grid_rows_kb.
+constexpr int kKbRowThreads = 1024;
+// (one row of 8192 cells and the queue of one vector per thread fit a CU)
+constexpr int kb_row_vec(bool wide) { return wide ? 1 : 2; }
+template <int kX, bool kBlockTeam, bool kMulti>
+__global__ void __launch_bounds__(kKbRowThreads)
+k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __restrict__ img_set,
+               FftPlan plan, int team, int rb, int64_t gi0, int n_img, float2* __restrict__ inter,
+               const float2* __restrict__ tw, int blocked) {
+    extern __shared__ float4 grk_lds4[];
+    const int n = plan.n, h = n / 2, tid = threadIdx.x;
+    double* re = (double*)grk_lds4;      // [rb][n]
+    double* im = re + (size_t)rb * n;    // [rb][n]
+    unsigned short* queue = (unsigned short*)(im + (size_t)rb * n);
+    __shared__ int n_queued;
+    __shared__ int red[kKbRowThreads / 64];
+    const int li = (int)(blockIdx.x % (unsigned)n_img);
+    const int r0 = (int)(blockIdx.x / (unsigned)n_img) * rb, nr = min(rb, h + 1 - r0);
     const int64_t gi = gi0 + li;
     const SetDesc sd = set_of<kMulti>(first, sets, img_set, gi);
     const GatherArgs& g = sd.g;
-    const int img = (int)(gi - sd.img_base);
-    const int ch = img % g.n_ch;
-    const int r0 = tile_id * rb;
-    const int nr = min(rb, h + 1 - r0);
-    const int r1 = r0 + nr - 1;
-    const int K = sd.kb_size, mid = K / 2;
-    int lo = max(0, r0 - mid);
-    const int hi = min(h, r1 + mid);
-    if (r1 + mid >= h) lo = max(0, min(lo, n - r1 - mid));
-    const int* rsg = sd.row_start + (int64_t)ch * (n + 1);
-    const int e0 = rsg[lo], e1 = rsg[hi + 1];
-    for (int i = threadIdx.x; i < nr * n; i += blockDim.x) tile[i] = make_float2(0.f, 0.f);
-    __syncthreads();
-
-    const uint32_t* ent = sd.entries + (int64_t)ch * 2 * g.n_bl;
+    const int img = (int)(gi - sd.img_base), ch = img % g.n_ch;
+    for (int i = tid; i < nr * n; i += kKbRowThreads) re[i] = im[i] = 0.0;
+    const StageGrid sg{nullptr, sd.u_m, sd.v_m, sd.flags, g.freq_hz, sd.du, sd.dv, sd.min_uv,
+                       g.n_bl, g.n_ch, n, g.pol, nullptr, nullptr};
     const float2* rec = (const float2*)g.vis + 4 * ((int64_t)img * g.n_bl);
     const double nu = g.freq_hz[ch];
-    const double wl = wavelength_of(nu);
     const int p0 = g.pol == 1 ? 3 : (g.pol == 3 ? 1 : 0);
     const int p1 = g.pol == 3 ? 2 : 3;
+    const int stride = kb_cell_stride(g.n_bl);
     int n_ok = 0;
-    for (int e = e0 + (int)threadIdx.x; e < e1; e += (int)blockDim.x) {
-        const uint32_t ev = ent[e];
-        const unsigned bl = ev >> 14;
-        const int own = (ev >> 13) & 1u ? -1 : 1;  // sign of the listed cell
-        float2 v = select_pol2(rec[4 * (size_t)bl + p0],
-                               g.pol >= 2 ? rec[4 * (size_t)bl + p1] : make_float2(0.f, 0.f), g.pol);
-        if (g.corrections) v = cmul(v, unit_phasor(((g.phase_coef[bl] * nu) / kVelLight)));
-        if (!vis_ok(v)) continue;
-        int up, vp;
-        if (!cell_of(sd.u_m[bl], sd.v_m[bl], wl, sd.du, sd.dv, sd.min_uv, n, up, vp)) continue;
-        // the listed cell's plan row (its column x, as the plan wraps it), and
-        // the kernel rows of the fractional position
-        const int p = wrap_index(own * up, n);
-        if (p >= r0 && p <= r1) n_ok += (p == 0 || p == h) ? 1 : 2;
-        const double ue = (double)sd.u_m[bl] / wl / sd.du;
-        const double ve = (double)sd.v_m[bl] / wl / sd.dv;
-        int kx = (int)round((ue - (double)up) * 1023.0);
-        int ky = (int)round((ve - (double)vp) * 1023.0);
-        kx = (kx + 1534) % 1023;
-        ky = (ky + 1534) % 1023;
-        const double* xk = sd.kb_table + (int64_t)kx * K;
-        const double* yk = sd.kb_table + (int64_t)ky * K;
-        const int n_fp = (p == 0 || p == h) ? 1 : 2;  // own footprint, then the partner's
-        for (int f = 0; f < n_fp; f++) {
-            const int sgn = f == 0 ? own : -own;
-            for (int c = 0; c < K; c++) {
-                int x;
-                if (!kb_cell(up - mid + c, sgn, n, x) || x < r0 || x > r1) continue;
-                const double wx = xk[c];
-                float2* row = tile + (size_t)(x - r0) * n;
-                for (int j = 0; j < K; j++) {
-                    int y;
-                    if (!kb_cell(vp - mid + j, sgn, n, y)) continue;
-                    const double w = yk[j] * wx;
-                    lds_add(&row[y], (float)((double)v.x * w),
-                            (float)((double)sgn * (double)v.y * w));
-                }
-            }
-        }
-    }
+    const int queued = kb_accumulate<kKbRowThreads, kb_row_vec(kBlockTeam), kX, true>(
+        sg, wavelength_of(nu), sd.kb_size, sd.kb_table, sd.entries + (int64_t)ch * stride, stride,
+        r0, nr, re, im, queue, &n_queued,
+        [&](int bl) {
+            float2 v = select_pol2(rec[4 * (size_t)bl + p0],
+                                   g.pol >= 2 ? rec[4 * (size_t)bl + p1] : make_float2(0.f, 0.f),
+                                   g.pol);
+            if (g.corrections) v = cmul(v, unit_phasor(((g.phase_coef[bl] * nu) / kVelLight)));
+            return v;
+        },
+        // a nearest cell stands for its mirror too, except in the
+        // self-conjugate rows 0 and N/2, which hold both
+        [&](int r, int) { n_ok += (r0 + r == 0 || 2 * (r0 + r) == n) ? 1 : 2; });
     const int tot = block_sum_int(n_ok, red);
-    if (threadIdx.x == 0 && tot) atomicAdd(&sd.isums[img], (uint32_t)tot);
+    if (tid == 0 && tot) atomicAdd(&sd.isums[img], (uint32_t)tot);
+    // each cell's two sums become one FP32 complex value in its re slot
+    for (int i = tid; i < nr * n; i += kKbRowThreads) {
+        const float2 c = make_float2((float)re[i], (float)im[i]);
+        *(float2*)&re[i] = c;
+    }
     __syncthreads();
-    const int rounds = kBlockTeam ? nr : (nr + teams - 1) / teams;
+    const int teams = kBlockTeam ? 1 : kKbRowThreads / team;
+    const int t_id = kBlockTeam ? 0 : tid / team, lane = kBlockTeam ? tid : tid % team;
     const int64_t h1 = h + 1;
-    for (int k = 0; k < rounds; k++) {
-        const int r = kBlockTeam ? k : k * teams + t_id;
-        if (!kBlockTeam && r >= nr) break;
-        float2* row = tile + (size_t)r * n;
-        const float2* res = fft_row<S, kBlockTeam>(row, tmp, plan, tw, lane, team);
+    for (int r = t_id; r < nr; r += teams) {
+        const float2* res = (float2*)re + (size_t)r * n;
+        if (queued)  // (uniform) else zeros
+            res = fft_row<1, kBlockTeam>((float2*)re + (size_t)r * n, (float2*)im + (size_t)r * n,
+                                         plan, tw, lane, team);
         const int v = r0 + r;
         if (blocked) {  // element (v, x) at ((x / 32) (N/2+1) + v) 32 + x % 32
             float2* dst = inter + (int64_t)li * h1 * n + (int64_t)v * kInterBlockCols;
@@ -1697,28 +1707,30 @@ hipError_t launch_grid_rows_kb(const SetDesc& first, const SetDesc* sets, const 
                                float* inter, const float* tw, bool blocked, hipStream_t stream) {
     if (n_img == 0) return hipSuccess;
     if (first.kb_size < 1) return hipErrorInvalidValue;
-    const int n = plan.n;
-    const int team = fft_team_for(n);
-    const bool block_team = team == kFftThreads;
-    const int teams = block_team ? 1 : kFftThreads / team;
-    // rows per tile: a footprint covers K rows, so taller tiles re-read fewer
-    // entries; as many rows as fit up to 8, and at least ~2048 workgroups
-    const int64_t want = std::max<int64_t>(1, (int64_t)(n / 2 + 1) * n_img / 2048);
-    int rb = (int)std::max<int64_t>(
-        1, std::min<int64_t>({(int64_t)grid_rows_tile_rows(n), want, 8}));
-    auto lds_of = [&](int r) { return sizeof(float2) * ((size_t)r * n + (size_t)teams * n); };
-    while (rb > 1 && !lds_fits(lds_of(rb))) rb--;
-    const size_t lds = lds_of(rb);
-    if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-    const int n_rb = (n / 2 + 1 + rb - 1) / rb;
-    const int64_t blocks = (int64_t)n_rb * n_img;
-    if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-    const bool multi = n_sets > 1;
-    auto k = block_team
-                 ? (multi ? k_grid_rows_kb<1, true, true> : k_grid_rows_kb<1, true, false>)
-                 : (multi ? k_grid_rows_kb<1, false, true> : k_grid_rows_kb<1, false, false>);
-    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kFftThreads), lds, stream, first, sets,
-                       img_set, plan, team, rb, gi0, (float2*)inter, (const float2*)tw,
+    const int n = plan.n, h1 = n / 2 + 1;
+    const bool block_team = n > 1024;
+    const int team = block_team ? kKbRowThreads : fft_team_for(n);
+    // as many rows as a CU's LDS holds (the taller the slab, the fewer slabs
+    // compute a footprint's weights again), fewer while the images leave under
+    // four workgroups per CU (rows above the array's reach have no work)
+    const size_t queue = kb_queue_bytes(kKbRowThreads, kb_row_vec(block_team));
+    int rb = (int)std::min<int64_t>(h1, (g_lds_limit - (int64_t)queue) / (16 * (int64_t)n));
+    if (rb < 1) return hipErrorInvalidConfiguration;
+    while (rb > 2 && (int64_t)n_img * ((h1 + rb - 1) / rb) < 4 * device_cu_count()) rb = (rb + 1) / 2;
+    const size_t lds = (size_t)16 * n * rb + queue;
+    const int64_t blocks = (int64_t)n_img * ((h1 + rb - 1) / rb);
+    if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    // (a group's sets share kb_size)
+    auto pick = [&](auto kx) {
+        constexpr int X = decltype(kx)::value;
+        return block_team ? (n_sets > 1 ? k_grid_rows_kb<X, true, true> : k_grid_rows_kb<X, true, false>)
+                          : (n_sets > 1 ? k_grid_rows_kb<X, false, true>
+                                        : k_grid_rows_kb<X, false, false>);
+    };
+    const auto k = first.kb_size <= 8 ? pick(std::integral_constant<int, 8>{})
+                                      : pick(std::integral_constant<int, 0>{});
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kKbRowThreads), lds, stream, first, sets,
+                       img_set, plan, team, rb, gi0, n_img, (float2*)inter, (const float2*)tw,
                        blocked ? 1 : 0);
     return hipGetLastError();
 }
@@ -1903,10 +1915,6 @@ hipError_t set_kernel_attributes() {
         hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
         if (r != hipSuccess && e == hipSuccess) e = r;
     };
-    set((const void*)k_grid_rows_kb<1, true, false>);
-    set((const void*)k_grid_rows_kb<1, false, false>);
-    set((const void*)k_grid_rows_kb<1, true, true>);
-    set((const void*)k_grid_rows_kb<1, false, true>);
     set((const void*)k_grid_half_direct);
     set((const void*)k_grid_rows_direct_fft<false>);
     set((const void*)k_grid_rows_direct_fft<true>);
@@ -1925,6 +1933,13 @@ hipError_t set_kernel_attributes() {
     set((const void*)k_grid_slabs);
     set((const void*)k_grid_kb_slabs<8>);
     set((const void*)k_grid_kb_slabs<0>);
+#define X(K) \
+    set((const void*)k_grid_rows_kb<K, true, true>);  \
+    set((const void*)k_grid_rows_kb<K, true, false>); \
+    set((const void*)k_grid_rows_kb<K, false, true>); \
+    set((const void*)k_grid_rows_kb<K, false, false>);
+    X(8) X(0)
+#undef X
     set((const void*)k_grid_half_rows);
     set((const void*)k_plan_count);
     set((const void*)k_plan_scatter);

@@ -193,13 +193,16 @@ hipError_t launch_grid_rows_fft(const SetDesc& first, const SetDesc* sets, const
 hipError_t launch_cols_half(const SetDesc& first, const SetDesc* sets, const int* img_set,
                             int n_sets, const FftPlan& plan, int64_t gi0, int n_img,
                             const float* inter, const float* tw, hipStream_t stream);
-// Row pass of convolutional (Kaiser-Bessel) gridding on the generic kernels:
-// every plan row 0 .. N/2 of every image is gridded, transformed and written,
-// row-major as launch_grid_rows_fft writes or, with `blocked`, in the
-// column-blocked layout of the register second pass (N = 128 .. 2048); a
-// tile gathers the plan entries of its rows +- K/2 and, near row N/2, of the
-// rows whose Hermitian partners' footprints reach it.  The sets' kb_size must
-// be > 0.
+// Row pass of convolutional (Kaiser-Bessel) gridding, any side: every plan row
+// 0 .. N/2 of every image is gridded, transformed and written, row-major as
+// launch_grid_rows_fft writes or, with `blocked`, in the column-blocked layout
+// of the register second pass (N = 128 .. 2048).  It needs no plan: the sets'
+// cells (launch_kb_cells: SetDesc::entries, kb_cell_stride(n_bl) words per
+// channel) and, from launch_direct_prep, the count sums at zero and the phase
+// coefficients.  The sets' kb_size must be > 0.
+__host__ __device__ constexpr int kb_cell_stride(int n_bl) { return (n_bl + 3) & ~3; }
+hipError_t launch_kb_cells(const SetDesc* sets, int n_sets, int max_bl, int max_ch,
+                           hipStream_t stream);
 hipError_t launch_grid_rows_kb(const SetDesc& first, const SetDesc* sets, const int* img_set,
                                int n_sets, const FftPlan& plan, int64_t gi0, int n_img,
                                float* inter, const float* tw, bool blocked, hipStream_t stream);

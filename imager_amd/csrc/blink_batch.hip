@@ -407,7 +407,7 @@ k_grid_rows_direct_win(SetDesc first, const SetDesc* __restrict__ sets,
     bool outside = false;
     auto at = [&](int r, int c) -> float2* {
         const int j = c <= e_c ? c : (c >= N - e_c ? c - c_shift : -1);
-        return j >= 0 ? &tile[r * s + j] : nullptr;
+        return j >= 0 ? &tile[__mul24(r, s) + j] : nullptr;
     };
     const int n_ok = direct_walk<2, true>(sd, img, ch, N, 0, n_win, tid, NT, at, &outside);
     if (__syncthreads_or(outside ? 1 : 0)) {
@@ -617,7 +617,7 @@ __device__ __forceinline__ void vis_compact_one(const SetDesc& sd, int64_t img, 
         // that the compaction need not wait for the plan
         const double cf = phase_coefficient(g.corrections, sd.w_m, sd.cable_m, (unsigned)bl);
         const double nu = g.freq_hz[img % g.n_ch];
-        v = cmul(v, unit_phasor(((cf * nu) / kVelLight)));
+        v = cmul(v, unit_phasor(cf * (nu / kVelLight)));
     }
     if (!vis_ok(v)) v = make_float2(__builtin_nanf(""), __builtin_nanf(""));
     sd.compact[i] = v;

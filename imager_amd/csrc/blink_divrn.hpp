@@ -35,13 +35,10 @@ BLINK_HOST_DEVICE inline double div_rn(double a, double b, double y) {
 // when p is within 1e-6 of a half-integer, not finite, or |p| >= 2^29 (about
 // one cell in a million): the caller then takes the two divisions.
 BLINK_HOST_DEVICE inline bool round_quotient_fast(double a, double k, int& out) {
-    const double p = a * k;
-    if (!(std::fabs(p) < 536870912.0)) return false;
-    const double f = std::floor(p);
-    const double t = p - f;  // in [0, 1]; exact but for -0.5 < p < 0 (error < 2^-54)
-    if (std::fabs(t - 0.5) <= 1e-6) return false;
-    out = (int)f + (t > 0.5 ? 1 : 0);
-    return true;
+    const double p = a * k, q = std::rint(p);  // p - q is exact
+    out = (int)q;
+    // (false for NaN; no short circuit, which would be a branch)
+    return (int)(std::fabs(p - q) < 0.5 - 1e-6) & (int)(std::fabs(q) < 536870912.0);
 }
 
 // |x| in (1e-30, 1e30): no quotient, product or remainder of two such values

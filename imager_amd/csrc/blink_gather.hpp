@@ -77,7 +77,7 @@ struct GatherBatch {
         for (int u = 0; u < U; u++) {
             if (idx[u] < 0) continue;
             float2 v = select_pol2(x0[u], x1[u], g.pol);
-            if (g.corrections) v = cmul(v, unit_phasor(((cf[u] * nu) / kVelLight)));
+            if (g.corrections) v = cmul(v, unit_phasor(cf[u] * (nu / kVelLight)));
             if (!vis_ok(v)) continue;
             if (ev[u] & (1u << 13)) v.y = -v.y;
             total += sink(idx[u], (int)(ev[u] & 0x1fffu), v);
@@ -119,8 +119,10 @@ __device__ __forceinline__ bool plan_cell(float u_m, float v_m, const CellUnit& 
 #pragma clang fp contract(off)
     if (sd.min_uv == -INFINITY) {
         const double um = (double)u_m, vm = (double)v_m;
-        if (cu.fast && round_quotient_fast(um, cu.ku, up) && round_quotient_fast(vm, cu.kv, vp))
-            return true;
+        // (both evaluated: one branch instead of two nested ones)
+        const bool qu_fast = round_quotient_fast(um, cu.ku, up);
+        const bool qv_fast = round_quotient_fast(vm, cu.kv, vp);
+        if ((int)cu.fast & (int)qu_fast & (int)qv_fast) return true;
         const bool fast = cu.fast && div_rn_range(um) && div_rn_range(vm);
         double u, v, qu, qv;
         if (fast) {
@@ -176,18 +178,22 @@ struct WalkBatch {
     // next round in flight while this round is consumed.
     __device__ __forceinline__ void load(const SetDesc& sd, const float2* rec, int p0, int p1,
                                          int b0, int tid, int nt) {
+        // (32-bit byte offsets from uniform bases: n_bl < 2^18, records of 32 bytes)
+        auto at = [](const auto* base, uint32_t bytes) {
+            return *(decltype(base))((const char*)base + bytes);
+        };
         const int n_bl = sd.g.n_bl;
 #pragma unroll
         for (int k = 0; k < U; k++) {
             const int b = b0 + tid + k * nt;
-            const int bl = min(b, n_bl - 1);
-            const int f = sd.flags[bl];
+            const uint32_t bl = (uint32_t)min(b, n_bl - 1);
+            const int f = at(sd.flags, 4 * bl);
             fl[k] = b < n_bl ? f : 1;
-            uu[k] = sd.u_m[bl];
-            vv[k] = sd.v_m[bl];
-            x0[k] = rec[4 * (size_t)bl + p0];
-            x1[k] = rec[4 * (size_t)bl + p1];
-            cf[k] = sd.g.phase_coef[bl];
+            uu[k] = at(sd.u_m, 4 * bl);
+            vv[k] = at(sd.v_m, 4 * bl);
+            x0[k] = at(rec + p0, 32 * bl);
+            x1[k] = at(rec + p1, 32 * bl);
+            cf[k] = at(sd.g.phase_coef, 8 * bl);
         }
     }
 };
@@ -228,28 +234,24 @@ __device__ __forceinline__ int direct_walk(const SetDesc& sd, int64_t img, int c
             // same for every image of a channel)
             if (top) *top = max(*top, max(in1 ? r - r0 : -1, in2 ? r2 - r0 : -1));
             float2 v = select_pol2(cur.x0[k], cur.x1[k], g.pol);
-            if (g.corrections) v = cmul(v, unit_phasor(((cur.cf[k] * nu) / kVelLight)));
+            if (g.corrections) v = cmul(v, unit_phasor(cur.cf[k] * (nu / kVelLight)));
             if (!vis_ok(v)) continue;
-            if (in1) {
-                float2* d = at(r - r0, c);
+            // one of the two cells, the visibility's or its conjugate's, is
+            // here (both in the self-conjugate rows): one accumulation per
+            // lane, whichever it is, and a second where both are
+            auto put = [&](int row, int pos, float im) {
+                float2* d = at(row - r0, pos);
                 if constexpr (kWin)
                     if (!d) {
                         *outside = true;
-                        continue;
+                        return;
                     }
-                lds_add(d, v.x, v.y);
-                n_ok += (r == 0 || 2 * r == n) ? 1 : 2;
-            }
-            if (in2) {
-                float2* d = at(r2 - r0, c == 0 ? 0 : n - c);
-                if constexpr (kWin)
-                    if (!d) {
-                        *outside = true;
-                        continue;
-                    }
-                lds_add(d, v.x, -v.y);
-                n_ok += (r2 == 0 || 2 * r2 == n) ? 1 : 2;
-            }
+                lds_add(d, v.x, im);
+                n_ok += (row == 0 || 2 * row == n) ? 1 : 2;
+            };
+            const int c2 = c == 0 ? 0 : n - c;
+            put(in1 ? r : r2, in1 ? c : c2, in1 ? v.y : -v.y);
+            if (in1 && in2) put(r2, c2, -v.y);
         }
         cur = nxt;
     }

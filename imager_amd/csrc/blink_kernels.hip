@@ -265,20 +265,27 @@ k_grid_atomic(StageGrid g, int64_t n_img) {
     }
 }
 
+// Cells per thread of the cell kernels.
+constexpr int kCellsPer = 4;
+static unsigned cell_blocks(int stride) { return (unsigned)((stride + 256 * kCellsPer - 1) / (256 * kCellsPer)); }
+
 // Cells of every (channel, baseline), packed row << 16 | column (kNoCell where
 // not gridded), channels `stride` apart (a multiple of 4; the tail is kNoCell).
 __global__ void __launch_bounds__(256)
 k_stage_cells(StageGrid g, int stride, uint32_t* __restrict__ cells) {
-    const int bl = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (bl >= stride) return;
     for (int ch = blockIdx.y; ch < g.n_ch; ch += gridDim.y) {
-        uint32_t packed = kNoCell;
-        int up, vp;
-        if (bl < g.n_bl && !g.flags[bl] &&
-            plan_cell(g.u_m[bl], g.v_m[bl], CellUnit(g.freq_hz[ch], g), g, up, vp))
-            packed = ((uint32_t)wrap_index(vp, g.n_pixels) << 16) |
-                     (uint32_t)wrap_index(up, g.n_pixels);
-        cells[(int64_t)ch * stride + bl] = packed;
+        const CellUnit cu(g.freq_hz[ch], g);  // (its divisions cost several cells)
+#pragma unroll
+        for (int k = 0; k < kCellsPer; k++) {
+            const int bl = (int)(blockIdx.x * kCellsPer + k) * 256 + (int)threadIdx.x;
+            if (bl >= stride) break;
+            uint32_t packed = kNoCell;
+            int up, vp;
+            if (bl < g.n_bl && !g.flags[bl] && plan_cell(g.u_m[bl], g.v_m[bl], cu, g, up, vp))
+                packed = ((uint32_t)wrap_index(vp, g.n_pixels) << 16) |
+                         (uint32_t)wrap_index(up, g.n_pixels);
+            cells[(int64_t)ch * stride + bl] = packed;
+        }
     }
 }
 
@@ -444,7 +451,7 @@ hipError_t launch_stage_grid(const float* vis, int n_ant, int n_ch, int n_t, con
     if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
     const int stride = (int)stage_cell_stride(n_bl);
     if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k_stage_cells, dim3((unsigned)((stride + 255) / 256), (unsigned)std::min(n_ch, 65535)),
+    hipLaunchKernelGGL(k_stage_cells, dim3(cell_blocks(stride), (unsigned)std::min(n_ch, 65535)),
                        dim3(256), 0, stream, g, stride, cells);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -736,7 +743,7 @@ hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const 
     const int64_t blocks = n_img * ((n_pixels + rows - 1) / rows);
     if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
     const int stride = (int)stage_cell_stride(n_bl);
-    hipLaunchKernelGGL(k_stage_cells, dim3((unsigned)((stride + 255) / 256), (unsigned)std::min(n_ch, 65535)),
+    hipLaunchKernelGGL(k_stage_cells, dim3(cell_blocks(stride), (unsigned)std::min(n_ch, 65535)),
                        dim3(256), 0, stream, g, stride, cells);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1119,7 +1126,7 @@ k_grid_half_direct(SetDesc sd, int64_t img0, float2* __restrict__ half) {
     for (int i = threadIdx.x; i < q; i += kDirectThreads) ghd_lds4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     __syncthreads();
     const int n_ok = direct_walk<2>(sd, img, ch, n, 0, h + 1, (int)threadIdx.x, kDirectThreads,
-                                    [&](int r, int c) { return &tile[r * n + c]; });
+                                    [&](int r, int c) { return &tile[__mul24(r, n) + c]; });
     const int tot = block_sum_int(n_ok, red);
     if (threadIdx.x == 0 && tot) atomicAdd(&sd.isums[img], (uint32_t)tot);
     __syncthreads();
@@ -1551,7 +1558,7 @@ k_grid_rows_direct_fft(SetDesc first, const SetDesc* __restrict__ sets,
     int top = -1;
     const int n_ok = direct_walk<2>(
         sd, img, ch, n, 0, h + 1, (int)threadIdx.x, kDirectThreads,
-        [&](int r, int c) { return &tile[r * n + c]; }, nullptr, &top);
+        [&](int r, int c) { return &tile[__mul24(r, n) + c]; }, nullptr, &top);
     const int n_rows = block_max_int(top, red) + 1;
     const int tot = block_sum_int(n_ok, red);
     if (threadIdx.x == 0 && tot) atomicAdd(&sd.isums[img], (uint32_t)tot);
@@ -1597,15 +1604,18 @@ __global__ void __launch_bounds__(256)
 k_kb_cells(const SetDesc* __restrict__ sets) {
     const SetDesc sd = sets[blockIdx.z];
     const int n_bl = sd.g.n_bl, n = sd.n_pixels, stride = kb_cell_stride(n_bl);
-    const int bl = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (bl >= stride) return;
     for (int ch = blockIdx.y; ch < sd.g.n_ch; ch += gridDim.y) {
-        uint32_t packed = kNoCell;
-        int up, vp;
-        if (bl < n_bl && !sd.flags[bl] &&
-            plan_cell(sd.u_m[bl], sd.v_m[bl], CellUnit(sd.g.freq_hz[ch], sd), sd, up, vp))
-            packed = ((uint32_t)wrap_index(up, n) << 16) | (uint32_t)wrap_index(vp, n);
-        sd.entries[(int64_t)ch * stride + bl] = packed;
+        const CellUnit cu(sd.g.freq_hz[ch], sd);
+#pragma unroll
+        for (int k = 0; k < kCellsPer; k++) {
+            const int bl = (int)(blockIdx.x * kCellsPer + k) * 256 + (int)threadIdx.x;
+            if (bl >= stride) break;
+            uint32_t packed = kNoCell;
+            int up, vp;
+            if (bl < n_bl && !sd.flags[bl] && plan_cell(sd.u_m[bl], sd.v_m[bl], cu, sd, up, vp))
+                packed = ((uint32_t)wrap_index(up, n) << 16) | (uint32_t)wrap_index(vp, n);
+            sd.entries[(int64_t)ch * stride + bl] = packed;
+        }
     }
 }
 
@@ -1614,8 +1624,7 @@ hipError_t launch_kb_cells(const SetDesc* sets, int n_sets, int max_bl, int max_
     if (n_sets == 0 || max_bl == 0 || max_ch == 0) return hipSuccess;
     if (n_sets > 65535) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(k_kb_cells,
-                       dim3((unsigned)((kb_cell_stride(max_bl) + 255) / 256),
-                            (unsigned)std::min(max_ch, 65535), (unsigned)n_sets),
+                       dim3(cell_blocks(kb_cell_stride(max_bl)), (unsigned)std::min(max_ch, 65535), (unsigned)n_sets),
                        dim3(256), 0, stream, sets);
     return hipGetLastError();
 }
@@ -1665,7 +1674,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
             float2 v = select_pol2(rec[4 * (size_t)bl + p0],
                                    g.pol >= 2 ? rec[4 * (size_t)bl + p1] : make_float2(0.f, 0.f),
                                    g.pol);
-            if (g.corrections) v = cmul(v, unit_phasor(((g.phase_coef[bl] * nu) / kVelLight)));
+            if (g.corrections) v = cmul(v, unit_phasor(g.phase_coef[bl] * (nu / kVelLight)));
             return v;
         },
         // a nearest cell stands for its mirror too, except in the

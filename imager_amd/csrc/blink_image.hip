@@ -31,6 +31,8 @@ namespace blink {
 
 namespace {
 
+constexpr int kMaxStageRows = 64;  // rows per workgroup of the generic row pass
+
 // Stockham exchange of RegFft through one FP32 plane: slot(i) is the LDS
 // address of element i.
 template <class F, int P, bool kBlock, class Slot>
@@ -222,71 +224,83 @@ k_stage_cols(StageFftArgs a, int n_part, const float2* __restrict__ tw) {
     });
 }
 
-// Any other side: LDS Stockham passes (fft_row).  Rows: one row per team.
-template <int S, bool kBlockTeam, bool kImage>
+// Any other side: LDS Stockham passes over a tile of rows (fft_tile).  `rows` rows
+// per workgroup, all of one image.
+template <int S, bool kImage>
 __global__ void __launch_bounds__(1024)
-k_stage_rows_any(StageFftArgs a, FftPlan plan, int team, const float2* __restrict__ tw) {
+k_stage_rows_any(StageFftArgs a, FftPlan plan, int rows, const float2* __restrict__ tw) {
     extern __shared__ float4 stage_any_lds4[];
-    const int n = plan.n;
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* buf = (float2*)stage_any_lds4 + (size_t)t_id * 2 * n;
     __shared__ double red[16];
-    const int wg_per_img = (n + teams - 1) / teams;
+    __shared__ int used[kMaxStageRows];
+    const int n = plan.n, nt = (int)blockDim.x, tid = threadIdx.x;
+    float2* tile = (float2*)stage_any_lds4;       // [rows][n]
+    float2* twl = tile + (size_t)rows * n;        // twiddle table copy [n]
+    load_twiddles(twl, tw, n);
+    const int wg_per_img = (n + rows - 1) / rows;
     const int64_t img = blockIdx.x / wg_per_img;
-    const int r = (int)(blockIdx.x % wg_per_img) * teams + t_id;
-    const bool active = r < n;
-    const int64_t row = img * n + r;
-    bool any = false;
+    const int r0 = (int)(blockIdx.x % wg_per_img) * rows, nr = min(rows, n - r0);
+    const int64_t at = (img * n + r0) * n;
+    if (kImage && tid < rows) used[tid] = 0;
+    __syncthreads();
     double sum = 0.0;
-    if (active) {
-        const float2* src = a.in + row * n;
-        float2* grow = a.grids + row * n;
-        float* crow = a.counts + row * n;
-        for (int i = lane; i < n; i += team) {
-            const float2 v = src[i];
-            buf[i] = v;
+    for (int i0 = tid; i0 < nr * n; i0 += 4 * nt) {  // four loads in flight
+        float2 v[4];
+        float c[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = i0 + k * nt;
+            v[k] = make_float2(0.f, 0.f);
+            c[k] = 0.f;
+            if (i >= nr * n) continue;
+            v[k] = a.in[at + i];
+            if constexpr (kImage) c[k] = a.counts[at + i];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = i0 + k * nt;
+            if (i >= nr * n) break;
+            tile[i] = v[k];
             if constexpr (kImage) {
-                const float c = crow[i];
-                sum += (double)c;
-                any |= any_bits(v);
-                if (a.clear && any_bits(v)) grow[i] = make_float2(0.f, 0.f);
-                if (a.clear && __float_as_uint(c) != 0u) crow[i] = 0.f;
+                sum += (double)c[k];
+                if (any_bits(v[k])) {
+                    used[i / n] = 1;
+                    if (a.clear) a.grids[at + i] = make_float2(0.f, 0.f);
+                }
+                if (a.clear && __float_as_uint(c[k]) != 0u) a.counts[at + i] = 0.f;
             }
         }
     }
-    bool used = active;
     if constexpr (kImage) {
         const double t = block_sum_double(sum, red);
-        if (threadIdx.x == 0) a.part[blockIdx.x] = t;
-        if constexpr (kBlockTeam) {
-            used = __syncthreads_or(any ? 1 : 0);
-        } else {
-            const uint64_t m = __ballot(any) >> (threadIdx.x & 63 & ~(team - 1));
-            used = active && (m & (team == 64 ? ~0ull : (1ull << team) - 1)) != 0;
-        }
-        if (active && lane == 0) a.used[row] = used ? 1 : 0;
+        if (tid == 0) a.part[blockIdx.x] = t;
     }
-    team_sync<kBlockTeam>();
-    if (!used) return;  // uniform per team
-    const float2* res = fft_row<S, kBlockTeam>(buf, buf + n, plan, tw, lane, team);
-    float2* dst = a.out + row * n;
-    for (int i = lane; i < n; i += team) dst[kImage ? shift_index(i, n) : i] = res[i];
+    __syncthreads();
+    if constexpr (kImage) {
+        if (tid < nr) a.used[img * n + r0 + tid] = used[tid] ? 1 : 0;
+        int any = 0;
+        for (int r = 0; r < nr; r++) any |= used[r];
+        if (!any) return;  // uniform
+    }
+    fft_tile<S>(tile, nr, n, plan, twl);
+    for (int i = tid; i < nr * n; i += nt) {
+        const int r = i / n;
+        if constexpr (kImage) {
+            if (used[r]) a.out[at + r * n + shift_index(i - r * n, n)] = tile[i];
+        } else {
+            a.out[at + i] = tile[i];
+        }
+    }
 }
 
 // Columns in place, w = 2^lw of them per workgroup (fewer in the last one).
-template <int S, bool kBlockTeam, bool kImage>
+template <int S, bool kImage>
 __global__ void __launch_bounds__(1024)
-k_stage_cols_any(StageFftArgs a, FftPlan plan, int team, int lw, int n_part,
-                 const float2* __restrict__ tw) {
+k_stage_cols_any(StageFftArgs a, FftPlan plan, int lw, int n_part, const float2* __restrict__ tw) {
     extern __shared__ float4 stage_any_cols_lds4[];
     const int n = plan.n, ld = n + 1, w = 1 << lw;  // padded LDS rows
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* tile = (float2*)stage_any_cols_lds4;  // [w][ld]
-    float2* tmp = tile + (size_t)w * ld + (size_t)t_id * n;
+    float2* tile = (float2*)stage_any_cols_lds4;    // [w][ld]
+    float2* twl = tile + (size_t)w * ld;            // twiddle table copy [n]
+    load_twiddles(twl, tw, n);
     const int n_cb = (n + w - 1) >> lw;
     const unsigned bid = xcd_order(blockIdx.x, gridDim.x);
     const int64_t img = bid / n_cb;
@@ -294,8 +308,7 @@ k_stage_cols_any(StageFftArgs a, FftPlan plan, int team, int lw, int n_part,
     const int w_here = min(w, n - c0);
     float2* base = a.out + img * n * n + c0;
     const unsigned char* used = a.used + img * n;
-    const int total = n << lw;
-    const int nt = (int)blockDim.x;
+    const int total = n << lw, nt = (int)blockDim.x;
     for (int i0 = threadIdx.x; i0 < total; i0 += 4 * nt) {
         float2 p[4];
 #pragma unroll
@@ -313,18 +326,7 @@ k_stage_cols_any(StageFftArgs a, FftPlan plan, int team, int lw, int n_part,
     float scale = 1.f;
     if constexpr (kImage) scale = scale_of(a.part + img * n_part, n_part);
     __syncthreads();
-    const int rounds = kBlockTeam ? w_here : (w_here + teams - 1) / teams;
-    for (int k = 0; k < rounds; k++) {
-        const int c = kBlockTeam ? k : k * teams + t_id;
-        if (!kBlockTeam && c >= w_here) break;
-        float2* col = tile + (size_t)c * ld;
-        const float2* res = fft_row<S, kBlockTeam>(col, tmp, plan, tw, lane, team);
-        if (res != col) {
-            for (int i = lane; i < n; i += team) col[i] = res[i];
-            team_sync<kBlockTeam>();
-        }
-    }
-    __syncthreads();
+    fft_tile<S>(tile, w_here, ld, plan, twl);
     for (int i = threadIdx.x; i < total; i += nt) {
         const int r = i >> lw, c = i & (w - 1);
         if (c >= w_here) continue;
@@ -336,15 +338,19 @@ k_stage_cols_any(StageFftArgs a, FftPlan plan, int team, int lw, int n_part,
 
 // ------------------------------------------------------------ launchers
 
-// Lanes per row of the generic kernels: up to 64 inside a wavefront, above
-// 1024 the whole workgroup.
-static int any_team(int n) {
-    if (n <= 64) return 16;
-    if (n <= 256) return 32;
-    if (n <= 1024) return 64;
-    return n <= 4096 ? 256 : 512;
+// Rows per workgroup of the generic row pass: what 512 threads hold at about
+// 12 values each, fewer while the launch has under 512 workgroups.
+static int any_rows(int n, int64_t n_img) {
+    int rows = std::max(1, std::min(kMaxStageRows, 6144 / n));
+    while (rows > 1 && n_img * ((n + rows - 1) / rows) < 512) rows = (rows + 1) / 2;
+    return rows;
 }
-static int any_teams(int n) { return n <= 1024 ? 256 / any_team(n) : 1; }
+
+static int any_threads(const FftPlan& plan, int64_t values) {
+    int nt = 256;
+    while (nt < 1024 && ((int64_t)nt * plan.cap < values || nt * plan.cap < plan.n)) nt *= 2;
+    return nt;
+}
 
 // Row groups per workgroup: up to 4 while 1024 workgroups remain (4 per CU).
 template <int N>
@@ -362,7 +368,7 @@ int stage_fft_parts(int n, int64_t n_img) {
     case NN: return NN / (RowShape<NN>::NT / RowShape<NN>::L * row_iters<NN>(n_img));
         X(128) X(256) X(512) X(1024) X(2048) X(4096)
 #undef X
-        default: return (n + any_teams(n) - 1) / any_teams(n);
+        default: return (n + any_rows(n, n_img) - 1) / any_rows(n, n_img);
     }
 }
 
@@ -393,42 +399,33 @@ static hipError_t cols_n(const StageFftArgs& a, int64_t n_img, int n_part, const
 template <int S, bool kImage>
 static hipError_t rows_any(const StageFftArgs& a, const FftPlan& plan, int64_t n_img,
                            const float2* tw, hipStream_t s) {
-    const int n = plan.n, team = any_team(n), teams = any_teams(n);
-    const size_t lds = sizeof(float2) * 2 * (size_t)n * teams;
-    const int64_t blocks = n_img * ((n + teams - 1) / teams);
+    const int n = plan.n, rows = any_rows(n, n_img);
+    const size_t lds = sizeof(float2) * ((size_t)n * rows + n);
+    const int64_t blocks = n_img * ((n + rows - 1) / rows);
     if (blocks > 0x7fffffff || (int64_t)lds > g_lds_limit) return hipErrorInvalidConfiguration;
-    const dim3 grid((unsigned)blocks), block(team * teams);
-    if (n > 1024)
-        hipLaunchKernelGGL((k_stage_rows_any<S, true, kImage>), grid, block, lds, s, a, plan, team, tw);
-    else
-        hipLaunchKernelGGL((k_stage_rows_any<S, false, kImage>), grid, block, lds, s, a, plan, team, tw);
+    hipLaunchKernelGGL((k_stage_rows_any<S, kImage>), dim3((unsigned)blocks),
+                       dim3(any_threads(plan, (int64_t)n * rows)), lds, s, a, plan, rows, tw);
     return hipGetLastError();
 }
 
 template <int S, bool kImage>
 static hipError_t cols_any(const StageFftArgs& a, const FftPlan& plan, int64_t n_img, int n_part,
                            const float2* tw, hipStream_t s) {
-    const int n = plan.n, team = any_team(n), teams = any_teams(n);
-    auto lds_for = [&](int lw) {
-        return sizeof(float2) * (((size_t)(n + 1) << lw) + (size_t)teams * n);
-    };
-    // 16 columns (128-byte runs) while two workgroups fit in LDS and 512
-    // workgroups remain (two per CU); narrower blocks for few images
+    const int n = plan.n;
+    auto lds_for = [&](int lw) { return sizeof(float2) * (((size_t)(n + 1) << lw) + n); };
+    // 16 columns (128-byte runs), fewer while the threads do not hold them, two
+    // workgroups (from 4 columns on, one) do not fit in LDS, or the launch has
+    // under 512 workgroups (two per CU)
     int lw = 4;
-    while (lw > 1 && (2 * (int64_t)lds_for(lw) > g_lds_limit ||
-                      n_img * ((n + (1 << lw) - 1) >> lw) < 512))
+    while (lw > 0 && (((int64_t)n << lw) > 1024 * plan.cap || (int64_t)lds_for(lw) > g_lds_limit ||
+                      (lw > 2 && 2 * (int64_t)lds_for(lw) > g_lds_limit) ||
+                      (lw > 1 && n_img * ((n + (1 << lw) - 1) >> lw) < 512)))
         lw--;
-    while (lw > 0 && (int64_t)lds_for(lw) > g_lds_limit) lw--;
     const size_t lds = lds_for(lw);
     const int64_t blocks = n_img * ((n + (1 << lw) - 1) >> lw);
     if (blocks > 0x7fffffff || (int64_t)lds > g_lds_limit) return hipErrorInvalidConfiguration;
-    const dim3 grid((unsigned)blocks), block(team * teams);
-    if (n > 1024)
-        hipLaunchKernelGGL((k_stage_cols_any<S, true, kImage>), grid, block, lds, s, a, plan, team,
-                           lw, n_part, tw);
-    else
-        hipLaunchKernelGGL((k_stage_cols_any<S, false, kImage>), grid, block, lds, s, a, plan, team,
-                           lw, n_part, tw);
+    hipLaunchKernelGGL((k_stage_cols_any<S, kImage>), dim3((unsigned)blocks),
+                       dim3(any_threads(plan, (int64_t)n << lw)), lds, s, a, plan, lw, n_part, tw);
     return hipGetLastError();
 }
 
@@ -474,11 +471,10 @@ hipError_t set_stage_kernel_attributes() {
     X(128) X(256) X(512) X(1024) X(2048) X(4096)
 #undef X
 #undef Y
-#define X(S, B, I)                                   \
-    set((const void*)k_stage_rows_any<S, B, I>);     \
-    set((const void*)k_stage_cols_any<S, B, I>);
-    X(1, true, true) X(1, false, true) X(1, true, false) X(1, false, false)
-    X(-1, true, false) X(-1, false, false)
+#define X(S, I)                                   \
+    set((const void*)k_stage_rows_any<S, I>);     \
+    set((const void*)k_stage_cols_any<S, I>);
+    X(1, true) X(1, false) X(-1, false)
 #undef X
     return e;
 }

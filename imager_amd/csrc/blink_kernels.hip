@@ -28,19 +28,8 @@ int device_cu_count() {
 // not launched.
 static bool lds_fits(size_t bytes) { return (int64_t)bytes <= g_lds_limit; }
 
-// Workgroup of the generic direct row passes (one per image) and its teams.
-constexpr int kDirectThreads = 1024, kDirectTeam = 64;
-
-// Sides up to kTwLdsMax copy the twiddle table into LDS in the generic
-// second-pass kernels, so that the Stockham passes do not wait on global
-// loads between team syncs (768 x 180^2: 121 -> 115 us per launch; the
-// plan-path row kernel, whose workgroups are short, measured 444 -> 469 us
-// with it and keeps the global table).
-constexpr int kTwLdsMax = 1024;
-__host__ __device__ constexpr size_t tw_lds_bytes(int n) {
-    return n <= kTwLdsMax ? sizeof(float2) * (size_t)n : 0;
-}
-
+// Workgroup of the generic direct row passes (one per image).
+constexpr int kDirectThreads = 1024;
 
 // ------------------------------------------------------------------ helpers
 
@@ -1260,20 +1249,17 @@ hipError_t launch_average(const float* images, int64_t image_size, int n_images,
 // row-pass buffer `inter` (image index relative to the chunk).  Empty rows are
 // not written: the column pass reads the plan and treats them as zero.  The
 // number of gridded cells per image goes to isums (integer atomics).
-template <int S, bool kBlockTeam, bool kMulti>
-__global__ void __launch_bounds__(kFftThreads)
+template <bool kMulti>
+__global__ void __launch_bounds__(1024)
 k_grid_rows_fft(SetDesc first, const SetDesc* __restrict__ sets, const int* __restrict__ img_set,
-                FftPlan plan, int team, int rb, int64_t gi0, float2* __restrict__ inter,
+                FftPlan plan, int rb, int64_t gi0, float2* __restrict__ inter,
                 const float2* __restrict__ tw) {
     extern __shared__ float4 grf_lds4[];
     const int n = plan.n;
     float2* tile = (float2*)grf_lds4;                 // [rb][n]
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* tmp = tile + (size_t)rb * n + (size_t)t_id * n;
+    float2* twl = tile + (size_t)rb * n;              // twiddle table copy [n]
     __shared__ int rs[kMaxTileRows + 1];
-    __shared__ int red[kFftThreads / 64];
+    __shared__ int red[1024 / 64];
 
     // Rows 0 .. N/2 only: the gridded plane is Hermitian, so row N - v is the
     // conjugate mirror of row v and the column pass rebuilds it.
@@ -1299,9 +1285,10 @@ k_grid_rows_fft(SetDesc first, const SetDesc* __restrict__ sets, const int* __re
     if ((int)threadIdx.x <= nr) rs[threadIdx.x] = rsg[r0 + threadIdx.x];
     __syncthreads();
     if (rs[nr] == rs[0]) return;  // uniform: no entries in this tile
-    // "U" weighting: a count per tile cell after the team scratch
-    unsigned* cnt = (unsigned*)(tile + (size_t)rb * n + (size_t)teams * n);
+    // "U" weighting: a count per tile cell after the table
+    unsigned* cnt = (unsigned*)(twl + n);
     const bool uniform = sd.uniform != 0;
+    load_twiddles(twl, tw, n);
     for (int i = threadIdx.x; i < nr * n; i += blockDim.x) tile[i] = make_float2(0.f, 0.f);
     if (uniform)
         for (int i = threadIdx.x; i < nr * n; i += blockDim.x) cnt[i] = 0u;
@@ -1326,16 +1313,11 @@ k_grid_rows_fft(SetDesc first, const SetDesc* __restrict__ sets, const int* __re
         }
         __syncthreads();
     }
-    const int rounds = kBlockTeam ? nr : (nr + teams - 1) / teams;
-    for (int k = 0; k < rounds; k++) {
-        const int r = kBlockTeam ? k : k * teams + t_id;
-        if (!kBlockTeam && r >= nr) break;
-        if (rs[r + 1] == rs[r]) continue;  // uniform per team
-        float2* row = tile + (size_t)r * n;
-        const float2* res = fft_row<S, kBlockTeam>(row, tmp, plan, tw, lane, team);
-        float2* dst = inter + ((int64_t)li * (h + 1) + r0 + r) * n;
-        for (int i = lane; i < n; i += team) store_stream(&dst[i], res[i]);
-        team_sync<kBlockTeam>();
+    fft_tile<1>(tile, nr, n, plan, twl);
+    float2* dst = inter + ((int64_t)li * (h + 1) + r0) * n;
+    for (int i = threadIdx.x; i < nr * n; i += blockDim.x) {
+        const int r = i / n;
+        if (rs[r + 1] != rs[r]) store_stream(&dst[i], tile[i]);  // (rows without entries: not read)
     }
 }
 
@@ -1347,28 +1329,24 @@ k_grid_rows_fft(SetDesc first, const SetDesc* __restrict__ sets, const int* __re
 // are the conjugates of rows p.  A workgroup owns `cb` (even) buffer columns
 // = cb/2 pairs, staged through LDS with 16-byte loads, transformed by the
 // teams, scaled by 1/sum and stored fftshifted with imaginary parts 0.
-template <int S, bool kBlockTeam, bool kMulti>
-__global__ void __launch_bounds__(kFftThreads)
+template <bool kMulti>
+__global__ void __launch_bounds__(1024)
 k_cols_half(SetDesc first, const SetDesc* __restrict__ sets, const int* __restrict__ img_set,
-            FftPlan plan, int team, int cb, int64_t gi0, const float2* __restrict__ inter,
+            FftPlan plan, int pairs, int64_t gi0, const float2* __restrict__ inter,
             const float2* __restrict__ tw) {
     extern __shared__ float4 ch_lds4[];
-    const int n = plan.n, h = n / 2, pairs = cb / 2;
+    const int n = plan.n, h = n / 2;
     const int ld = n + 1;                                   // padded LDS row
     float2* rows = (float2*)ch_lds4;                        // [pairs][ld]
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* tmp = rows + (size_t)pairs * ld + (size_t)t_id * n;
-    float2* twl = rows + (size_t)pairs * ld + (size_t)teams * n;  // [n] when n <= kTwLdsMax
-    unsigned char* nonempty = (unsigned char*)twl + tw_lds_bytes(n);
-    const float2* twp = n <= kTwLdsMax ? twl : tw;
-    if (n <= kTwLdsMax)
-        for (int i = threadIdx.x; i < n; i += blockDim.x) twl[i] = tw[i];
+    float2* twl = rows + (size_t)pairs * ld;                // twiddle table copy [n]
+    unsigned char* nonempty = (unsigned char*)(twl + n);
+    load_twiddles(twl, tw, n);
 
-    const int n_cb = n / cb;
-    const int cbk = (int)(blockIdx.x % n_cb);
-    const int li = (int)(blockIdx.x / n_cb);
+    // neighbouring blocks share lines of the buffer's rows: one XCD each
+    const unsigned bid = xcd_order(blockIdx.x, gridDim.x);
+    const int n_cb = (h + pairs - 1) / pairs;
+    const int cbk = (int)(bid % n_cb);
+    const int li = (int)(bid / n_cb);
     const int64_t gi = gi0 + li;
     const SetDesc sd = set_of<kMulti>(first, sets, img_set, gi);
     if (!sd.images) return;  // a set imaged for its average only (uniform per workgroup)
@@ -1381,7 +1359,8 @@ k_cols_half(SetDesc first, const SetDesc* __restrict__ sets, const int* __restri
         nonempty[i] = sd.all_rows || rsg[i + 1] != rsg[i];
     __syncthreads();
 
-    const int c0 = cbk * cb;
+    const int c0 = cbk * 2 * pairs;
+    pairs = min(pairs, h - cbk * pairs);  // (the last block's)
     const float2* src = inter + (int64_t)li * (h + 1) * n + c0;
     // four loads in flight per thread, then their LDS writes
     const int stage = (h + 1) * pairs, nt = (int)blockDim.x;
@@ -1405,18 +1384,7 @@ k_cols_half(SetDesc first, const SetDesc* __restrict__ sets, const int* __restri
         }
     }
     __syncthreads();
-    const int rounds = kBlockTeam ? pairs : (pairs + teams - 1) / teams;
-    for (int k = 0; k < rounds; k++) {
-        const int t = kBlockTeam ? k : k * teams + t_id;
-        if (!kBlockTeam && t >= pairs) break;
-        float2* zr = rows + (size_t)t * ld;
-        const float2* res = fft_row<S, kBlockTeam>(zr, tmp, plan, twp, lane, team);
-        if (res != zr) {
-            for (int i = lane; i < n; i += team) zr[i] = res[i];
-            team_sync<kBlockTeam>();
-        }
-    }
-    __syncthreads();
+    fft_tile<1>(rows, pairs, ld, plan, twl);
     const float s = (float)(1.0 / (double)count);
     float2* out = sd.images + (int64_t)img * n * n;
     // the plan is transposed: pair t holds Z_t[x] = img[y][x] + i img[y + 1][x]
@@ -1436,49 +1404,54 @@ k_cols_half(SetDesc first, const SetDesc* __restrict__ sets, const int* __restri
 
 // ------------------------------------------------------------ launchers
 
-static int fft_team_for(int n) {
-    // lanes per row: about 8-16 values per lane, one wave or the whole block
-    if (n <= 128) return 16;
-    if (n <= 512) return 32;
-    if (n <= 1024) return 64;
-    return kFftThreads;
-}
-
+// Radices for n: 15s, then 10s (or 5s), 9s, and the 2s in even shares of at most 16,
+// so that the passes are few; odd radices go first (the first pass writes
+// with a lane stride of R, free of bank conflicts when R is odd).
 bool make_fft_plan(int n, FftPlan& plan) {
     if (n < 2 || n > kMaxPixels) return false;
+    int f[14] = {}, rem = n;
+    for (int r : {2, 3, 5, 7, 11, 13})
+        while (rem % r == 0) rem /= r, f[r]++;
+    if (rem != 1) return false;
+    int odd[kMaxFftPasses], even[kMaxFftPasses], n_odd = 0, n_even = 0;
+    for (int r : {13, 11, 7})
+        while (f[r] > 0) odd[n_odd++] = r, f[r]--;
+    while (f[3] > 0 && f[5] > 0) odd[n_odd++] = 15, f[3]--, f[5]--;
+    for (; f[5] > 0; f[5]--) {
+        if (f[2] > 0) even[n_even++] = 10, f[2]--;
+        else odd[n_odd++] = 5;
+    }
+    for (; f[3] > 1; f[3] -= 2) odd[n_odd++] = 9;
+    if (f[3]) {
+        if (f[2] > 1) even[n_even++] = 12, f[2] -= 2;
+        else if (f[2]) even[n_even++] = 6, f[2]--;
+        else odd[n_odd++] = 3;
+    }
+    for (int passes = (f[2] + 3) / 4; passes > 0; passes--) {
+        const int e = (f[2] + passes - 1) / passes;
+        even[n_even++] = 1 << e;
+        f[2] -= e;
+    }
     plan.n = n;
     plan.n_passes = 0;
-    int rem = n, span = 1;
-    while (rem > 1) {
-        int r;
-        if (rem % 16 == 0) r = 16;
-        else if (rem % 8 == 0) r = 8;
-        else if (rem % 4 == 0) r = 4;
-        else if (rem % 2 == 0) r = 2;
-        else if (rem % 3 == 0) r = 3;
-        else if (rem % 5 == 0) r = 5;
-        else if (rem % 7 == 0) r = 7;
-        else if (rem % 11 == 0) r = 11;
-        else if (rem % 13 == 0) r = 13;
-        else return false;
-        if (plan.n_passes >= kMaxFftPasses) return false;
+    plan.cap = kPassValues;
+    int span = 1;
+    for (int i = 0; i < n_odd + n_even; i++) {
+        const int r = i < n_odd ? odd[i] : even[i - n_odd];
         plan.radix[plan.n_passes] = r;
-        plan.span[plan.n_passes] = span;
-        plan.n_passes++;
+        plan.span[plan.n_passes++] = span;
+        plan.cap = std::min(plan.cap, kPassValues / r * r);
         span *= r;
-        rem /= r;
     }
     return true;
 }
 
-int grid_rows_tile_rows(int n) {
-    const int team = fft_team_for(n);
-    const int teams = team == kFftThreads ? 1 : kFftThreads / team;
-    const int64_t budget = g_lds_budget - (int64_t)teams * n * 8;
-    int rb = (int)(budget / ((int64_t)n * 8));
-    rb = std::min(rb, kMaxTileRows);
-    if (rb >= teams) rb = (rb / teams) * teams;
-    return std::max(1, std::min(rb, n));
+// Threads of a workgroup (256, 512 or 1024) that transforms `values` values of
+// rows of length n at once (at least one row).
+static int fft_threads(const FftPlan& plan, int64_t values) {
+    int nt = 256;
+    while (nt < 1024 && ((int64_t)nt * plan.cap < values || nt * plan.cap < plan.n)) nt *= 2;
+    return nt;
 }
 
 hipError_t launch_grid_rows_fft(const SetDesc& first, const SetDesc* sets, const int* img_set,
@@ -1486,32 +1459,25 @@ hipError_t launch_grid_rows_fft(const SetDesc& first, const SetDesc* sets, const
                                 float* inter, const float* tw, hipStream_t stream) {
     if (n_img == 0) return hipSuccess;
     const int n = plan.n;
-    const int team = fft_team_for(n);
-    const bool block_team = team == kFftThreads;
-    const int teams = block_team ? 1 : kFftThreads / team;
     // rows per tile: as many as fit up to 4, and at least ~2048 workgroups in
     // the launch, so that a few images still spread over the whole chip.  The
     // gather of plan entries is latency bound: small tiles keep more
     // workgroups in flight (4 rows measured fastest against 2 to 16 at 180^2).
     const int64_t want = (int64_t)(n / 2 + 1) * n_img / 2048;
-    int rb = (int)std::max<int64_t>(
-        1, std::min<int64_t>({(int64_t)grid_rows_tile_rows(n), want, 4}));
+    int rb = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)n, want, 4}));
     // uniform weighting keeps a count per tile cell beside the tile
     const bool uniform = first.uniform != 0;
     auto lds_of = [&](int r) {
-        return sizeof(float2) * ((size_t)r * n + (size_t)teams * n) +
-               (uniform ? sizeof(unsigned) * (size_t)r * n : 0);
+        return sizeof(float2) * ((size_t)r * n + n) + (uniform ? sizeof(unsigned) * (size_t)r * n : 0);
     };
     while (rb > 1 && !lds_fits(lds_of(rb))) rb--;
+    const int nt = fft_threads(plan, (int64_t)rb * n);
     const int n_rb = (n / 2 + 1 + rb - 1) / rb;
     const size_t lds = lds_of(rb);
-    if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-    const dim3 grid((unsigned)((int64_t)n_rb * n_img));
-    const bool multi = n_sets > 1;
-    auto k = block_team
-                 ? (multi ? k_grid_rows_fft<1, true, true> : k_grid_rows_fft<1, true, false>)
-                 : (multi ? k_grid_rows_fft<1, false, true> : k_grid_rows_fft<1, false, false>);
-    hipLaunchKernelGGL(k, grid, dim3(kFftThreads), lds, stream, first, sets, img_set, plan, team,
+    const int64_t blocks = (int64_t)n_rb * n_img;
+    if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    auto k = n_sets > 1 ? k_grid_rows_fft<true> : k_grid_rows_fft<false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(nt), lds, stream, first, sets, img_set, plan,
                        rb, gi0, (float2*)inter, (const float2*)tw);
     return hipGetLastError();
 }
@@ -1520,15 +1486,14 @@ hipError_t launch_grid_rows_fft(const SetDesc& first, const SetDesc* sets, const
 // timestep per channel, as k_grid_rows_direct does it for the register
 // sides: one workgroup per image with the whole half plane (plan rows
 // 0 .. N/2 of an even or odd side) in LDS, every baseline walked in order
-// (direct_walk), then rows 0 .. the highest holding a cell transformed by
-// teams of one wave and stored row-major as the generic second pass reads
-// them, and the image's row starts written (the rows above empty).  Sides
-// whose half plane
-// and team scratch fit in LDS (up to 186).  The count sums start at zero
-// (the direct set-up launch).
+// (direct_walk), then rows 0 .. the highest holding a cell transformed
+// (fft_tile) and stored row-major as the generic second pass reads them, and
+// the image's row starts written (the rows above empty).  Sides up to
+// kDirectMaxSide, whose half plane leaves room for the table.  The count sums
+// start at zero (the direct set-up launch).
+constexpr int kDirectMaxSide = 186;
 static size_t direct_fft_lds_bytes(int n) {
-    return sizeof(float2) *
-           ((size_t)(n / 2 + 1) * n + (size_t)(kDirectThreads / kDirectTeam) * n + n);
+    return sizeof(float2) * ((size_t)(n / 2 + 1) * n + n);
 }
 
 template <bool kMulti>
@@ -1537,14 +1502,9 @@ k_grid_rows_direct_fft(SetDesc first, const SetDesc* __restrict__ sets,
                        const int* __restrict__ img_set, FftPlan plan, int64_t gi0,
                        float2* __restrict__ inter, const float2* __restrict__ tw) {
     extern __shared__ float4 grd_lds4[];
-    constexpr int teams = kDirectThreads / kDirectTeam;
     const int n = plan.n, h = n / 2;
-    float2* tile = (float2*)grd_lds4;  // [h + 1][n]
-    const int t_id = (int)threadIdx.x / kDirectTeam, lane = (int)threadIdx.x % kDirectTeam;
-    float2* tmp = tile + (size_t)(h + 1) * n + (size_t)t_id * n;
-    // twiddle table copy [n] after the teams' scratch: the passes read it
-    // from LDS instead of waiting on global loads between team syncs
-    float2* twl = tile + (size_t)(h + 1) * n + (size_t)teams * n;
+    float2* tile = (float2*)grd_lds4;          // [h + 1][n]
+    float2* twl = tile + (size_t)(h + 1) * n;  // twiddle table copy [n]
     __shared__ int red[kDirectThreads / 64];
 
     const int li = (int)xcd_order(blockIdx.x, gridDim.x);
@@ -1553,7 +1513,7 @@ k_grid_rows_direct_fft(SetDesc first, const SetDesc* __restrict__ sets,
     const int img = (int)(gi - sd.img_base);
     const int ch = img % sd.g.n_ch;
     for (int i = threadIdx.x; i < (h + 1) * n; i += kDirectThreads) tile[i] = make_float2(0.f, 0.f);
-    for (int i = threadIdx.x; i < n; i += kDirectThreads) twl[i] = tw[i];
+    load_twiddles(twl, tw, n);
     __syncthreads();
     int top = -1;
     const int n_ok = direct_walk<2>(
@@ -1565,13 +1525,9 @@ k_grid_rows_direct_fft(SetDesc first, const SetDesc* __restrict__ sets,
     __syncthreads();
     // rows 0 .. n_rows - 1 (the highest holding a cell); the row starts tell
     // the second pass that the others are empty
-    for (int r = t_id; r < n_rows; r += teams) {
-        float2* row = tile + (size_t)r * n;
-        const float2* res = fft_row<1, false>(row, tmp, plan, twl, lane, kDirectTeam);
-        float2* dst = inter + ((int64_t)li * (h + 1) + r) * n;
-        for (int i = lane; i < n; i += kDirectTeam) store_stream(&dst[i], res[i]);
-        team_sync<false>();
-    }
+    fft_tile<1>(tile, n_rows, n, plan, twl);
+    float2* dst = inter + (int64_t)li * (h + 1) * n;
+    for (int i = threadIdx.x; i < n_rows * n; i += kDirectThreads) store_stream(&dst[i], tile[i]);
     int* rsg = sd.row_start + (int64_t)ch * (n + 1);
     for (int i = threadIdx.x; i <= n; i += kDirectThreads) rsg[i] = min(i, n_rows);
 }
@@ -1582,7 +1538,7 @@ bool direct_half_plane_fits(int n) {
 
 bool direct_row_pass_fits(int n) {
     if (batch_reg_supported(n)) return batch_direct_supported(n);
-    return n >= 2 && n <= kMaxPixels && lds_fits(direct_fft_lds_bytes(n));
+    return n >= 2 && n <= kDirectMaxSide && lds_fits(direct_fft_lds_bytes(n));
 }
 
 hipError_t launch_grid_rows_direct_fft(const SetDesc& first, const SetDesc* sets,
@@ -1640,10 +1596,10 @@ hipError_t launch_kb_cells(const SetDesc* sets, int n_sets, int max_bl, int max_
 constexpr int kKbRowThreads = 1024;
 // (one row of 8192 cells and the queue of one vector per thread fit a CU)
 constexpr int kb_row_vec(bool wide) { return wide ? 1 : 2; }
-template <int kX, bool kBlockTeam, bool kMulti>
+template <int kX, bool kWide, bool kMulti>
 __global__ void __launch_bounds__(kKbRowThreads)
 k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __restrict__ img_set,
-               FftPlan plan, int team, int rb, int64_t gi0, int n_img, float2* __restrict__ inter,
+               FftPlan plan, int rb, int64_t gi0, int n_img, float2* __restrict__ inter,
                const float2* __restrict__ tw, int blocked) {
     extern __shared__ float4 grk_lds4[];
     const int n = plan.n, h = n / 2, tid = threadIdx.x;
@@ -1667,7 +1623,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     const int p1 = g.pol == 3 ? 2 : 3;
     const int stride = kb_cell_stride(g.n_bl);
     int n_ok = 0;
-    const int queued = kb_accumulate<kKbRowThreads, kb_row_vec(kBlockTeam), kX, true>(
+    const int queued = kb_accumulate<kKbRowThreads, kb_row_vec(kWide), kX, true>(
         sg, wavelength_of(nu), sd.kb_size, sd.kb_table, sd.entries + (int64_t)ch * stride, stride,
         r0, nr, re, im, queue, &n_queued,
         [&](int bl) {
@@ -1688,26 +1644,26 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
         *(float2*)&re[i] = c;
     }
     __syncthreads();
-    const int teams = kBlockTeam ? 1 : kKbRowThreads / team;
-    const int t_id = kBlockTeam ? 0 : tid / team, lane = kBlockTeam ? tid : tid % team;
+    const float2* rows = (float2*)re;
+    if (queued) {  // (uniform) else zeros
+        float2* twl = (float2*)im;  // (rb >= 1 rows of n)
+        load_twiddles(twl, tw, n);
+        __syncthreads();
+        fft_tile<1>((float2*)re, nr, n, plan, twl);
+    }
     const int64_t h1 = h + 1;
-    for (int r = t_id; r < nr; r += teams) {
-        const float2* res = (float2*)re + (size_t)r * n;
-        if (queued)  // (uniform) else zeros
-            res = fft_row<1, kBlockTeam>((float2*)re + (size_t)r * n, (float2*)im + (size_t)r * n,
-                                         plan, tw, lane, team);
-        const int v = r0 + r;
-        if (blocked) {  // element (v, x) at ((x / 32) (N/2+1) + v) 32 + x % 32
-            float2* dst = inter + (int64_t)li * h1 * n + (int64_t)v * kInterBlockCols;
-            for (int i = lane; i < n; i += team)
-                store_stream(&dst[(int64_t)(i / kInterBlockCols) * h1 * kInterBlockCols +
-                                  i % kInterBlockCols],
-                             res[i]);
-        } else {
-            float2* dst = inter + ((int64_t)li * h1 + v) * n;
-            for (int i = lane; i < n; i += team) store_stream(&dst[i], res[i]);
-        }
-        team_sync<kBlockTeam>();
+    if (!blocked) {
+        float2* dst = inter + ((int64_t)li * h1 + r0) * n;
+        for (int i = tid; i < nr * n; i += kKbRowThreads) store_stream(&dst[i], rows[i]);
+        return;
+    }
+    // element (v, x) at ((x / 32) (N/2+1) + v) 32 + x % 32 (n a power of two)
+    float2* dst = inter + (int64_t)li * h1 * n + (int64_t)r0 * kInterBlockCols;
+    for (int i = tid; i < nr * n; i += kKbRowThreads) {
+        const int r = i / n, x = i - r * n;
+        store_stream(&dst[(int64_t)(x / kInterBlockCols) * h1 * kInterBlockCols +
+                          r * kInterBlockCols + x % kInterBlockCols],
+                     rows[i]);
     }
 }
 
@@ -1717,12 +1673,11 @@ hipError_t launch_grid_rows_kb(const SetDesc& first, const SetDesc* sets, const 
     if (n_img == 0) return hipSuccess;
     if (first.kb_size < 1) return hipErrorInvalidValue;
     const int n = plan.n, h1 = n / 2 + 1;
-    const bool block_team = n > 1024;
-    const int team = block_team ? kKbRowThreads : fft_team_for(n);
+    const bool wide = n > 1024;
     // as many rows as a CU's LDS holds (the taller the slab, the fewer slabs
     // compute a footprint's weights again), fewer while the images leave under
     // four workgroups per CU (rows above the array's reach have no work)
-    const size_t queue = kb_queue_bytes(kKbRowThreads, kb_row_vec(block_team));
+    const size_t queue = kb_queue_bytes(kKbRowThreads, kb_row_vec(wide));
     int rb = (int)std::min<int64_t>(h1, (g_lds_limit - (int64_t)queue) / (16 * (int64_t)n));
     if (rb < 1) return hipErrorInvalidConfiguration;
     while (rb > 2 && (int64_t)n_img * ((h1 + rb - 1) / rb) < 4 * device_cu_count()) rb = (rb + 1) / 2;
@@ -1732,14 +1687,13 @@ hipError_t launch_grid_rows_kb(const SetDesc& first, const SetDesc* sets, const 
     // (a group's sets share kb_size)
     auto pick = [&](auto kx) {
         constexpr int X = decltype(kx)::value;
-        return block_team ? (n_sets > 1 ? k_grid_rows_kb<X, true, true> : k_grid_rows_kb<X, true, false>)
-                          : (n_sets > 1 ? k_grid_rows_kb<X, false, true>
-                                        : k_grid_rows_kb<X, false, false>);
+        return wide ? (n_sets > 1 ? k_grid_rows_kb<X, true, true> : k_grid_rows_kb<X, true, false>)
+                    : (n_sets > 1 ? k_grid_rows_kb<X, false, true> : k_grid_rows_kb<X, false, false>);
     };
     const auto k = first.kb_size <= 8 ? pick(std::integral_constant<int, 8>{})
                                       : pick(std::integral_constant<int, 0>{});
     hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kKbRowThreads), lds, stream, first, sets,
-                       img_set, plan, team, rb, gi0, n_img, (float2*)inter, (const float2*)tw,
+                       img_set, plan, rb, gi0, n_img, (float2*)inter, (const float2*)tw,
                        blocked ? 1 : 0);
     return hipGetLastError();
 }
@@ -1754,29 +1708,24 @@ hipError_t launch_grid_rows_kb(const SetDesc& first, const SetDesc* sets, const 
 // are not 16-byte aligned); the store applies the odd-side fftshift
 // (shift_index: p <-> p + m + 1 for p < m, the middle element fixed,
 // src/pacer_imager.cpp:30-35,110-128) element by element.
-template <int S, bool kBlockTeam, bool kMulti>
-__global__ void __launch_bounds__(kFftThreads)
+template <bool kMulti>
+__global__ void __launch_bounds__(1024)
 k_cols_half_odd(SetDesc first, const SetDesc* __restrict__ sets, const int* __restrict__ img_set,
-                FftPlan plan, int team, int pairs, int64_t gi0, const float2* __restrict__ inter,
+                FftPlan plan, int pairs, int64_t gi0, const float2* __restrict__ inter,
                 const float2* __restrict__ tw) {
     extern __shared__ float4 cho_lds4[];
     const int n = plan.n, h = n / 2;
     const int ld = n + 1;
-    float2* rows = (float2*)cho_lds4;  // [pairs][ld]
-    const int teams = kBlockTeam ? 1 : (int)blockDim.x / team;
-    const int t_id = kBlockTeam ? 0 : (int)threadIdx.x / team;
-    const int lane = kBlockTeam ? (int)threadIdx.x : (int)threadIdx.x % team;
-    float2* tmp = rows + (size_t)pairs * ld + (size_t)t_id * n;
-    float2* twl = rows + (size_t)pairs * ld + (size_t)teams * n;  // [n] when n <= kTwLdsMax
-    unsigned char* nonempty = (unsigned char*)twl + tw_lds_bytes(n);
-    const float2* twp = n <= kTwLdsMax ? twl : tw;
-    if (n <= kTwLdsMax)
-        for (int i = threadIdx.x; i < n; i += blockDim.x) twl[i] = tw[i];
+    float2* rows = (float2*)cho_lds4;         // [pairs][ld]
+    float2* twl = rows + (size_t)pairs * ld;  // twiddle table copy [n]
+    unsigned char* nonempty = (unsigned char*)(twl + n);
+    load_twiddles(twl, tw, n);
 
     const int n_slots = h + 1;
     const int n_cb = (n_slots + pairs - 1) / pairs;
-    const int cbk = (int)(blockIdx.x % n_cb);
-    const int li = (int)(blockIdx.x / n_cb);
+    const unsigned bid = xcd_order(blockIdx.x, gridDim.x);
+    const int cbk = (int)(bid % n_cb);
+    const int li = (int)(bid / n_cb);
     const int64_t gi = gi0 + li;
     const SetDesc sd = set_of<kMulti>(first, sets, img_set, gi);
     if (!sd.images) return;  // uniform per workgroup
@@ -1808,18 +1757,7 @@ k_cols_half_odd(SetDesc first, const SetDesc* __restrict__ sets, const int* __re
         if (v > 0) zr[n - v] = make_float2(a.x + b.y, b.x - a.y);    // row N - v
     }
     __syncthreads();
-    const int rounds = kBlockTeam ? np : (np + teams - 1) / teams;
-    for (int k = 0; k < rounds; k++) {
-        const int t = kBlockTeam ? k : k * teams + t_id;
-        if (!kBlockTeam && t >= np) break;
-        float2* zr = rows + (size_t)t * ld;
-        const float2* res = fft_row<S, kBlockTeam>(zr, tmp, plan, twp, lane, team);
-        if (res != zr) {
-            for (int i = lane; i < n; i += team) zr[i] = res[i];
-            team_sync<kBlockTeam>();
-        }
-    }
-    __syncthreads();
+    fft_tile<1>(rows, np, ld, plan, twl);
     const float s = (float)(1.0 / (double)count);
     float2* out = sd.images + (int64_t)img * n * n;
     for (int i = threadIdx.x; i < np * n; i += (int)blockDim.x) {
@@ -1833,21 +1771,20 @@ k_cols_half_odd(SetDesc first, const SetDesc* __restrict__ sets, const int* __re
     }
 }
 
-// Buffer columns (image rows) per workgroup of k_cols_half: the largest even divisor of
-// n, at most 64, whose LDS rows fit next to the team scratch and that still
-// gives at least 256 workgroups over the n_img images (one per CU), else the
-// smallest, 2 (a single 180^2 image then runs 90 workgroups, not 3).
-static int half_cols_block(int n, int teams, int64_t n_img, int max_cb) {
-    int fallback = 0;
-    for (int cb = std::min(max_cb, n); cb >= 2; cb--) {
-        if (cb % 2 || n % cb) continue;
-        const int64_t lds = sizeof(float2) * ((int64_t)(cb / 2) * (n + 1) + (int64_t)teams * n) +
-                            (int64_t)tw_lds_bytes(n) + (n / 2 + 1);
-        if (lds > g_lds_budget) continue;
-        if ((int64_t)(n / cb) * n_img >= 256) return cb;
-        fallback = cb;
-    }
-    return fallback;
+// Pairs of buffer columns (image rows) per workgroup of the second pass: 8
+// (128-byte runs of the buffer's rows) or, up to 256, 16, while the workgroup's threads hold them in
+// registers and two workgroups, or one, fit a CU's LDS; fewer while the launch
+// has under 512 workgroups (two per CU).
+static int half_pairs(const FftPlan& plan, int n_slots, int64_t n_img) {
+    const int n = plan.n;
+    int pairs = std::min(n <= 256 ? 16 : 8, n_slots);
+    auto lds_of = [&](int p) { return sizeof(float2) * ((size_t)p * (n + 1) + n) + n / 2 + 1; };
+    while (pairs > 1 && ((int64_t)pairs * n > 1024 * plan.cap ||
+                         (int64_t)lds_of(pairs) > g_lds_limit ||
+                         (pairs > 4 && 2 * (int64_t)lds_of(pairs) > g_lds_limit) ||
+                         (int64_t)((n_slots + pairs - 1) / pairs) * n_img < 512))
+        pairs--;
+    return pairs;
 }
 
 hipError_t launch_cols_half(const SetDesc& first, const SetDesc* sets, const int* img_set,
@@ -1855,51 +1792,18 @@ hipError_t launch_cols_half(const SetDesc& first, const SetDesc* sets, const int
                             const float* inter, const float* tw, hipStream_t stream) {
     if (n_img == 0) return hipSuccess;
     const int n = plan.n;
-    // Sides up to 256: teams of 16 lanes and at most one column pair per team,
-    // so that every pair of a workgroup is transformed in one round (768 x
-    // 180^2: 30-column blocks with 16-lane teams 84 us per launch, against
-    // 115 us with 60-column blocks and 32-lane teams in two rounds).
-    const bool one_round = n <= 256;
-    const int team = one_round ? 16 : fft_team_for(n);
-    const bool block_team = team == kFftThreads;
-    const int teams = block_team ? 1 : kFftThreads / team;
-    if (n % 2) {
-        // odd N: slots of column pairs per workgroup, as many as fit up to 32
-        // (one per team up to 256), and at least ~256 workgroups over the
-        // images
-        const int n_slots = n / 2 + 1;
-        auto lds_of = [&](int p) {
-            return sizeof(float2) * ((size_t)p * (n + 1) + (size_t)teams * n) + tw_lds_bytes(n) +
-                   (size_t)(n / 2 + 1);
-        };
-        int pairs = std::min(one_round ? teams : 32, n_slots);
-        while (pairs > 1 && (!lds_fits(lds_of(pairs)) ||
-                             (int64_t)((n_slots + pairs - 1) / pairs) * n_img < 256))
-            pairs--;
-        if (!lds_fits(lds_of(pairs))) return hipErrorInvalidConfiguration;
-        const int64_t blocks = (int64_t)((n_slots + pairs - 1) / pairs) * n_img;
-        if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-        const bool multi = n_sets > 1;
-        auto k = block_team
-                     ? (multi ? k_cols_half_odd<1, true, true> : k_cols_half_odd<1, true, false>)
-                     : (multi ? k_cols_half_odd<1, false, true> : k_cols_half_odd<1, false, false>);
-        hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kFftThreads), lds_of(pairs), stream,
-                           first, sets, img_set, plan, team, pairs, gi0, (const float2*)inter,
-                           (const float2*)tw);
-        return hipGetLastError();
-    }
-    const int cb = half_cols_block(n, teams, n_img, one_round ? 2 * teams : 64);
-    if (!cb) return hipErrorInvalidConfiguration;
-    const size_t lds = sizeof(float2) * ((size_t)(cb / 2) * (n + 1) + (size_t)teams * n) +
-                       tw_lds_bytes(n) + (size_t)(n / 2 + 1);
-    if (!lds_fits(lds)) return hipErrorInvalidConfiguration;
-    const int64_t blocks = (int64_t)(n / cb) * n_img;
-    if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    // odd N: the last column pairs with zeros
+    const int n_slots = n % 2 ? n / 2 + 1 : n / 2;
+    const int pairs = half_pairs(plan, n_slots, n_img);
+    const size_t lds = sizeof(float2) * ((size_t)pairs * (n + 1) + n) + (size_t)(n / 2 + 1);
+    const int64_t blocks = (int64_t)((n_slots + pairs - 1) / pairs) * n_img;
+    if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
     const bool multi = n_sets > 1;
-    auto k = block_team ? (multi ? k_cols_half<1, true, true> : k_cols_half<1, true, false>)
-                        : (multi ? k_cols_half<1, false, true> : k_cols_half<1, false, false>);
-    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kFftThreads), lds, stream, first, sets,
-                       img_set, plan, team, cb, gi0, (const float2*)inter, (const float2*)tw);
+    auto k = n % 2 ? (multi ? k_cols_half_odd<true> : k_cols_half_odd<false>)
+                   : (multi ? k_cols_half<true> : k_cols_half<false>);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(fft_threads(plan, (int64_t)pairs * n)), lds,
+                       stream, first, sets, img_set, plan, pairs, gi0, (const float2*)inter,
+                       (const float2*)tw);
     return hipGetLastError();
 }
 
@@ -1925,20 +1829,14 @@ hipError_t set_kernel_attributes() {
         if (r != hipSuccess && e == hipSuccess) e = r;
     };
     set((const void*)k_grid_half_direct);
+    set((const void*)k_grid_rows_fft<false>);
+    set((const void*)k_grid_rows_fft<true>);
+    set((const void*)k_cols_half<false>);
+    set((const void*)k_cols_half<true>);
+    set((const void*)k_cols_half_odd<false>);
+    set((const void*)k_cols_half_odd<true>);
     set((const void*)k_grid_rows_direct_fft<false>);
     set((const void*)k_grid_rows_direct_fft<true>);
-    set((const void*)k_grid_rows_fft<1, true, false>);
-    set((const void*)k_grid_rows_fft<1, false, false>);
-    set((const void*)k_grid_rows_fft<1, true, true>);
-    set((const void*)k_grid_rows_fft<1, false, true>);
-    set((const void*)k_cols_half<1, true, false>);
-    set((const void*)k_cols_half<1, false, false>);
-    set((const void*)k_cols_half<1, true, true>);
-    set((const void*)k_cols_half<1, false, true>);
-    set((const void*)k_cols_half_odd<1, true, false>);
-    set((const void*)k_cols_half_odd<1, false, false>);
-    set((const void*)k_cols_half_odd<1, true, true>);
-    set((const void*)k_cols_half_odd<1, false, true>);
     set((const void*)k_grid_slabs);
     set((const void*)k_grid_kb_slabs<8>);
     set((const void*)k_grid_kb_slabs<0>);

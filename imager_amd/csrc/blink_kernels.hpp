@@ -14,11 +14,9 @@ namespace blink {
 constexpr int kMaxPixels = 8192;      // largest grid side (plan entries pack positions in 13 bits)
 constexpr int kMaxBaselines = 1 << 18;  // plan packs the baseline in 18 bits
 constexpr int kTileThreads = 256;
-constexpr int kFftThreads = 256;
 // Columns per block of the register kernels' column-blocked row-pass buffer.
 constexpr int kInterBlockCols = 32;
 constexpr int kMaxTileRows = 16;
-constexpr int kMaxColWidth = 16;
 
 // LDS bytes a workgroup may allocate dynamically (device limit), and the
 // share the tile-sizing heuristics aim for.  Set once per process from the
@@ -134,7 +132,6 @@ struct StageFftArgs {
 int device_cu_count();
 
 bool make_fft_plan(int n, FftPlan& plan);
-int grid_rows_tile_rows(int n);
 hipError_t set_kernel_attributes();
 
 hipError_t launch_phase_correct(float* vis, int n_ant, int n_ch, int n_t, const float* w_m,

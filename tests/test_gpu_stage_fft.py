@@ -109,3 +109,23 @@ def test_image_nan_and_no_counts(ctx):
     assert not torch.isfinite(images[1].real).any()
     assert torch.isfinite(torch.view_as_real(images[2])).all()
     assert not torch.view_as_real(g).view(torch.int32).any()
+
+
+@pytest.mark.parametrize("n", [3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 15, 16, 18, 26, 33, 36, 84, 96, 130, 192, 243, 400, 500, 729,
+                               770, 968, 1040, 1331, 3072, 3125, 3600, 4004, 8192])
+def test_every_radix(ctx, n):
+    """Sides whose plans hold every radix, alone and together, one to four passes and more rows
+    than a workgroup's threads hold at once, forward and backward."""
+    import torch
+    batch = 3 if n < 1000 else 1
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.view_as_complex(torch.randn((batch, n, n, 2), device="cuda", generator=gen))
+    out = torch.empty_like(x)
+    for direction, f in ((1, lambda t: torch.fft.ifft2(t, norm="forward")), (-1, torch.fft.fft2)):
+        ctx.fft2d_c2c(x, out, n, batch, direction)
+        torch.cuda.synchronize()
+        want = f(x.to(torch.complex128))
+        err = (torch.linalg.vector_norm(out.to(torch.complex128) - want) /
+               torch.linalg.vector_norm(want)).item()
+        print(f"fft {n}^2 {direction}: {err:.2e} of {_tolerance(n):.2e}", flush=True)
+        assert err <= _tolerance(n)

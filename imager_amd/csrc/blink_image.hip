@@ -62,6 +62,16 @@ __device__ __forceinline__ void exchange_planes(float2 (&v)[F::V], float* buf, i
     }
 }
 
+// The first half of a twiddle table: w(m + N / 2) = -w(m).
+template <int N>
+struct TwHalf {
+    const float2* t;
+    __device__ __forceinline__ float2 operator()(int m) const {
+        const float2 w = t[m & (N / 2 - 1)];
+        return m & (N / 2) ? make_float2(-w.x, -w.y) : w;
+    }
+};
+
 template <class F, int S, bool kBlock, int P = 0, class TW, class Slot>
 __device__ __forceinline__ void run_planes(float2 (&v)[F::V], float* buf, int lane, const TW& tw,
                                            Slot slot) {
@@ -72,21 +82,28 @@ __device__ __forceinline__ void run_planes(float2 (&v)[F::V], float* buf, int la
     }
 }
 
+// Lanes per row, threads per workgroup.  One team per workgroup where a row needs
+// several wavefronts, so that the workgroups of a CU drift apart and one loads
+// while another transforms (4 x 4096^2: 759 -> 723 us per stage call).
 template <int N>
-struct RowShape;  // lanes per row, threads per workgroup
+struct RowShape;
 template <> struct RowShape<128> { static constexpr int L = 16, NT = 256; };
 template <> struct RowShape<256> { static constexpr int L = 32, NT = 256; };
 template <> struct RowShape<512> { static constexpr int L = 64, NT = 256; };
 template <> struct RowShape<1024> { static constexpr int L = 64, NT = 256; };
-template <> struct RowShape<2048> { static constexpr int L = 128, NT = 256; };
-template <> struct RowShape<4096> { static constexpr int L = 256, NT = 512; };
+template <> struct RowShape<2048> { static constexpr int L = 128, NT = 128; };
+template <> struct RowShape<4096> { static constexpr int L = 256, NT = 256; };
 
+// Columns and lanes per column of a workgroup: 64- or 128-byte runs, two or more
+// workgroups per CU up to 2048 (1024^2: 8 columns 251, 16 columns 260 us per
+// stage call of 24 images; 4096^2: 4 columns, two workgroups per CU, 752 against
+// 723 us).
 template <int N>
-struct ColShape;  // columns and lanes per column of a workgroup
+struct ColShape;
 template <> struct ColShape<128> { static constexpr int W = 16, L = 16; };
 template <> struct ColShape<256> { static constexpr int W = 16, L = 32; };
 template <> struct ColShape<512> { static constexpr int W = 16, L = 32; };
-template <> struct ColShape<1024> { static constexpr int W = 16, L = 64; };
+template <> struct ColShape<1024> { static constexpr int W = 8, L = 64; };
 template <> struct ColShape<2048> { static constexpr int W = 8, L = 128; };
 template <> struct ColShape<4096> { static constexpr int W = 8, L = 128; };
 
@@ -128,11 +145,11 @@ k_stage_rows(StageFftArgs a, int iters, const float2* __restrict__ tw) {
     constexpr int PL = padded_len(N);
     using F = RegFft<N, L>;
     extern __shared__ float stage_rows_lds[];
-    float2* twl = (float2*)stage_rows_lds;  // [N]
-    float* plane = stage_rows_lds + 2 * N;  // [TEAMS][PL]
+    float2* twl = (float2*)stage_rows_lds;  // [N / 2]
+    float* plane = stage_rows_lds + N;      // [TEAMS][PL]
     __shared__ double red[NT / 64];
     const int tid = threadIdx.x, team = tid / L, lane = tid % L;
-    for (int i = tid; i < N; i += NT) twl[i] = tw[i];
+    for (int i = tid; i < N / 2; i += NT) twl[i] = tw[i];
     __syncthreads();
     float* buf = plane + team * PL;
     double sum = 0.0;
@@ -171,7 +188,7 @@ k_stage_rows(StageFftArgs a, int iters, const float2* __restrict__ tw) {
             if (lane == 0) a.used[row] = used ? 1 : 0;
             if (!used) continue;  // uniform per team (per workgroup with kBlock)
         }
-        run_planes<F, S, kBlock>(v, buf, lane, TwTable{twl}, [](int i) { return pad_index(i); });
+        run_planes<F, S, kBlock>(v, buf, lane, TwHalf<N>{twl}, [](int i) { return pad_index(i); });
         float2* dst = a.out + row * N;
         F::store(v, lane, [&](int i, float2 x) {
             dst[kImage ? (i < N / 2 ? i + N / 2 : i - N / 2) : i] = x;
@@ -376,7 +393,7 @@ template <int N, int S, bool kImage>
 static hipError_t rows_n(const StageFftArgs& a, int64_t n_img, const float2* tw, hipStream_t s) {
     constexpr int TEAMS = RowShape<N>::NT / RowShape<N>::L;
     const int it = row_iters<N>(n_img);
-    const size_t lds = sizeof(float) * (2 * N + (size_t)TEAMS * padded_len(N));
+    const size_t lds = sizeof(float) * (N + (size_t)TEAMS * padded_len(N));
     const int64_t blocks = n_img * N / (TEAMS * it);
     if (blocks > 0x7fffffff || (int64_t)lds > g_lds_limit) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((k_stage_rows<N, S, kImage>), dim3((unsigned)blocks),

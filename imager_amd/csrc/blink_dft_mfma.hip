@@ -13,21 +13,31 @@
 // image is real.  Stage 2 multiplies by (float)(1 / sum counts) and writes the
 // imaginary part as 0.
 //
-// Both stages are one kernel, C[n][m] = sum_k D[n][k] A[m][k]:
-//   stage 1: A[m = (img, v)][k = u] = half rows,   C stored at inter[img][x = n][v]
-//   stage 2: A[m = (img, x)][k = v] = inter rows,  C stored at images[img][y = n][x]
-// Rows of the MFMA result are n and columns are m, so the 32 lanes that hold
-// one n store 32 consecutive m: one 256-byte segment.
+// Both stages fold the symmetry of the matrices: frequency rows j and N - j of
+// D hold conjugate values, so only j = 0 .. H is multiplied and every result
+// serves the two outputs x = H + j (p(x) = j, j < H) and x = H - j (p(x) =
+// N - j, j > 0).  With c, s = cos, sin(2 pi j k / N):
+//   stage 1: E[u] = G[u] + G[N - u], O[u] = G[u] - G[N - u] for 0 < u < H
+//            (E = G, O = 0 at u = 0 and H);  P = sum c E, Q = sum s O over
+//            u = 0 .. H;  T[H + j] = P + iQ, T[H - j] = P - iQ;
+//   stage 2: P = sum w c Re T, Q = sum w s Im T over v;  I[H + j] = P - Q,
+//            I[H - j] = P + Q.
+// That is a quarter (stage 1) and a half (stage 2) of the unfolded products,
+// and K = H + 1 in both.
+//
+// The matrix is the first MFMA operand (rows j), the data the second (columns
+// m), so the 32 lanes that hold one j store 32 consecutive m: one 256-byte
+// segment.
+//   stage 1: m = (img, v): half rows in,  inter[img][x][v] out
+//   stage 2: m = (img, x): inter rows in, images[img][y][x] out
 //
 // Precision: every operand x is split into hi = P(x) and lo = P(x - hi),
 // P = bf16 or fp16, and products use hi*hi + hi*lo + lo*hi (lo*lo is below
-// the FP32 rounding of the sum) with FP32 accumulation in MFMA.  D1 and D2
+// the FP32 rounding of the sum) with FP32 accumulation in MFMA.  The matrices
 // are built on the host in double and split there; the data are split on the
-// fly.  fp16 has 5 exponent bits, so each data row m is first scaled by a
-// power of two 2^e that brings its largest component below 2^15 (exact), and
-// the result column m is scaled back by 2^-e.  Complex products use
-// C_re = Dr Ar + Di (-Ai) and C_im = Dr Ai + Di Ar; -Ai is the sign-flipped
-// split of Ai.
+// fly.  fp16 has 5 exponent bits, so each (folded) data row m is first scaled
+// by a power of two 2^e that brings its largest component below 2^15 (exact),
+// and the result column m is scaled back by 2^-e.
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -36,12 +46,16 @@
 
 namespace blink {
 
+constexpr int kDftMaxTiles = (512 / 2 + 1 + 31) / 32;  // at N = 512, the largest side
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-// Plane order of a split DFT matrix, each [n_pad][k_pad] 16-bit values, k contiguous.
+// Planes of a split DFT matrix.  The matrix is stored as MFMA operands, in the
+// order in which a wave reads them: [32-row tile][16-column step][plane][lane]
+// [8], lane l holding row l % 32 and columns 8 (l / 32) .. + 7 of its step.
 enum { kReHi = 0, kReLo, kImHi, kImLo, kDftPlanes };
 
 template <int kPrec>
@@ -65,20 +79,14 @@ struct Prec<kDftFp16> {
     }
 };
 
-template <typename V>
-__device__ __forceinline__ V neg8(V x) {
-    u32x4 b = __builtin_bit_cast(u32x4, x);
-    b ^= 0x80008000u;
-    return __builtin_bit_cast(V, b);
-}
-
 struct DftGemmArgs {
-    const float2* a;          // data rows [m][lda], k < K valid
+    const float2* a;          // data rows [m][lda]
     int64_t lda;              // row stride of a (float2, even)
     int64_t m_rows;           // M
-    int K, k_pad;             // valid k; k_pad a multiple of 16
-    int n, n_pad;             // output rows n < N; n_pad a multiple of 64
-    const uint16_t* planes;   // kDftPlanes x [n_pad][k_pad]
+    int n, h;                 // N (even) and N / 2: K = h + 1 columns
+    int k_pad;                // K rounded up to 16
+    int n_tiles;              // 32-row tiles of the matrix rows j = 0 .. h
+    const uint16_t* planes;   // split matrix (see kDftPlanes)
     int R;                    // m -> (img = m / R, r = m % R)
     int64_t img_stride, n_stride;  // C[n][m] at out[img * img_stride + n * n_stride + r]
     float2* out;
@@ -87,238 +95,306 @@ struct DftGemmArgs {
     int64_t img0;             // set-relative index of the first image
 };
 
-// 8 consecutive complex values of a data row from k = kb, zero beyond K or
-// for rows past M.
-__device__ __forceinline__ void load8(const float2* row, bool ok, int kb, int K, float2 (&xs)[8]) {
-    if (ok && kb + 8 <= K) {
-        const float4* p4 = (const float4*)(row + kb);
+// The 8 folded values u = kb .. kb + 7 of a row of N: E into xs[0..7], O into
+// xs[8..15], zero beyond u = h.  `wide`: every octet lies within the row, so
+// its two ranges are loaded 16 bytes at a time (rows are 16-byte aligned, N is
+// even): u .. u + 7 forwards, and N - u - 8 .. N - u - 1 with N - u by itself.
+__device__ __forceinline__ void load_folded(const float2* row, int kb, int n, int h, bool wide,
+                                            float2 (&xs)[16]) {
+    float2 f[8], b[8];  // G[u], G[N - u] (0 < u < h)
+    if (wide) {
+        const float4* f4 = (const float4*)(row + kb);
+        const float4* b4 = (const float4*)(row + (n - kb - 8));
+        b[0] = kb ? row[n - kb] : make_float2(0.f, 0.f);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const float4 t = p4[q];
-            xs[2 * q] = make_float2(t.x, t.y);
-            xs[2 * q + 1] = make_float2(t.z, t.w);
+            const float4 t = f4[q], w = b4[q];
+            f[2 * q] = make_float2(t.x, t.y);
+            f[2 * q + 1] = make_float2(t.z, t.w);
+            // w = G[N - kb - 8 + 2q], G[N - kb - 7 + 2q]
+            if (q > 0) b[8 - 2 * q] = make_float2(w.x, w.y);
+            b[7 - 2 * q] = make_float2(w.z, w.w);
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < 8; e++)
-            xs[e] = (ok && kb + e < K) ? row[kb + e] : make_float2(0.f, 0.f);
+        for (int e = 0; e < 8; e++) {
+            const int u = kb + e;
+            f[e] = u <= h ? row[u] : make_float2(0.f, 0.f);
+            b[e] = (u > 0 && u < h) ? row[n - u] : make_float2(0.f, 0.f);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int u = kb + e;
+        const bool in = u <= h, pair = u > 0 && u < h;
+        xs[e].x = pair ? f[e].x + b[e].x : (in ? f[e].x : 0.f);
+        xs[e].y = pair ? f[e].y + b[e].y : (in ? f[e].y : 0.f);
+        xs[8 + e].x = pair ? f[e].x - b[e].x : 0.f;
+        xs[8 + e].y = pair ? f[e].y - b[e].y : 0.f;
     }
 }
 
-// Workgroup = 8 waves sharing one slice of NS = 32 * NSUB rows of D, held in
-// LDS for the workgroup's lifetime (rows padded by 16 bytes so that the 32
-// lanes reading one k column hit distinct banks).  The workgroup walks the m
-// tiles of 256 rows (one 32-row MFMA tile per wave) with a stride of the
-// number of workgroups per slice; each wave splits its data rows once per
-// k-step and applies them to its NSUB D tiles.  The next k-step's data are
-// loaded before the current step's MFMAs are issued.
-constexpr int kGemmThreads = 512;
-constexpr int kGemmRows = 32 * (kGemmThreads / 64);  // m rows per tile
+// The 8 values v = kb .. kb + 7 of a stage-1 row, zero beyond v = h (the row's
+// storage reaches k_pad).
+__device__ __forceinline__ void load_row8(const float2* row, int kb, int h, float2 (&xs)[8]) {
+    const float4* p4 = (const float4*)(row + kb);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4 t = p4[q];
+        const bool a = kb + 2 * q <= h, b = kb + 2 * q + 1 <= h;
+        xs[2 * q] = make_float2(a ? t.x : 0.f, a ? t.y : 0.f);
+        xs[2 * q + 1] = make_float2(b ? t.z : 0.f, b ? t.w : 0.f);
+    }
+}
 
-__host__ __device__ constexpr int dft_lds_ld(int k_pad) { return k_pad + 8; }
+constexpr int kOctetStride = 512 + 16;  // bytes: 32 rows x 16, and one bank group of padding
 
-template <int kPrec, bool kComplex, int NSUB>
-__global__ void __launch_bounds__(kGemmThreads) k_dft_gemm(DftGemmArgs g) {
+// 8 complex values -> hi and lo of the real and the imaginary parts.
+template <int kPrec>
+__device__ __forceinline__ void split8(const float2* x, float sc,
+                                       typename Prec<kPrec>::V (&v)[4]) {
+    using S = Prec<kPrec>;
+    using E = typename S::E;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float re = S::kScale ? x[e].x * sc : x[e].x;
+        const float im = S::kScale ? x[e].y * sc : x[e].y;
+        const E rh = (E)re, ih = (E)im;
+        v[0][e] = rh;
+        v[1][e] = (E)(re - (float)rh);
+        v[2][e] = ih;
+        v[3][e] = (E)(im - (float)ih);
+    }
+}
+
+// A workgroup takes 32 * kTiles data rows: its threads read them once, 8
+// columns of a row at a time (coalesced, every load of a batch in flight
+// together), and leave them in LDS as split MFMA operands, plane by plane:
+// 16 bytes per (row, octet).  Each wave then multiplies them by the 32-row
+// matrix tiles t = wave, wave + waves, ..., which come from L2 in operand
+// order (1 KB per load, the next step's under the current step's MFMAs): the
+// whole matrix is 4 k_pad bytes x 2 per row, 74 KB at N = 180, and every
+// workgroup reads the same.  fp16 first needs the largest component of each
+// row: the values wait in LDS as FP32, in the bytes of their own later
+// operands, for one barrier.
+//
+// Bound by HBM: at N = 180 the two stages of 768 images move 207 and 305 MB
+// and take 53 and 90 us (fp16), 3.9 and 3.4 TB/s; with the unfolded matrix in
+// LDS in slices of 64 rows, each of which read all the data (twice, for the
+// row maxima), they took 194 and 181 us.
+// Whole calls in us, before -> after: 768 x 180^2 fp16 575 -> 357, 100 x 256^2
+// fp16 197 -> 132, 40 x 512^2 fp16 373 -> 165, bf16 247 -> 164, 3 x 180^2 fp16
+// 82 -> 60.
+template <int kPrec, bool kComplex>
+__global__ void __launch_bounds__(64 * kDftMaxTiles) k_dft_gemm(DftGemmArgs g) {
     using S = Prec<kPrec>;
     using V = typename S::V;
-    using E = typename S::E;
-    constexpr int NS = 32 * NSUB;
+    constexpr int kTiles = kComplex ? 1 : 2;   // 32-row data tiles
+    constexpr int kHalves = kComplex ? 2 : 1;  // E and O, or T: 4 planes each
+    constexpr int kRows = 32 * kTiles;
+    constexpr int kBatch = kComplex ? 2 : 4;   // octets a thread loads together
     extern __shared__ float4 dft_lds4[];
-    uint16_t* dl = (uint16_t*)dft_lds4;  // [kDftPlanes][NS][ldk]
-    const int ldk = dft_lds_ld(g.k_pad);
-    const int n_slices = g.n_pad / NS;
-    const unsigned bid = xcd_order(blockIdx.x, gridDim.x);
-    const int slice = (int)(bid % n_slices);
-    const int grp = (int)(bid / n_slices);
-    const int n_grp = (int)(gridDim.x / n_slices);
-    const int n_base = slice * NS;
+    char* lds = (char*)dft_lds4;  // [8 planes][k_pad / 8 octets][kOctetStride]
+    __shared__ unsigned rmax[kRows];
+    const int n_oct = g.k_pad >> 3;
+    const int plane = n_oct * kOctetStride;
+    const int64_t m0 = (int64_t)xcd_order(blockIdx.x, gridDim.x) * kRows;
+    const int n_thr = (int)blockDim.x;
+    const int items = kRows * n_oct;
+    if (S::kScale) {
+        for (int i = (int)threadIdx.x; i < kRows; i += n_thr) rmax[i] = 0;
+        __syncthreads();
+    }
 
-    // the D slice, 16 bytes per thread and step
-    {
-        const size_t plane = (size_t)g.n_pad * g.k_pad;
-        const int cpr = g.k_pad / 8;  // 16-byte chunks per row
-        const int per_plane = NS * cpr;
-        for (int i = threadIdx.x; i < kDftPlanes * per_plane; i += kGemmThreads) {
-            const int p = i / per_plane, rem = i % per_plane;
-            const int r = rem / cpr, c = rem % cpr;
-            *(uint4*)(dl + ((size_t)p * NS + r) * ldk + 8 * c) =
-                *(const uint4*)(g.planes + p * plane + (size_t)(n_base + r) * g.k_pad + 8 * c);
+    const bool wide = g.k_pad <= g.n;
+    for (int base = (int)threadIdx.x; base < items; base += kBatch * n_thr) {
+        float2 xs[kBatch][8 * kHalves];
+        int row[kBatch], oct[kBatch];
+#pragma unroll
+        for (int b = 0; b < kBatch; b++) {
+            // past the end: the last item again, not kept
+            const int i = min(base + b * n_thr, items - 1);
+            row[b] = i / n_oct;
+            oct[b] = i - row[b] * n_oct;
+            // rows past M repeat the last one; their results are not stored
+            const float2* a = g.a + min(m0 + row[b], g.m_rows - 1) * g.lda;
+            if constexpr (kComplex) load_folded(a, 8 * oct[b], g.n, g.h, wide, xs[b]);
+            else load_row8(a, 8 * oct[b], g.h, xs[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < kBatch; b++) {
+            if (base + b * n_thr >= items) break;
+            char* at = lds + (row[b] >> 5) * 4 * plane + oct[b] * kOctetStride + (row[b] & 31) * 16;
+            if constexpr (S::kScale) {
+                float mx = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8 * kHalves; e++)
+                    mx = fmaxf(mx, fmaxf(fabsf(xs[b][e].x), fabsf(xs[b][e].y)));
+                atomicMax(&rmax[row[b]], __float_as_uint(mx));
+#pragma unroll
+                for (int c = 0; c < 4 * kHalves; c++)
+                    *(float4*)(at + c * plane) = make_float4(xs[b][2 * c].x, xs[b][2 * c].y,
+                                                             xs[b][2 * c + 1].x, xs[b][2 * c + 1].y);
+            } else {
+#pragma unroll
+                for (int p = 0; p < kHalves; p++) {
+                    V v[4];
+                    split8<kPrec>(&xs[b][8 * p], 1.f, v);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) *(V*)(at + (4 * p + c) * plane) = v[c];
+                }
+            }
         }
     }
     __syncthreads();
-
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int kq = (lane >> 5) * 8;  // this lane's k offset within a step
-    const size_t lplane = (size_t)NS * ldk;
-    const uint16_t* dlane = dl + (size_t)(lane & 31) * ldk + kq;
-    const int64_t m_tiles = (g.m_rows + kGemmRows - 1) / kGemmRows;
-
-    for (int64_t mt = grp; mt < m_tiles; mt += n_grp) {
-        const int64_t m0 = mt * kGemmRows + wave * 32;
-        if (m0 >= g.m_rows) continue;  // wave-uniform: no rows for this wave
-        const int64_t mrow = m0 + (lane & 31);
-        const bool mok = mrow < g.m_rows;
-        const float2* arow = g.a + (mok ? mrow : 0) * g.lda + kq;
-        const int kv = g.K - kq;  // valid k relative to this lane's offset
-
-        // fp16: power-of-two scale from the row's largest component
-        float sc = 1.f, unsc = 1.f;
-        if constexpr (S::kScale) {
-            float mx = 0.f;
-            for (int k0 = 0; k0 < g.k_pad; k0 += 16) {
-                float2 xs[8];
-                load8(arow, mok, k0, kv, xs);
-#pragma unroll
-                for (int e = 0; e < 8; e++) mx = fmaxf(mx, fmaxf(fabsf(xs[e].x), fabsf(xs[e].y)));
-            }
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            if (mx > 0.f && mx < INFINITY) {
-                int ex;
-                (void)frexpf(mx, &ex);                       // mx < 2^ex
-                const int e = max(-126, min(126, 15 - ex));  // mx * 2^e < 2^15
-                sc = __int_as_float((127 + e) << 23);
-                unsc = __int_as_float((127 - e) << 23);
-            }
+    // fp16: power-of-two scale of a row from its largest component
+    auto row_exp = [&](int r) {
+        const float mx = __uint_as_float(rmax[r]);
+        int e = 0;
+        if (mx > 0.f && mx < INFINITY) {
+            int ex;
+            (void)frexpf(mx, &ex);               // mx < 2^ex
+            e = max(-126, min(126, 15 - ex));    // mx * 2^e < 2^15
         }
-
-        f32x16 cre[NSUB], cim[NSUB];
+        return e;
+    };
+    if constexpr (S::kScale) {
+        for (int i = (int)threadIdx.x; i < items; i += n_thr) {
+            const int r = i / n_oct, o = i - r * n_oct;
+            const float sc = __int_as_float((127 + row_exp(r)) << 23);
+            char* at = lds + (r >> 5) * 4 * plane + o * kOctetStride + (r & 31) * 16;
 #pragma unroll
-        for (int s = 0; s < NSUB; s++) {
-            cre[s] = f32x16{};
-            cim[s] = f32x16{};
-        }
-        float2 xs[8];
-        load8(arow, mok, 0, kv, xs);
-        for (int k0 = 0; k0 < g.k_pad; k0 += 16) {
-            V ar_h, ar_l, ai_h, ai_l;
+            for (int p = 0; p < kHalves; p++) {
+                float2 x[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                float2 x = xs[e];
-                if constexpr (S::kScale) {
-                    x.x *= sc;
-                    x.y *= sc;
+                for (int c = 0; c < 4; c++) {
+                    const float4 t = *(const float4*)(at + (4 * p + c) * plane);
+                    x[2 * c] = make_float2(t.x, t.y);
+                    x[2 * c + 1] = make_float2(t.z, t.w);
                 }
-                const E rh = (E)x.x, ih = (E)x.y;
-                ar_h[e] = rh;
-                ar_l[e] = (E)(x.x - (float)rh);
-                ai_h[e] = ih;
-                ai_l[e] = (E)(x.y - (float)ih);
-            }
-            if (k0 + 16 < g.k_pad) load8(arow, mok, k0 + 16, kv, xs);
-            const V ni_h = neg8(ai_h), ni_l = neg8(ai_l);
+                V v[4];
+                split8<kPrec>(x, sc, v);
 #pragma unroll
-            for (int s = 0; s < NSUB; s++) {
-                const uint16_t* dp = dlane + (size_t)s * 32 * ldk + k0;
-                const V dr_h = *(const V*)(dp + kReHi * lplane);
-                const V dr_l = *(const V*)(dp + kReLo * lplane);
-                const V di_h = *(const V*)(dp + kImHi * lplane);
-                const V di_l = *(const V*)(dp + kImLo * lplane);
-                cre[s] = S::mfma(dr_h, ar_h, cre[s]);
-                cre[s] = S::mfma(dr_h, ar_l, cre[s]);
-                cre[s] = S::mfma(dr_l, ar_h, cre[s]);
-                cre[s] = S::mfma(di_h, ni_h, cre[s]);
-                cre[s] = S::mfma(di_h, ni_l, cre[s]);
-                cre[s] = S::mfma(di_l, ni_h, cre[s]);
-                if constexpr (kComplex) {
-                    cim[s] = S::mfma(dr_h, ai_h, cim[s]);
-                    cim[s] = S::mfma(dr_h, ai_l, cim[s]);
-                    cim[s] = S::mfma(dr_l, ai_h, cim[s]);
-                    cim[s] = S::mfma(di_h, ar_h, cim[s]);
-                    cim[s] = S::mfma(di_h, ar_l, cim[s]);
-                    cim[s] = S::mfma(di_l, ar_h, cim[s]);
-                }
+                for (int c = 0; c < 4; c++) *(V*)(at + (4 * p + c) * plane) = v[c];
             }
+        }
+        __syncthreads();
+    }
+
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = (int)threadIdx.x >> 6, waves = n_thr >> 6;
+    const int n_ks = g.k_pad >> 4;
+    const char* dlane = lds + (lane >> 5) * kOctetStride + (lane & 31) * 16;
+    for (int t = wave; t < g.n_tiles; t += waves) {
+        const V* dp = (const V*)g.planes + (size_t)t * n_ks * (kDftPlanes * 64) + lane;
+        // complex: P = p0 + i p1, Q = q0 + i q1; real: P, Q of data tile 0 and 1
+        f32x16 p0{}, p1{}, q0{}, q1{};
+        V d[kDftPlanes];
+#pragma unroll
+        for (int c = 0; c < kDftPlanes; c++) d[c] = dp[64 * c];
+        for (int ks = 0; ks < n_ks; ks++) {
+            V x[8], nd[kDftPlanes];
+            const V* dn = dp + (ks + 1 < n_ks ? ks + 1 : ks) * (kDftPlanes * 64);
+#pragma unroll
+            for (int c = 0; c < kDftPlanes; c++) nd[c] = dn[64 * c];
+#pragma unroll
+            for (int c = 0; c < 8; c++)
+                x[c] = *(const V*)(dlane + c * plane + ks * (2 * kOctetStride));
+            // complex: x = Er, Ei, Or, Oi (hi, lo); real: Re, Im of tile 0, then of tile 1
+            constexpr int kP1 = kComplex ? 2 : 4, kQ0 = kComplex ? 4 : 2;
+            auto mac = [&](const V& hi, const V& lo, int c, f32x16& acc) {
+                acc = S::mfma(hi, x[c], acc);
+                acc = S::mfma(hi, x[c + 1], acc);
+                acc = S::mfma(lo, x[c], acc);
+            };
+            mac(d[kReHi], d[kReLo], 0, p0);
+            mac(d[kReHi], d[kReLo], kP1, p1);
+            mac(d[kImHi], d[kImLo], kQ0, q0);
+            mac(d[kImHi], d[kImLo], 6, q1);
+#pragma unroll
+            for (int c = 0; c < kDftPlanes; c++) d[c] = nd[c];
         }
 
-        // acc[i] holds C[n = n_base + 32 s + 8(i/4) + 4(lane/32) + i%4][m = mrow]
-        if (!mok) continue;
-        const int64_t img = mrow / g.R;
-        const int r = (int)(mrow % g.R);
-        float scale = unsc;
-        if (g.isums) {
-            const uint32_t count = g.isums[g.img0 + img];
-            scale *= (float)(1.0 / (double)count);
-            if (g.count_sums && r == 0 && n_base == 0 && lane < 32)
-                g.count_sums[g.img0 + img] = (double)count;
-        }
-        float2* ob = g.out + img * g.img_stride + r;
+        // acc[i] holds row j = 32 t + 8(i/4) + 4(lane/32) + i%4 of column m
 #pragma unroll
-        for (int s = 0; s < NSUB; s++) {
+        for (int mt = 0; mt < kTiles; mt++) {
+            const int64_t m = m0 + 32 * mt + (lane & 31);
+            if (m >= g.m_rows) continue;
+            const int64_t img = m / g.R;
+            const int r = (int)(m - img * g.R);
+            float scale = 1.f;
+            if constexpr (S::kScale)
+                scale = __int_as_float((127 - row_exp(32 * mt + (lane & 31))) << 23);
+            if (!kComplex) {
+                const uint32_t count = g.isums[g.img0 + img];
+                scale *= (float)(1.0 / (double)count);
+                if (g.count_sums && r == 0 && t == 0 && lane < 32)
+                    g.count_sums[g.img0 + img] = (double)count;
+            }
+            float2* ob = g.out + img * g.img_stride + r;
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int nn = n_base + 32 * s + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-                if (nn >= g.n) continue;
-                if constexpr (kComplex)
-                    ob[(int64_t)nn * g.n_stride] =
-                        make_float2(cre[s][i] * scale, cim[s][i] * scale);
-                else
-                    store_stream(&ob[(int64_t)nn * g.n_stride], make_float2(cre[s][i] * scale, 0.f));
+                const int j = 32 * t + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                float2 up, dn;  // outputs h + j, h - j
+                if constexpr (kComplex) {
+                    up = make_float2((p0[i] - q1[i]) * scale, (p1[i] + q0[i]) * scale);
+                    dn = make_float2((p0[i] + q1[i]) * scale, (p1[i] - q0[i]) * scale);
+                } else {
+                    const float p = mt ? p1[i] : p0[i], q = mt ? q1[i] : q0[i];
+                    up = make_float2((p - q) * scale, 0.f);
+                    dn = make_float2((p + q) * scale, 0.f);
+                }
+                float2* pu = &ob[(int64_t)(g.h + j) * g.n_stride];
+                float2* pd = &ob[(int64_t)(g.h - j) * g.n_stride];
+                if constexpr (kComplex) {
+                    if (j < g.h) *pu = up;
+                    if (j > 0 && j <= g.h) *pd = dn;
+                } else {
+                    if (j < g.h) store_stream(pu, up);
+                    if (j > 0 && j <= g.h) store_stream(pd, dn);
+                }
             }
         }
     }
 }
 
 static int pad16(int k) { return (k + 15) / 16 * 16; }
-static int pad64(int n) { return (n + 63) / 64 * 64; }
+static int dft_tiles(int n) { return (n / 2 + 1 + 31) / 32; }
 
 int dft_inter_stride(int n) { return pad16(n / 2 + 1); }
 
-constexpr int kGemmLdsMax = 160 * 1024;
+constexpr int kGemmLdsMax = 160 * 1024 - 1024;  // beside the row maxima
 
-// LDS of a workgroup holding NS = 32 * nsub rows of D.
-static size_t gemm_lds(int k_pad, int nsub) {
-    return sizeof(uint16_t) * kDftPlanes * (size_t)(32 * nsub) * dft_lds_ld(k_pad);
-}
-
-template <int kPrec, bool kComplex>
-static void gemm_kernels(const void* (&k)[2]) {
-    k[0] = (const void*)k_dft_gemm<kPrec, kComplex, 1>;
-    k[1] = (const void*)k_dft_gemm<kPrec, kComplex, 2>;
-}
+static size_t gemm_lds(int k_pad) { return (size_t)8 * (k_pad / 8) * kOctetStride; }
 
 hipError_t set_dft_kernel_attributes() {
-    const void* ks[8][2];
-    gemm_kernels<kDftBf16, true>(ks[0]);
-    gemm_kernels<kDftBf16, false>(ks[1]);
-    gemm_kernels<kDftFp16, true>(ks[2]);
-    gemm_kernels<kDftFp16, false>(ks[3]);
-    for (int i = 0; i < 4; i++)
-        for (int j = 0; j < 2; j++) {
-            const hipError_t e = hipFuncSetAttribute(
-                ks[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, kGemmLdsMax);
-            if (e != hipSuccess) return e;
-        }
+    const void* ks[] = {(const void*)k_dft_gemm<kDftBf16, true>,
+                        (const void*)k_dft_gemm<kDftBf16, false>,
+                        (const void*)k_dft_gemm<kDftFp16, true>,
+                        (const void*)k_dft_gemm<kDftFp16, false>};
+    for (const void* k : ks) {
+        const hipError_t e =
+            hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kGemmLdsMax);
+        if (e != hipSuccess) return e;
+    }
     return hipSuccess;
 }
 
+// One wave per 32-row matrix tile: 3 at N = 180, and 9, with 144 KB of LDS, at
+// the largest side.
 template <bool kComplex>
 static hipError_t launch_gemm(const DftGemmArgs& g, int prec, hipStream_t stream) {
     if (g.m_rows == 0) return hipSuccess;
-    // two D tiles per wave when the slice fits, else one
-    const int nsub = (g.n_pad % 64 == 0 && gemm_lds(g.k_pad, 2) <= (size_t)kGemmLdsMax) ? 2 : 1;
-    const size_t lds = gemm_lds(g.k_pad, nsub);
-    if (lds > (size_t)kGemmLdsMax) return hipErrorInvalidConfiguration;
-    const int n_cu = device_cu_count();
-    const int n_slices = g.n_pad / (32 * nsub);
-    const int64_t m_tiles = (g.m_rows + kGemmRows - 1) / kGemmRows;
-    const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(2, kGemmLdsMax / lds));
-    const int64_t want = (n_cu * per_cu + n_slices - 1) / n_slices;  // workgroups per slice
-    const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(m_tiles, want));
-    const int64_t blocks = groups * n_slices;
-    if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-    const dim3 grid((unsigned)blocks), block(kGemmThreads);
-    if (prec == kDftFp16) {
-        if (nsub == 2)
-            hipLaunchKernelGGL((k_dft_gemm<kDftFp16, kComplex, 2>), grid, block, lds, stream, g);
-        else
-            hipLaunchKernelGGL((k_dft_gemm<kDftFp16, kComplex, 1>), grid, block, lds, stream, g);
-    } else {
-        if (nsub == 2)
-            hipLaunchKernelGGL((k_dft_gemm<kDftBf16, kComplex, 2>), grid, block, lds, stream, g);
-        else
-            hipLaunchKernelGGL((k_dft_gemm<kDftBf16, kComplex, 1>), grid, block, lds, stream, g);
-    }
+    const size_t lds = gemm_lds(g.k_pad);
+    constexpr int kRows = kComplex ? 32 : 64;
+    const int64_t blocks = (g.m_rows + kRows - 1) / kRows;
+    if (lds > (size_t)kGemmLdsMax || g.n_tiles > kDftMaxTiles || blocks > 0x7fffffff)
+        return hipErrorInvalidConfiguration;
+    const dim3 grid((unsigned)blocks), block(64 * std::max(2, g.n_tiles));
+    if (prec == kDftFp16)
+        hipLaunchKernelGGL((k_dft_gemm<kDftFp16, kComplex>), grid, block, lds, stream, g);
+    else
+        hipLaunchKernelGGL((k_dft_gemm<kDftBf16, kComplex>), grid, block, lds, stream, g);
     return hipGetLastError();
 }
 
@@ -329,10 +405,10 @@ hipError_t launch_dft_rows(const float* half, const uint16_t* planes1, float* in
     g.a = (const float2*)half;
     g.lda = n;
     g.m_rows = n_img * (h + 1);
-    g.K = n;
-    g.k_pad = pad16(n);
     g.n = n;
-    g.n_pad = pad64(n);
+    g.h = h;
+    g.k_pad = pad16(h + 1);
+    g.n_tiles = dft_tiles(n);
     g.planes = planes1;
     g.R = h + 1;
     g.n_stride = dft_inter_stride(n);
@@ -349,10 +425,10 @@ hipError_t launch_dft_cols(const float* inter, const uint16_t* planes2, float* i
     g.a = (const float2*)inter;
     g.lda = dft_inter_stride(n);
     g.m_rows = n_img * n;
-    g.K = h + 1;
-    g.k_pad = pad16(h + 1);
     g.n = n;
-    g.n_pad = pad64(n);
+    g.h = h;
+    g.k_pad = pad16(h + 1);
+    g.n_tiles = dft_tiles(n);
     g.planes = planes2;
     g.R = n;
     g.n_stride = n;
@@ -364,8 +440,8 @@ hipError_t launch_dft_cols(const float* inter, const uint16_t* planes2, float* i
     return launch_gemm<false>(g, prec, stream);
 }
 
-// Host: the split planes of D1 (stage 1) or D2 (stage 2) in double, rounded
-// to nearest even; zero padding beyond N rows and K columns.
+// Host: rows j = 0 .. H of the matrix exp(+2 pi i j k / N), k = 0 .. H, times
+// w_k in stage 2, in double, rounded to nearest even; zero in the padding.
 static uint16_t bf16_bits(double v) {
     float f = (float)v;
     uint32_t u;
@@ -394,32 +470,26 @@ static double fp16_value(uint16_t b) {
 
 void make_dft_planes(int n, int stage, int prec, std::vector<uint16_t>& planes) {
     const int h = n / 2;
-    const int K = stage == 1 ? n : h + 1;
-    const int k_pad = pad16(K), n_pad = pad64(n);
-    const size_t plane = (size_t)n_pad * k_pad;
-    planes.assign(kDftPlanes * plane, 0);
+    const int n_ks = pad16(h + 1) / 16;
+    planes.assign((size_t)dft_tiles(n) * n_ks * kDftPlanes * 512, 0);
     auto bits = [&](double v) { return prec == kDftFp16 ? fp16_bits(v) : bf16_bits(v); };
     auto value = [&](uint16_t b) { return prec == kDftFp16 ? fp16_value(b) : bf16_value(b); };
-    for (int r = 0; r < n; r++) {
-        const int pr = r < h ? r + h : r - h;  // fftshift: output r takes frequency index pr
-        for (int k = 0; k < K; k++) {
-            const long long idx = ((long long)k * pr) % n;
+    for (int j = 0; j <= h; j++) {
+        for (int k = 0; k <= h; k++) {
+            const long long idx = ((long long)k * j) % n;
             const double a = 2.0 * M_PI * (double)idx / (double)n;
             const double w = (stage == 1 || k == 0 || k == h) ? 1.0 : 2.0;
             const double c = w * std::cos(a), s = w * std::sin(a);
             const uint16_t ch = bits(c), sh = bits(s);
-            const size_t at = (size_t)r * k_pad + k;
-            planes[kReHi * plane + at] = ch;
-            planes[kReLo * plane + at] = bits(c - value(ch));
-            planes[kImHi * plane + at] = sh;
-            planes[kImLo * plane + at] = bits(s - value(sh));
+            const int lane = j % 32 + 32 * (k % 16 / 8);
+            uint16_t* at = planes.data() +
+                           ((size_t)(j / 32) * n_ks + k / 16) * (kDftPlanes * 512) + lane * 8 + k % 8;
+            at[kReHi * 512] = ch;
+            at[kReLo * 512] = bits(c - value(ch));
+            at[kImHi * 512] = sh;
+            at[kImLo * 512] = bits(s - value(sh));
         }
     }
-}
-
-size_t dft_planes_bytes(int n, int stage) {
-    const int K = stage == 1 ? n : n / 2 + 1;
-    return sizeof(uint16_t) * kDftPlanes * (size_t)pad64(n) * pad16(K);
 }
 
 }  // namespace blink

@@ -233,11 +233,10 @@ hipError_t launch_dft_rows(const float* half, const uint16_t* planes1, float* in
 hipError_t launch_dft_cols(const float* inter, const uint16_t* planes2, float* images, int n,
                            int64_t n_img, int64_t img0, const uint32_t* isums,
                            double* count_sums, int prec, hipStream_t stream);
-// Allows the DFT kernels' LDS-resident matrix slices (up to 160 KiB).
+// Allows the DFT kernels' LDS-resident data rows (up to 159 KiB).
 hipError_t set_dft_kernel_attributes();
 // Split planes of D1 (stage 1) or D2 (stage 2) for side n and precision prec.
 void make_dft_planes(int n, int stage, int prec, std::vector<uint16_t>& planes);
-size_t dft_planes_bytes(int n, int stage);
 
 // Register-FFT batched kernels (power-of-two sides 128..2048); the row-pass
 // buffer is transposed: inter[img][u][v].

@@ -512,81 +512,79 @@ k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
 }
 
 // Footprints of the rows r0 .. r0 + nr - 1 (grid rows v, or with kSwap grid columns
-// u) accumulated in LDS planes re, im [nr][n].  The workgroup walks the cells
-// of a channel (packed row << 16 | position, `stride` of them) a chunk at a time,
-// queues (baseline, sign) wherever the nearest row of that footprint lies
+// u) accumulated in LDS planes re, im [nr][n].  Each wavefront walks its share of
+// the cells of a channel (packed row << 16 | position, `stride` of them), queues
+// (baseline, sign) in LDS wherever the nearest row of that footprint lies
 // within K / 2 rows (cyclically: a superset of the footprints that reach the
-// rows), and each thread then spreads one queued footprint over those of its
+// rows), and whenever 64 are queued each lane spreads one over those of its
 // rows that are here (a mask, so that the lanes of a wavefront take few
-// turns).  value(bl) gives the visibility; count(row, position) is called once
+// turns).  The queues are the wavefronts' own: no barrier until the cells are
+// through, so that one wavefront's loads and set-up lie under the others'
+// updates.  value(bl) gives the visibility; count(row, position) is called once
 // per gridded nearest cell in the rows.
 // The work is the K x K updates of every footprint.  The cells are FP64 planes:
 // ds_add_f64 costs 21 clocks per wavefront instruction whatever collides, where
 // the footprints of a dense core make compare-and-swaps of FP32 cells retry.
 // kX: largest K whose weights along a row stay in registers; each weight read in
 // the inner loop would be a gather of 64 cache lines per wavefront.
-// Returns the number of footprints queued.
-constexpr int kb_chunk(int nt, int vec) { return nt * 4 * vec; }  // baselines per chunk
-constexpr size_t kb_queue_bytes(int nt, int vec) {
-    return 2 * sizeof(unsigned short) * (size_t)kb_chunk(nt, vec);
-}
-template <int NT, int kVec, int kX, bool kSwap, class Value, class Count>
+// With a queue and barriers for the whole workgroup, chunk by chunk, 64 x 180^2,
+// K = 7 took 335 us (now 313), 32 x 1024^2 284 (270), 4 x 4096^2 846 (568).
+// The planes must be cleared and visible before, and are complete after the next
+// barrier.  Returns the number of footprints that the wavefront queued.
+constexpr int kKbQueue = 64 + 2 * 2 * 64;  // entries of a wavefront: two cells per lane and walk
+constexpr size_t kb_queue_bytes(int nt) { return sizeof(uint32_t) * (size_t)(nt / 64) * kKbQueue; }
+template <int NT, int kX, bool kSwap, class Value, class Count>
 __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int K,
                                               const double* __restrict__ kt,
                                               const uint32_t* __restrict__ cl, int stride, int r0,
-                                              int nr, double* re, double* im,
-                                              unsigned short* queue, int* n_queued, Value value,
-                                              Count count) {
+                                              int nr, double* re, double* im, uint32_t* queues,
+                                              Value value, Count count) {
 #pragma clang fp contract(off)
-    static_assert(kVec <= 4 && 2 * kb_chunk(NT, kVec) <= 65536, "queue entries: 15-bit offset and a sign");
-    const int n = g.n_pixels, mid = K / 2, tid = threadIdx.x, lane = tid & 63;
+    const int n = g.n_pixels, mid = K / 2, lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    uint32_t* queue = queues + wave * kKbQueue;
     // rows r0 - reach .. r0 + nr - 1 + reach (kb_cell places the negative rows of
     // an odd side one lower than wrap_index does)
     const int reach = mid + (n & 1), span = nr + 2 * reach;
-    auto near = [&](int r) {
-        int d = r - (r0 - reach);
+    auto near = [&](uint32_t r) {
+        int d = (int)r - (r0 - reach);
         d = d < 0 ? d + n : (d >= n ? d - n : d);
         return d < span || span >= n;
     };
-    int total = 0;
-    for (int base = 0; base < stride; base += kb_chunk(NT, kVec)) {
-        if (tid == 0) *n_queued = 0;
-        __syncthreads();
-        unsigned keep = 0;  // two bits per baseline: its own footprint, its conjugate's
-#pragma unroll
-        for (int k = 0; k < kVec; k++) {
-            const int b = base + 4 * (tid + k * NT);
-            const uint4 p = b < stride ? *(const uint4*)&cl[b]
-                                       : make_uint4(kNoCell, kNoCell, kNoCell, kNoCell);
+    auto load = [&](int base) {  // (stride is a multiple of 4)
+        const int b = base + 2 * lane;
+        return b < stride ? *(const uint2*)&cl[b] : make_uint2(kNoCell, kNoCell);
+    };
+    int total = 0, nq = 0;
+    int base = wave * 128;
+    uint2 cur = load(base);
+    for (;; base += 2 * NT) {
+        const bool more = base < stride;
+        if (more) {
+            const uint2 nxt = load(base + 2 * NT);
+            // an entry: baseline * 2, plus 1 for its conjugate's footprint
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const uint32_t c = j == 0 ? p.x : j == 1 ? p.y : j == 2 ? p.z : p.w;
-                if (c == kNoCell) continue;
-                const int r = (int)(c >> 16);
-                if (near(r)) keep |= 1u << (8 * k + 2 * j);
-                if (near(r == 0 ? 0 : n - r)) keep |= 2u << (8 * k + 2 * j);
+                const uint32_t c = j < 2 ? cur.x : cur.y, r = c >> 16;
+                const bool keep = c != kNoCell && near((j & 1) && r ? n - r : r);
+                const unsigned long long m = __ballot(keep);
+                if (keep)
+                    queue[nq + __builtin_amdgcn_mbcnt_hi(
+                                   (unsigned)(m >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
+                        4u * (unsigned)lane + 2u * (unsigned)base + (unsigned)j;
+                nq += __popcll(m);
             }
+            cur = nxt;
         }
-        int before = __popc(keep);
-        const int own = before;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(before, o, 64);
-            if (lane >= o) before += t;
-        }
-        int at = 0;
-        if (lane == 63) at = atomicAdd(n_queued, before);
-        at = __shfl(at, 63, 64) + before - own;
-        while (keep) {
-            const int bit = __ffs(keep) - 1;
-            keep &= keep - 1;
-            queue[at++] = (unsigned short)((4 * (tid + (bit >> 3) * NT) + ((bit >> 1) & 3)) * 2 +
-                                           (bit & 1));
-        }
-        __syncthreads();
-        const int nq = *n_queued;
-        total += nq;
-        for (int i = tid; i < nq; i += NT) {
-            const int q = queue[i], bl = base + (q >> 1), s = (q & 1) ? -1 : 1;
+        team_sync<false>();
+        while (nq >= 64 || (!more && nq)) {
+            const int m = min(nq, 64);
+            nq -= m;
+            total += m;
+            if (lane >= m) continue;
+            const uint32_t q = queue[nq + lane];
+            const int bl = (int)(q >> 1), s = (q & 1) ? -1 : 1;
             const float2 v = value(bl);
             KbSpot sp;
             if (!vis_ok(v) || !kb_spot(g, wl, bl, K, kt, sp)) continue;
@@ -635,62 +633,74 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
                 }
             }
         }
-        __syncthreads();
+        if (!more) return total;
+        team_sync<false>();
     }
-    return total;
 }
 
-// Stage path: workgroup (slab, image) owns `rows` consecutive grid rows; at the
-// end the non-zero cells are added to the global grid (no other workgroup
-// touches them).
-constexpr int kKbThreads = 512, kKbVec = 2;
+// Stage path: workgroup (slab, image) owns `rows` consecutive grid rows of the
+// first `n_rows`; at the end the non-zero cells are added to the global grid (no
+// other workgroup touches them).  n_rows = N, or N / 2 + 1 where every footprint
+// cell of the conjugate is the mirror cell (an even side wider than the kernel):
+// rows N - r are then the conjugates of rows r, added by the same workgroup.
+constexpr int kKbThreads = 512;
 template <int kX>
 __global__ void __launch_bounds__(kKbThreads)
-k_grid_kb_slabs(StageGrid g, int rows, int stride, const uint32_t* __restrict__ cells, int K,
-                const double* __restrict__ kt) {
+k_grid_kb_slabs(StageGrid g, int n_rows, int rows, int stride, const uint32_t* __restrict__ cells,
+                int K, const double* __restrict__ kt) {
     extern __shared__ float4 kb_slabs_lds4[];
     const int n = g.n_pixels;
     double* re = (double*)kb_slabs_lds4;                     // [rows][n]
     double* im = re + (size_t)rows * n;                      // [rows][n]
     unsigned* cnt = (unsigned*)(im + (size_t)rows * n);      // [rows][n]
-    unsigned short* queue = (unsigned short*)(cnt + (size_t)rows * n);
-    __shared__ int n_queued;
-    const int n_slab = (n + rows - 1) / rows;
-    const int r0 = (int)(blockIdx.x % (unsigned)n_slab) * rows, nr = min(rows, n - r0);
+    uint32_t* queues = cnt + (size_t)rows * n;
+    const int n_slab = (n_rows + rows - 1) / rows;
+    const int r0 = (int)(blockIdx.x % (unsigned)n_slab) * rows, nr = min(rows, n_rows - r0);
     const int64_t img = blockIdx.x / (unsigned)n_slab;
     const int tid = threadIdx.x;
     for (int i = tid; i < rows * n; i += kKbThreads) {
         re[i] = im[i] = 0.0;
         cnt[i] = 0u;
     }
-    kb_accumulate<kKbThreads, kKbVec, kX, false>(
+    __syncthreads();
+    kb_accumulate<kKbThreads, kX, false>(
         g, wavelength_of(g.freq_hz[img % g.n_ch]), K, kt, cells + (img % g.n_ch) * stride, stride,
-        r0, nr, re, im, queue, &n_queued, [&](int bl) { return stage_value(g, img, bl); },
+        r0, nr, re, im, queues, [&](int bl) { return stage_value(g, img, bl); },
         [&](int r, int c) { atomicAdd(&cnt[r * n + c], 1u); });
-    float2* grid = g.grids + img * (int64_t)n * n + (int64_t)r0 * n;
-    float* counts = g.counts + img * (int64_t)n * n + (int64_t)r0 * n;
+    __syncthreads();
+    float2* grid = g.grids + img * (int64_t)n * n;
+    float* counts = g.counts + img * (int64_t)n * n;
+    auto add = [&](int64_t at, double x, double y, unsigned k) {
+        if (!(x == 0.0 && y == 0.0)) {
+            const float2 o = grid[at];
+            grid[at] = make_float2((float)((double)o.x + x), (float)((double)o.y + y));
+        }
+        if (k) counts[at] += (float)k;
+    };
     for (int i = tid; i < nr * n; i += kKbThreads) {
         const double x = re[i], y = im[i];
         const unsigned k = cnt[i];
-        if (!(x == 0.0 && y == 0.0)) {
-            const float2 o = grid[i];
-            grid[i] = make_float2((float)((double)o.x + x), (float)((double)o.y + y));
-        }
-        if (k) counts[i] += (float)k;
+        const int r = r0 + i / n, c = i % n;
+        add((int64_t)r * n + c, x, y, k);
+        if (n_rows < n && r != 0 && 2 * r != n)
+            add((int64_t)(n - r) * n + (c ? n - c : 0), x, -y, k);
     }
 }
 
 static size_t kb_slab_lds(int n, int rows) {
-    return (size_t)20 * n * rows + kb_queue_bytes(kKbThreads, kKbVec);
+    return (size_t)20 * n * rows + kb_queue_bytes(kKbThreads);
 }
 
+// Rows to accumulate: see k_grid_kb_slabs.
+static int kb_grid_rows(int n, int K) { return n % 2 == 0 && K < n ? n / 2 + 1 : n; }
 // Rows per slab: up to 8 (the wider, the fewer slabs compute a footprint's
 // weights again), fewer while that leaves under four workgroups per CU or
-// fills more than a third of a CU's LDS.
-static int kb_slab_rows(int n, int64_t n_img) {
+// fills more than a third of a CU's LDS (16 x 256^2, K 7: 4 rows 147 us, 8 rows 161, 16 rows
+// 321).
+static int kb_slab_rows(int n, int K, int64_t n_img) {
     int rows = 8;
     while (rows > 1 && (3 * (int64_t)kb_slab_lds(n, rows) > g_lds_limit ||
-                        n_img * ((n + rows - 1) / rows) < 4 * device_cu_count()))
+                        n_img * ((kb_grid_rows(n, K) + rows - 1) / rows) < 4 * device_cu_count()))
         rows /= 2;
     return rows;
 }
@@ -698,17 +708,18 @@ static int kb_slab_rows(int n, int64_t n_img) {
 // Slabs pay their set-up (clearing, walking the channel's cells, the flush) per
 // workgroup, global atomics 4 K^2 round trips per visibility.  Costs fitted to
 // measurements (us): slabs 20 + 0.022 per workgroup (0.035 where one fills a CU's
-// LDS) + 1.1e-5 per footprint cell, atomics 2.3e-4 per footprint cell.  Measured,
-// atomics -> slabs: 16 x 256^2, 32896 baselines, K 7 4914 -> 287; 1 x 180^2 803 ->
-// 74; 2 x 225^2, K 15 5926 -> 232; 8256 baselines: 4 x 1024^2 349 -> 85, 2 x 4096^2
-// 187 -> 285.
+// LDS) + 1.1e-5 per footprint cell (half with the mirror), atomics 2.3e-4 per
+// footprint cell.  Measured, atomics -> slabs: 16 x 256^2, 32896 baselines, K 7
+// 4914 -> 147; 1 x 180^2 803 -> 75; 2 x 225^2, K 15 5926 -> 231; 8256 baselines:
+// 4 x 1024^2 349 -> 33, 2 x 4096^2 187 -> 177.
 bool kb_grid_slabs(int n, int n_bl, int64_t n_img, int K) {
     if (n > kMaxPixels || n_img == 0) return false;
-    const int rows = kb_slab_rows(n, n_img);
-    const double wgs = (double)n_img * ((n + rows - 1) / rows);
+    const int rows = kb_slab_rows(n, K, n_img);
+    const int n_rows = kb_grid_rows(n, K);
+    const double wgs = (double)n_img * ((n_rows + rows - 1) / rows);
     const double cells = (double)n_img * n_bl * K * K;
     const double per = 2 * (int64_t)kb_slab_lds(n, rows) > g_lds_limit ? 0.035 : 0.022;
-    return 20.0 + per * wgs + 1.1e-5 * cells < 2.3e-4 * cells;
+    return 20.0 + per * wgs + (n_rows < n ? 5.5e-6 : 1.1e-5) * cells < 2.3e-4 * cells;
 }
 
 hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const float* u_m,
@@ -727,9 +738,10 @@ hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const 
                            n_rec, kernel_size, table);
         return hipGetLastError();
     }
-    const int rows = kb_slab_rows(n_pixels, n_img);
+    const int n_rows = kb_grid_rows(n_pixels, kernel_size);
+    const int rows = kb_slab_rows(n_pixels, kernel_size, n_img);
     const size_t lds = kb_slab_lds(n_pixels, rows);
-    const int64_t blocks = n_img * ((n_pixels + rows - 1) / rows);
+    const int64_t blocks = n_img * ((n_rows + rows - 1) / rows);
     if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
     const int stride = (int)stage_cell_stride(n_bl);
     hipLaunchKernelGGL(k_stage_cells, dim3(cell_blocks(stride), (unsigned)std::min(n_ch, 65535)),
@@ -737,8 +749,8 @@ hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const 
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const auto k = kernel_size <= 8 ? k_grid_kb_slabs<8> : k_grid_kb_slabs<0>;
-    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kKbThreads), lds, stream, g, rows, stride,
-                       cells, kernel_size, table);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(kKbThreads), lds, stream, g, n_rows, rows,
+                       stride, cells, kernel_size, table);
     return hipGetLastError();
 }
 
@@ -1588,15 +1600,16 @@ hipError_t launch_kb_cells(const SetDesc* sets, int n_sets, int max_bl, int max_
 // Row pass of convolutional gridding, any side: workgroup (slab, image) owns
 // `rb` consecutive plan rows (grid columns u) of 0 .. N/2, accumulates their
 // footprints in FP64 (kb_accumulate), transforms each row (the planes become
-// the row and its Stockham partner) and writes it, row-major or in the
+// the rows and their twiddles) and writes it, row-major or in the
 // column-blocked layout of the register second pass.  The slabs nearest u = 0,
-// the dense core, are launched first.  It measured, against a gather of plan
-// entries with FP32 cells (and a window of the plane at 256^2) before: 256
-// channels x 256^2, K = 7, 1336 -> see launch_grid_rows_kb.
+// the dense core, are launched first.  Bound by the LDS atomics: the LDS is busy
+// 83 % of the time at 256^2 (20 clocks per wavefront instruction, a third of them
+// bank conflicts).  Against a gather of plan entries with FP32 cells (a window of
+// the plane at 256^2), whole calls: 256 x 256^2, K = 7 1336 -> 820 us, 64 x 180^2
+// 1627 -> 313, 100 x 300^2, K = 9 2973 -> 578, 32 x 1024^2 418 -> 270, 4 x 4096^2
+// 880 -> 568.
 constexpr int kKbRowThreads = 1024;
-// (one row of 8192 cells and the queue of one vector per thread fit a CU)
-constexpr int kb_row_vec(bool wide) { return wide ? 1 : 2; }
-template <int kX, bool kWide, bool kMulti>
+template <int kX, bool kMulti>
 __global__ void __launch_bounds__(kKbRowThreads)
 k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __restrict__ img_set,
                FftPlan plan, int rb, int64_t gi0, int n_img, float2* __restrict__ inter,
@@ -1605,8 +1618,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     const int n = plan.n, h = n / 2, tid = threadIdx.x;
     double* re = (double*)grk_lds4;      // [rb][n]
     double* im = re + (size_t)rb * n;    // [rb][n]
-    unsigned short* queue = (unsigned short*)(im + (size_t)rb * n);
-    __shared__ int n_queued;
+    uint32_t* queues = (uint32_t*)(im + (size_t)rb * n);
     __shared__ int red[kKbRowThreads / 64];
     const int li = (int)(blockIdx.x % (unsigned)n_img);
     const int r0 = (int)(blockIdx.x / (unsigned)n_img) * rb, nr = min(rb, h + 1 - r0);
@@ -1615,6 +1627,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     const GatherArgs& g = sd.g;
     const int img = (int)(gi - sd.img_base), ch = img % g.n_ch;
     for (int i = tid; i < nr * n; i += kKbRowThreads) re[i] = im[i] = 0.0;
+    __syncthreads();
     const StageGrid sg{nullptr, sd.u_m, sd.v_m, sd.flags, g.freq_hz, sd.du, sd.dv, sd.min_uv,
                        g.n_bl, g.n_ch, n, g.pol, nullptr, nullptr};
     const float2* rec = (const float2*)g.vis + 4 * ((int64_t)img * g.n_bl);
@@ -1623,9 +1636,9 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     const int p1 = g.pol == 3 ? 2 : 3;
     const int stride = kb_cell_stride(g.n_bl);
     int n_ok = 0;
-    const int queued = kb_accumulate<kKbRowThreads, kb_row_vec(kWide), kX, true>(
+    const int queued = kb_accumulate<kKbRowThreads, kX, true>(
         sg, wavelength_of(nu), sd.kb_size, sd.kb_table, sd.entries + (int64_t)ch * stride, stride,
-        r0, nr, re, im, queue, &n_queued,
+        r0, nr, re, im, queues,
         [&](int bl) {
             float2 v = select_pol2(rec[4 * (size_t)bl + p0],
                                    g.pol >= 2 ? rec[4 * (size_t)bl + p1] : make_float2(0.f, 0.f),
@@ -1638,6 +1651,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
         [&](int r, int) { n_ok += (r0 + r == 0 || 2 * (r0 + r) == n) ? 1 : 2; });
     const int tot = block_sum_int(n_ok, red);
     if (tid == 0 && tot) atomicAdd(&sd.isums[img], (uint32_t)tot);
+    const bool any = __syncthreads_or(queued);
     // each cell's two sums become one FP32 complex value in its re slot
     for (int i = tid; i < nr * n; i += kKbRowThreads) {
         const float2 c = make_float2((float)re[i], (float)im[i]);
@@ -1645,7 +1659,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     }
     __syncthreads();
     const float2* rows = (float2*)re;
-    if (queued) {  // (uniform) else zeros
+    if (any) {  // (uniform) else zeros
         float2* twl = (float2*)im;  // (rb >= 1 rows of n)
         load_twiddles(twl, tw, n);
         __syncthreads();
@@ -1673,11 +1687,10 @@ hipError_t launch_grid_rows_kb(const SetDesc& first, const SetDesc* sets, const 
     if (n_img == 0) return hipSuccess;
     if (first.kb_size < 1) return hipErrorInvalidValue;
     const int n = plan.n, h1 = n / 2 + 1;
-    const bool wide = n > 1024;
     // as many rows as a CU's LDS holds (the taller the slab, the fewer slabs
     // compute a footprint's weights again), fewer while the images leave under
     // four workgroups per CU (rows above the array's reach have no work)
-    const size_t queue = kb_queue_bytes(kKbRowThreads, kb_row_vec(wide));
+    const size_t queue = kb_queue_bytes(kKbRowThreads);
     int rb = (int)std::min<int64_t>(h1, (g_lds_limit - (int64_t)queue) / (16 * (int64_t)n));
     if (rb < 1) return hipErrorInvalidConfiguration;
     while (rb > 2 && (int64_t)n_img * ((h1 + rb - 1) / rb) < 4 * device_cu_count()) rb = (rb + 1) / 2;
@@ -1687,8 +1700,7 @@ hipError_t launch_grid_rows_kb(const SetDesc& first, const SetDesc* sets, const 
     // (a group's sets share kb_size)
     auto pick = [&](auto kx) {
         constexpr int X = decltype(kx)::value;
-        return wide ? (n_sets > 1 ? k_grid_rows_kb<X, true, true> : k_grid_rows_kb<X, true, false>)
-                    : (n_sets > 1 ? k_grid_rows_kb<X, false, true> : k_grid_rows_kb<X, false, false>);
+        return n_sets > 1 ? k_grid_rows_kb<X, true> : k_grid_rows_kb<X, false>;
     };
     const auto k = first.kb_size <= 8 ? pick(std::integral_constant<int, 8>{})
                                       : pick(std::integral_constant<int, 0>{});
@@ -1841,10 +1853,8 @@ hipError_t set_kernel_attributes() {
     set((const void*)k_grid_kb_slabs<8>);
     set((const void*)k_grid_kb_slabs<0>);
 #define X(K) \
-    set((const void*)k_grid_rows_kb<K, true, true>);  \
-    set((const void*)k_grid_rows_kb<K, true, false>); \
-    set((const void*)k_grid_rows_kb<K, false, true>); \
-    set((const void*)k_grid_rows_kb<K, false, false>);
+    set((const void*)k_grid_rows_kb<K, true>);        \
+    set((const void*)k_grid_rows_kb<K, false>);
     X(8) X(0)
 #undef X
     set((const void*)k_grid_half_rows);

@@ -100,7 +100,7 @@ def test_stage_gridding_adds_to_what_is_there(ctx, n_ant, n_ch, n_t, n, pol, min
 
 @pytest.mark.parametrize("n_ant,n_ch,n,K", [(48, 2, 64, 1), (40, 3, 45, 7), (64, 1, 180, 8), (64, 2, 225, 9),
                                             (96, 5, 256, 7), (24, 1, 16, 31), (200, 1, 61, 16), (10, 1, 1024, 7),
-                                            (128, 2, 1001, 4)])
+                                            (128, 2, 1001, 4), (32, 2, 10, 9), (32, 2, 10, 10), (32, 1, 8, 9)])
 @pytest.mark.parametrize("pol,min_uv", [("XX", -np.inf), ("I", 2.0)])
 def test_stage_footprints_add_to_what_is_there(ctx, n_ant, n_ch, n, K, pol, min_uv):
     """blink_gridding_kernel over its slabs and its atomics (the smallest and sparsest sets), odd and

@@ -972,14 +972,18 @@ static int build_batch(blink_ctx* ctx, const blink_image_set* sets, int n_sets, 
     // and nearest-cell gridding, sets with one timestep per channel (every
     // image has a plan of its own) and dense grids (more than
     // kDirectMinPerRow baselines per plan row); with one workgroup per image,
-    // a group needs images for at least half the CUs, unless it runs beside
-    // the call's main group (one 180^2 image: 0.129 against 0.047 ms on the
-    // plan path).
+    // a group needs images for at least half the CUs (one 180^2 image: 0.129
+    // against 0.044 ms on the plan path), or for an eighth of them where it
+    // runs beside the call's main group (six sides together, direct -> plan:
+    // 4 images of each 278 -> 230 us, 11 371 -> 308, 22 532 -> 519; 43 945 ->
+    // 993, 86 1810 -> 1870).  In a caller's arena, which a plan might not fit,
+    // every group beside the main one.
     std::vector<char> set_direct(n_sets, 0);
     const int64_t cus = device_cu_count();
     for (BatchGroup& g : bp.groups) {
         const bool beside_main = bp.groups.size() > 1 && &g - bp.groups.data() != bp.main;
-        if (bp.direct_mode < 0 && 2 * g.n_img < cus && !beside_main) continue;
+        const int64_t least = !beside_main ? cus / 2 : (arena ? 0 : cus / 8);
+        if (bp.direct_mode < 0 && g.n_img < least) continue;
         // (the DFT transforms' half plane too: the same walk, no row FFT)
         if (g.uniform || bp.direct_mode == 0) continue;
         // convolutional gridding: the windowed direct row pass (256^2) only

@@ -801,13 +801,13 @@ __global__ void __launch_bounds__(kUnitThreads)
 k_plan_count(const SetDesc* __restrict__ sets, const PlanUnit* __restrict__ units, int parts,
              int n_max, int* __restrict__ partial, uint32_t* __restrict__ cells) {
     extern __shared__ int unit_lds[];
-    int* hist = unit_lds;  // [n]
+    int* hist = unit_lds;  // [N/2 + 1]
     const int unit = blockIdx.x / parts, part = blockIdx.x % parts;
     const PlanUnit pu = units[unit];
     const SetDesc sd = sets[pu.set];
-    const int n = sd.n_pixels, n_bl = sd.g.n_bl;
+    const int n = sd.n_pixels, h1 = n / 2 + 1, n_bl = sd.g.n_bl;
     const CellUnit cu(sd.g.freq_hz[pu.ch], sd);
-    for (int i = threadIdx.x; i < n; i += kUnitThreads) hist[i] = 0;
+    for (int i = threadIdx.x; i < h1; i += kUnitThreads) hist[i] = 0;
     __syncthreads();
     int b0, b1;
     part_range(n_bl, parts, part, b0, b1);
@@ -851,33 +851,33 @@ k_plan_count(const SetDesc* __restrict__ sets, const PlanUnit* __restrict__ unit
     }
     __syncthreads();
     int* out = partial + ((int64_t)unit * parts + part) * n_max;
-    for (int i = threadIdx.x; i < n; i += kUnitThreads) out[i] = hist[i];
+    for (int i = threadIdx.x; i < h1; i += kUnitThreads) out[i] = hist[i];
 }
 
 __global__ void __launch_bounds__(kUnitThreads)
 k_plan_scan(const SetDesc* __restrict__ sets, const PlanUnit* __restrict__ units, int parts,
             int n_max, int* __restrict__ partial) {
     extern __shared__ int unit_lds[];
-    int* row_tot = unit_lds;  // [n] entries per row over all parts, then row starts
+    int* row_tot = unit_lds;  // [N/2 + 1] entries per row over all parts, then row starts
     __shared__ int warp_tot[kUnitThreads / 64];
     const int unit = blockIdx.x;
     const PlanUnit pu = units[unit];
     const SetDesc sd = sets[pu.set];
-    const int n = sd.n_pixels;
+    const int n = sd.n_pixels, h1 = n / 2 + 1;
     int* rs = sd.row_start + (int64_t)pu.ch * (n + 1);
     int* base = partial + (int64_t)unit * parts * n_max;
     const int tid = threadIdx.x;
     // row totals: one thread per row, parts summed in order (coalesced reads)
-    for (int i = tid; i < n; i += kUnitThreads) {
+    for (int i = tid; i < h1; i += kUnitThreads) {
         int t = 0;
-#pragma unroll 8
+#pragma unroll 16
         for (int p = 0; p < parts; p++) t += base[(int64_t)p * n_max + i];
         row_tot[i] = t;
     }
     __syncthreads();
     // exclusive scan of the row totals: contiguous chunks per thread
-    const int chunk = (n + kUnitThreads - 1) / kUnitThreads;
-    const int c0 = min(tid * chunk, n), c1 = min(c0 + chunk, n);
+    const int chunk = (h1 + kUnitThreads - 1) / kUnitThreads;
+    const int c0 = min(tid * chunk, h1), c1 = min(c0 + chunk, h1);
     int local = 0;
     for (int i = c0; i < c1; i++) local += row_tot[i];
     int total;
@@ -889,27 +889,26 @@ k_plan_scan(const SetDesc* __restrict__ sets, const PlanUnit* __restrict__ units
     }
     __syncthreads();
     // row starts, and each part's first slot in every row (one thread per row)
-    for (int i = tid; i < n; i += kUnitThreads) {
+    for (int i = tid; i < h1; i += kUnitThreads) {
         int r = row_tot[i];
         rs[i] = r;
-        for (int p0 = 0; p0 < parts; p0 += 8) {
-            int h[8];  // eight independent loads in flight, then the running sums
+        for (int p0 = 0; p0 < parts; p0 += 16) {
+            int h[16];  // independent loads in flight, then the running sums
 #pragma unroll
-            for (int k = 0; k < 8; k++)
+            for (int k = 0; k < 16; k++)
                 h[k] = p0 + k < parts ? base[(int64_t)(p0 + k) * n_max + i] : 0;
 #pragma unroll
-            for (int k = 0; k < 8; k++)
+            for (int k = 0; k < 16; k++)
                 if (p0 + k < parts) {
                     base[(int64_t)(p0 + k) * n_max + i] = r;
                     r += h[k];
                 }
         }
     }
-    if (tid == 0) rs[n] = total;
+    for (int i = h1 + tid; i <= n; i += kUnitThreads) rs[i] = total;  // (not planned)
     // the non-empty rows 0 .. N/2 and their first entries (row_list_len)
-    const int h = n / 2, h1 = h + 1;
     int* rl = sd.row_list + (int64_t)pu.ch * row_list_len(n);
-    auto start = [&](int i) { return i < n ? row_tot[i] : total; };
+    auto start = [&](int i) { return i < h1 ? row_tot[i] : total; };
     const int hc = (h1 + kUnitThreads - 1) / kUnitThreads;
     const int q0 = min(tid * hc, h1), q1 = min(q0 + hc, h1);
     int cnt = 0;
@@ -934,10 +933,10 @@ k_plan_scatter(const SetDesc* __restrict__ sets, const PlanUnit* __restrict__ un
     const int unit = blockIdx.x / parts, part = blockIdx.x % parts;
     const PlanUnit pu = units[unit];
     const SetDesc sd = sets[pu.set];
-    const int n = sd.n_pixels, n_bl = sd.g.n_bl;
-    int* first = unit_lds;            // [n] the part's first global slot per row
-    int* lstart = first + n_max;      // [n] the row's first local slot
-    int* lfill = lstart + n_max;      // [n]
+    const int n = sd.n_pixels, h1 = n / 2 + 1, n_bl = sd.g.n_bl;
+    int* first = unit_lds;            // [h1] the part's first global slot per row
+    int* lstart = first + n_max;      // [h1] the row's first local slot
+    int* lfill = lstart + n_max;      // [h1]
     uint32_t* lent = (uint32_t*)(lfill + n_max);              // [2 kPlanPartMax]
     unsigned short* lrow = (unsigned short*)(lent + 2 * kPlanPartMax);  // [2 kPlanPartMax]
     const int* off = partial + ((int64_t)unit * parts + part) * n_max;
@@ -945,16 +944,17 @@ k_plan_scatter(const SetDesc* __restrict__ sets, const PlanUnit* __restrict__ un
     const int tid = threadIdx.x;
     // the part's count per row is the next part's first slot (or the row
     // end) minus its own; local starts are their exclusive scan
-    const int chunk = (n + kUnitThreads - 1) / kUnitThreads;
-    const int c0 = min(tid * chunk, n), c1 = min(c0 + chunk, n);
-    int local = 0;
-    for (int i = c0; i < c1; i++) {
+    for (int i = tid; i < h1; i += kUnitThreads) {
         const int o = off[i];
         const int e = part + 1 < parts ? off[n_max + i] : rs[i + 1];
         first[i] = o;
         lfill[i] = e - o;  // count, for now
-        local += e - o;
     }
+    __syncthreads();
+    const int chunk = (h1 + kUnitThreads - 1) / kUnitThreads;
+    const int c0 = min(tid * chunk, h1), c1 = min(c0 + chunk, h1);
+    int local = 0;
+    for (int i = c0; i < c1; i++) local += lfill[i];
     int n_local;
     int run = unit_scan(local, warp_tot, &n_local);
     for (int i = c0; i < c1; i++) {

@@ -764,7 +764,10 @@ hipError_t launch_grid_kb(const float* vis, int n_ant, int n_ch, int n_t, const 
 //   scatter  each part sorts its entries by row in LDS and writes them out
 //            as contiguous runs (no FP64 work, no scattered 4-byte stores).
 // Entry order inside a row is not fixed; the sums it feeds are FP32 sums in
-// any order either way.
+// any order either way.  Histograms and slots cover the planned rows 0 .. N/2;
+// the scan is bound by its chains of loads (16 parts of a row in flight: 48
+// channels x 4096^2 25 us, all N rows with 8 in flight 38), the scatter by the
+// part's row counts (22 us; 38 in strided chunks of all rows).
 
 constexpr int kUnitThreads = 512;
 // baselines per thread in a plan part (parts hold at most kPlanPartMax)
@@ -1229,13 +1232,30 @@ hipError_t launch_shift_norm(float* images, int nx, int ny, int n_images, const 
 }
 
 // Mean over images per pixel, summed in image order in FP32
-// (src/gpu/gpu_utils.cpp:143-150; real part only for src/utils.cpp:4-22).
+// (src/gpu/gpu_utils.cpp:143-150; real part only for src/utils.cpp:4-22).  One
+// thread per pixel, kBatch images' loads ahead of their sums: images too small to
+// fill the card with one load per thread are bound by latency (768 x 180^2 197 ->
+// 33 us); large ones by HBM, where the plain loop is faster (24 x 1024^2 30
+// against 35).
+constexpr int64_t kSmallImage = 256 * 1024;
+template <int kBatch>
 __global__ void k_average(const float2* __restrict__ images, int64_t image_size, int n_images,
                           int real_only, float2* __restrict__ out) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < image_size; i += stride) {
         float2 t = images[i];
-        for (int k = 1; k < n_images; k++) {
+        int k = 1;
+        for (; kBatch > 1 && k + kBatch <= n_images; k += kBatch) {
+            float2 v[kBatch];
+#pragma unroll
+            for (int b = 0; b < kBatch; b++) v[b] = images[i + (int64_t)(k + b) * image_size];
+#pragma unroll
+            for (int b = 0; b < kBatch; b++) {
+                t.x += v[b].x;
+                t.y += v[b].y;
+            }
+        }
+        for (; k < n_images; k++) {
             const float2 v = images[i + (int64_t)k * image_size];
             t.x += v.x;
             t.y += v.y;
@@ -1248,8 +1268,11 @@ __global__ void k_average(const float2* __restrict__ images, int64_t image_size,
 hipError_t launch_average(const float* images, int64_t image_size, int n_images, int real_only,
                           float* avg, hipStream_t stream) {
     if (image_size == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_average, dim3(grid_for(image_size, 256, 65536)), dim3(256), 0, stream,
-                       (const float2*)images, image_size, n_images, real_only, (float2*)avg);
+    const bool small = image_size < kSmallImage;
+    const int threads = small ? 64 : 256;
+    hipLaunchKernelGGL(small ? k_average<16> : k_average<1>, dim3(grid_for(image_size, threads, 65536)),
+                       dim3(threads), 0, stream, (const float2*)images, image_size, n_images,
+                       real_only, (float2*)avg);
     return hipGetLastError();
 }
 

@@ -141,6 +141,11 @@ def physical_bytes(kernel: str, o, stats, n_img: int, transform: str = "fft",
       direct_prep    w and the phase coefficient per baseline, the count sums
                      (at 256^2 also u, v, flags for the |u|, |v| maxima)
       fft_cols       the non-empty plan rows (8 N B each) + the image (8 N^2 B)
+      kb_cells, grid_rows_kb
+                     convolutional gridding has no plan: a packed cell (4 B) per
+                     channel and baseline; the row pass reads the cells and the
+                     records (once; a slab of rows each reads them again in cache)
+                     and writes every row 0 .. N/2
       vis_compact    the records (32 B) + the compacted value (8 B) per baseline
       plan           per channel: u, v, flags (12 B) read, the packed cell (4 B)
                      written and read back per baseline, the entries written
@@ -149,13 +154,10 @@ def physical_bytes(kernel: str, o, stats, n_img: int, transform: str = "fft",
       dft_cols       the stage-1 product + the image"""
     n, n_bl = o.n_pixels, o.n_bl
     entries, nonempty = stats
-    window = direct and n == DIRECT_WINDOW_SIDE
-    if kernel_size and not direct:
+    window = direct and n == DIRECT_WINDOW_SIDE and not kernel_size
+    if kernel_size:
         # convolutional gridding writes and reads every plan row 0 .. N/2
         nonempty = np.full_like(nonempty, n // 2 + 1)
-    elif kernel_size:
-        # on the direct row pass, the rows up to the last cell's plus K/2
-        nonempty = np.minimum(nonempty + kernel_size // 2, n // 2 + 1)
     ch = np.arange(n_img) % o.n_ch
     e_sum = float(entries[ch].sum())
     r_sum = float(nonempty[ch].sum())
@@ -163,15 +165,15 @@ def physical_bytes(kernel: str, o, stats, n_img: int, transform: str = "fft",
     pad = -(-h1 // 16) * 16
     if kernel == "grid_rows_fft" and direct:
         return 12.0 * n_bl + 32.0 * n_bl * n_img + 8.0 * n * r_sum
-    if kernel == "direct_prep":
+    if kernel == "direct_prep" or (kernel == "plan" and kernel_size):
         return (24.0 if window else 12.0) * n_bl + 4.0 * n_img
     if kernel == "grid_rows_fft":
         vis_b = 8.0 if compacted(n_bl, n) else 32.0
         return 4.0 * e_sum + vis_b * n_bl * n_img + 8.0 * n * r_sum
-    if kernel == "grid_rows_kb" and direct:   # u, v, flags and records once, the rows
-        return 12.0 * n_bl + 32.0 * n_bl * n_img + 8.0 * n * r_sum
-    if kernel == "grid_rows_kb":   # entries and records once (a lower bound), every row
-        return 4.0 * e_sum + 32.0 * n_bl * n_img + 8.0 * n * r_sum
+    if kernel == "kb_cells":       # u, v, flags once, a packed cell per channel and baseline
+        return 12.0 * n_bl + 4.0 * n_bl * o.n_ch
+    if kernel == "grid_rows_kb":   # cells and records once (a lower bound), every row
+        return 4.0 * n_bl * min(n_img, o.n_ch) + 32.0 * n_bl * n_img + 8.0 * n * r_sum
     if kernel == "fft_cols":
         return 8.0 * n * r_sum + 8.0 * n * n * n_img
     if kernel == "vis_compact":
@@ -194,16 +196,17 @@ def dft_flops(kernel: str, n_pix: int, n_img: int):
                 useful 8 (H+1) N^2, executed 12 split real products;
       dft_cols: real part of N rows times the (H+1) x N matrix per image,
                 useful 4 (H+1) N^2, executed 6 split real products;
-    executed flops count every MFMA over the padded tile grid (m in tiles of
-    256, n of 64, k of 16)."""
+    executed flops count every MFMA over the padded tile grid of the folded
+    products (matrix rows 0 .. H in tiles of 32, H + 1 columns in steps of 16, data
+    rows in tiles of 32 and 64), so useful exceeds executed."""
     h1 = n_pix // 2 + 1
-    n_pad = -(-n_pix // 64) * 64
+    n_pad = -(-h1 // 32) * 32
     if kernel == "dft_rows":
-        m, k, terms, useful = n_img * h1, n_pix, 12, 8.0 * h1 * n_pix * n_pix * n_img
+        m, tile, terms, useful = n_img * h1, 32, 12, 8.0 * h1 * n_pix * n_pix * n_img
     else:
-        m, k, terms, useful = n_img * n_pix, h1, 6, 4.0 * h1 * n_pix * n_pix * n_img
-    m_pad = -(-m // 256) * 256
-    k_pad = -(-k // 16) * 16
+        m, tile, terms, useful = n_img * n_pix, 64, 6, 4.0 * h1 * n_pix * n_pix * n_img
+    m_pad = -(-m // tile) * tile
+    k_pad = -(-h1 // 16) * 16
     executed = terms * 2.0 * m_pad * n_pad * k_pad
     return useful, executed
 
@@ -576,7 +579,8 @@ def main():
                     "useful_flops_per_launch": useful,
                     "useful_tflops": useful / avg_s / 1e12,
                     "note": f"dense {prec} MFMA peak; executed = 3 split terms x 4 (dft_rows) "
-                            "or 2 (dft_cols) real products over padded tiles"}
+                            "or 2 (dft_cols) real products over padded tiles of the "
+                            "folded matrix"}
         else:
             phys = physical_bytes(dom, obs, stats, imgs_per_launch, args.transform,
                                   args.kernel_size, direct)
@@ -622,7 +626,8 @@ def main():
         for k, v in kernels.items():
             if k == "plan":   # no plan units on the direct path: an empty launch
                 b = 0.0 if direct else \
-                    v["launches_per_step"] * physical_bytes(k, obs, stats, obs.n_ch)
+                    v["launches_per_step"] * physical_bytes(k, obs, stats, obs.n_ch,
+                                                            kernel_size=args.kernel_size)
             else:
                 b = physical_bytes(k, obs, stats, job["images_per_step"], args.transform,
                                    args.kernel_size, direct)

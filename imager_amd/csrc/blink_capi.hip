@@ -986,7 +986,8 @@ static int build_batch(blink_ctx* ctx, const blink_image_set* sets, int n_sets, 
         if (bp.direct_mode < 0 && g.n_img < least) continue;
         // (the DFT transforms' half plane too: the same walk, no row FFT)
         if (g.uniform || bp.direct_mode == 0) continue;
-        // convolutional gridding: the windowed direct row pass (256^2) only
+        // convolutional gridding never has a plan (below): at 256^2 its set-up
+        // launch only goes by the direct row pass's name in the profile
         if (g.kb_size && !(g.kb_blocked && direct_uses_window(g.n))) continue;
         if (is_dft(g.transform) ? !direct_half_plane_fits(g.n) : !direct_row_pass_fits(g.n))
             continue;

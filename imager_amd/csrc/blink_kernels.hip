@@ -1279,7 +1279,7 @@ hipError_t launch_average(const float* images, int64_t image_size, int n_images,
 // ------------------------------------- batched: gridding fused with row FFT
 
 // Workgroup = (tile of RB rows, image).  Plan entries of the tile are
-// gathered (pol, phase correction, NaN/MAX_VIS), accumulated with LDS atomics
+// gathered (pol, phase correction, NaN/MAX_VIS), accumulated with lds_add
 // into the tile, each non-empty row is transformed in LDS and written to the
 // row-pass buffer `inter` (image index relative to the chunk).  Empty rows are
 // not written: the column pass reads the plan and treats them as zero.  The

@@ -439,7 +439,6 @@ hipError_t launch_stage_grid(const float* vis, int n_ant, int n_ch, int n_t, con
     const int64_t blocks = n_img * S;
     if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
     const int stride = (int)stage_cell_stride(n_bl);
-    if (!lds_fits(lds) || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(k_stage_cells, dim3(cell_blocks(stride), (unsigned)std::min(n_ch, 65535)),
                        dim3(256), 0, stream, g, stride, cells);
     const hipError_t e = hipGetLastError();
@@ -715,6 +714,7 @@ static int kb_slab_rows(int n, int K, int64_t n_img) {
 bool kb_grid_slabs(int n, int n_bl, int64_t n_img, int K) {
     if (n > kMaxPixels || n_img == 0) return false;
     const int rows = kb_slab_rows(n, K, n_img);
+    if (!lds_fits(kb_slab_lds(n, rows))) return false;  // one row and the queues: N > 7475
     const int n_rows = kb_grid_rows(n, K);
     const double wgs = (double)n_img * ((n_rows + rows - 1) / rows);
     const double cells = (double)n_img * n_bl * K * K;

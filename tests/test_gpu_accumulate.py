@@ -126,3 +126,26 @@ def test_stage_footprints_add_to_what_is_there(ctx, n_ant, n_ch, n, K, pol, min_
     big = float(np.nanmax(np.abs(o.vis))) * max(weight, 1.0)
     terms = 4.0 * o.n_bl
     assert np.abs(grids.cpu().numpy() - want).max() <= terms * 2.0 ** -24 * (big + 10.0)
+
+
+@pytest.mark.parametrize("n", [7392, 7488, 8192])
+def test_stage_footprints_of_the_largest_sides(ctx, n):
+    """Sides around the largest whose row of cells and queues fit in LDS (7475), with a set
+    dense enough that slabs would pay on either.  Counts exact; sums within the bound of an FP32 sum."""
+    import torch
+    K = 31
+    o = synth.small(n_ant=72, n_ch=1, n_t=1, n_pixels=n, seed=n)
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.flags, o.freq)]
+    ref, cref, _ = oracle.gridding(o.vis, o.n_ant, o.u, o.v, o.flags, o.freq, o.delta_u, o.delta_v,
+                                   o.min_uv, n, "XX", precision="f64", kernel_size=K, with_sinc=True)
+    grids = torch.zeros((1, 1, n, n), dtype=torch.complex64, device="cuda")
+    counts = torch.zeros((1, 1, n, n), device="cuda")
+    ctx.gridding_kernel(d[0], o.n_ant, 1, 1, d[1], d[2], d[3], d[4], o.delta_u, o.delta_v,
+                        o.min_uv, n, "XX", 0, K, grids, counts)
+    torch.cuda.synchronize()
+    assert np.array_equal(counts.cpu().numpy(), cref)
+    weight = float(np.abs(oracle.kb_kernels(K)).max()) ** 2
+    big = float(np.abs(o.vis).max()) * max(weight, 1.0)
+    # a cell sees the footprints of at most n_bl visibilities and their conjugates
+    err = np.abs(grids.cpu().numpy() - ref).max()
+    assert err <= 2.0 * o.n_bl * 2.0 ** -24 * 2.0 * o.n_bl * big

@@ -247,6 +247,22 @@ int ctx_scratch(blink_ctx* ctx, const char* name, size_t bytes, void** out) {
     return BLINK_OK;
 }
 
+// Cells of the stage gridding's slabs.  Null, for the atomics, where a capture
+// would have to allocate them.
+int grid_cells(blink_ctx* ctx, int n_ch, int n_bl, hipStream_t s, uint32_t** out) {
+    const size_t bytes = sizeof(uint32_t) * (size_t)n_ch * stage_cell_stride(n_bl);
+    *out = nullptr;
+    if (ctx->scratch["grid_cells"].bytes < bytes) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(s, &st));
+        if (st != hipStreamCaptureStatusNone) return BLINK_OK;
+    }
+    void* p;
+    const int rc = ctx_scratch(ctx, "grid_cells", bytes, &p);
+    if (!rc) *out = (uint32_t*)p;
+    return rc;
+}
+
 // tw[m] = exp(+2 pi i m / N), m < N, computed in double, rounded to FP32;
 // followed by lo[j] = tw[j] and hi[j] = exp(+2 pi i 64 j / N), j < 64 (the
 // two-level tables of the N = 4096 kernels).
@@ -535,14 +551,13 @@ BLINK_API int blink_gridding(blink_ctx* ctx, const float* vis, int n_ant, int n_
     hipStream_t s = (hipStream_t)stream;
     const int n_bl = n_ant * (n_ant + 1) / 2;
     const int64_t n_img = (int64_t)n_ch * n_t;
-    const bool slabs = algo == BLINK_GRID_TILED && stage_grid_slabs(n_pixels, n_bl, n_img);
-    void* cells = nullptr;
-    if (slabs && (rc = ctx_scratch(ctx, "grid_cells",
-                                   sizeof(uint32_t) * (size_t)n_ch * stage_cell_stride(n_bl), &cells)))
+    uint32_t* cells = nullptr;
+    if (algo == BLINK_GRID_TILED && stage_grid_slabs(n_pixels, n_bl, n_img) &&
+        (rc = grid_cells(ctx, n_ch, n_bl, s, &cells)))
         return rc;
-    LAUNCH(slabs ? "grid_slabs" : "grid_atomic", s,
+    LAUNCH(cells ? "grid_slabs" : "grid_atomic", s,
            launch_stage_grid(vis, n_ant, n_ch, n_t, u_m, v_m, bl_flags, freq_hz, delta_u, delta_v,
-                             min_uv, n_pixels, pol, (uint32_t*)cells, grids, counts, s));
+                             min_uv, n_pixels, pol, cells, grids, counts, s));
     if (weighting == BLINK_WEIGHTING_UNIFORM)
         LAUNCH("uniform_weight", s,
                launch_uniform_weight(grids, counts, (int64_t)n_img * n_pixels * n_pixels, s));
@@ -666,15 +681,13 @@ BLINK_API int blink_gridding_kernel(blink_ctx* ctx, const float* vis, int n_ant,
     if ((rc = kb_table(ctx, kernel_size, kernel_mode, &table))) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int n_bl = n_ant * (n_ant + 1) / 2;
-    void* cells = nullptr;
+    uint32_t* cells = nullptr;
     if (kb_grid_slabs(n_pixels, n_bl, (int64_t)n_ch * n_t, kernel_size) &&
-        (rc = ctx_scratch(ctx, "grid_cells",
-                          sizeof(uint32_t) * (size_t)n_ch * stage_cell_stride(n_bl), &cells)))
+        (rc = grid_cells(ctx, n_ch, n_bl, s, &cells)))
         return rc;
     LAUNCH("grid_kernel", s,
            launch_grid_kb(vis, n_ant, n_ch, n_t, u_m, v_m, bl_flags, freq_hz, delta_u, delta_v,
-                          min_uv, n_pixels, pol, kernel_size, table, (uint32_t*)cells, grids,
-                          counts, s));
+                          min_uv, n_pixels, pol, kernel_size, table, cells, grids, counts, s));
     if (weighting == BLINK_WEIGHTING_UNIFORM)
         LAUNCH("uniform_weight", s,
                launch_uniform_weight(grids, counts, (int64_t)n_ch * n_t * n_pixels * n_pixels, s));
@@ -745,7 +758,9 @@ BLINK_API int blink_image(blink_ctx* ctx, float* grids, float* counts, int n_pix
     // one another on the stream; at most a partial and a mark per row)
     const size_t rows = (size_t)n_pixels * stage_chunk(n_pixels, n_images);
     void* sums;
-    if ((rc = ctx_scratch(ctx, "image_sums", (sizeof(double) + 1) * rows, &sums))) return rc;
+    // (2 MiB hold a chunk of any side from 128: no growth under a later capture)
+    const size_t bytes = std::max<size_t>((sizeof(double) + 1) * rows, 2 << 20);
+    if ((rc = ctx_scratch(ctx, "image_sums", bytes, &sums))) return rc;
     StageFftArgs a{};
     a.in = a.grids = (float2*)grids;
     a.out = (float2*)images;

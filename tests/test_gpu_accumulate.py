@@ -149,3 +149,45 @@ def test_stage_footprints_of_the_largest_sides(ctx, n):
     # a cell sees the footprints of at most n_bl visibilities and their conjugates
     err = np.abs(grids.cpu().numpy() - ref).max()
     assert err <= 2.0 * o.n_bl * 2.0 ** -24 * 2.0 * o.n_bl * big
+
+
+@pytest.mark.parametrize("K", [0, 5])
+def test_stage_gridding_captured_without_scratch(K):
+    """A capture that needs more scratch for the cells than the context holds takes the atomics;
+    replays match the eager call.  Sums within the bound of two FP32 sums in different orders."""
+    import torch
+    from imager_amd import capi
+    ctx = capi.Context()
+    n, o = 64, synth.small(n_ant=64, n_ch=8, n_t=1, n_pixels=64, seed=3)
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.flags, o.freq)]
+    grids = torch.zeros((1, 8, n, n), dtype=torch.complex64, device="cuda")
+    counts = torch.zeros((1, 8, n, n), device="cuda")
+
+    def call(n_ch):
+        args = (d[0], o.n_ant, n_ch, 1, d[1], d[2], d[3], d[4], o.delta_u, o.delta_v, o.min_uv, n, "XX", 0)
+        if K:
+            ctx.gridding_kernel(*args, K, grids, counts)
+        else:
+            ctx.gridding(*args, grids, counts)
+
+    call(1)                       # the kernel table, and cells for one channel at most
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(8)
+    got = []
+    for _ in range(3):
+        grids.zero_()
+        counts.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got.append((grids.cpu().numpy().copy(), counts.cpu().numpy().copy()))
+    grids.zero_()
+    counts.zero_()
+    call(8)                       # eager: may allocate, and take the slabs
+    torch.cuda.synchronize()
+    big = float(np.abs(o.vis).max()) * (float(np.abs(oracle.kb_kernels(K)).max()) ** 2 if K else 1.0)
+    for g, c in got:
+        assert np.array_equal(c, counts.cpu().numpy())
+        terms = 2.0 * o.n_bl
+        assert np.abs(g - grids.cpu().numpy()).max() <= 2.0 * terms * 2.0 ** -24 * terms * big

@@ -528,6 +528,11 @@ k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
 // the inner loop would be a gather of 64 cache lines per wavefront.
 // With a queue and barriers for the whole workgroup, chunk by chunk, 64 x 180^2,
 // K = 7 took 335 us (now 313), 32 x 1024^2 284 (270), 4 x 4096^2 846 (568).
+// `edge` (slabs that also write the mirror rows, see k_grid_kb_slabs; otherwise null):
+// kb_cell keeps the coordinate -N of a footprint, at cell 0, and drops +N, so where a
+// position is +-N only one of a visibility's two footprints has the cell.  Those
+// cells stay out of the planes: edge[0 .. nr), [nr .. 2 nr) sum the real and imaginary
+// parts of position 0 of the rows, and [2 nr .. 4 nr) those of the mirror rows.
 // The planes must be cleared and visible before, and are complete after the next
 // barrier.  Returns the number of footprints that the wavefront queued.
 constexpr int kKbQueue = 64 + 2 * 2 * 64;  // entries of a wavefront: two cells per lane and walk
@@ -536,8 +541,8 @@ template <int NT, int kX, bool kSwap, class Value, class Count>
 __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int K,
                                               const double* __restrict__ kt,
                                               const uint32_t* __restrict__ cl, int stride, int r0,
-                                              int nr, double* re, double* im, uint32_t* queues,
-                                              Value value, Count count) {
+                                              int nr, double* re, double* im, double* edge,
+                                              uint32_t* queues, Value value, Count count) {
 #pragma clang fp contract(off)
     const int n = g.n_pixels, mid = K / 2, lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -592,6 +597,15 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
             const double* ck = kSwap ? sp.yk : sp.xk;
             const int rn = wrap_index(s * rp, n) - r0;
             if ((unsigned)rn < (unsigned)nr) count(rn, wrap_index(s * cp, n));
+            // column ce of the footprint lies at -N (this footprint's own) or at +N (the
+            // other sign's); with `edge`, K < N: one of the two at most
+            int ce = -1;
+            bool own = false;
+            if (edge) {
+                const int c_own = -s * n - (cp - mid), c_other = s * n - (cp - mid);
+                own = (unsigned)c_own < (unsigned)K;
+                if (own || (unsigned)c_other < (unsigned)K) ce = own ? c_own : c_other;
+            }
             double cw[kX > 0 ? kX : 1];
             int cx[kX > 0 ? kX : 1];
             if constexpr (kX > 0) {
@@ -601,7 +615,7 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
                     if (c >= K) continue;
                     cw[c] = ck[c];
                     int x;
-                    if (kb_cell(cp - mid + c, s, n, x)) cx[c] = x;
+                    if (c != ce && kb_cell(cp - mid + c, s, n, x)) cx[c] = x;
                 }
             }
             unsigned hit = 0;  // rows j of the footprint that are here
@@ -627,8 +641,14 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
                 } else {
                     for (int c = 0; c < K; c++) {
                         int x;
-                        if (kb_cell(cp - mid + c, s, n, x)) put(x, ck[c]);
+                        if (c != ce && kb_cell(cp - mid + c, s, n, x)) put(x, ck[c]);
                     }
+                }
+                if (ce >= 0) {
+                    double* e = edge + (own ? 0 : 2 * nr) + (y - r0);
+                    const double w = wr * ck[ce];
+                    atomicAdd(&e[0], (double)v.x * w);
+                    atomicAdd(&e[nr], (double)(own ? s : -s) * (double)v.y * w);
                 }
             }
         }
@@ -639,10 +659,13 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
 
 // Stage path: workgroup (slab, image) owns `rows` consecutive grid rows of the
 // first `n_rows`; at the end the non-zero cells are added to the global grid (no
-// other workgroup touches them).  n_rows = N, or N / 2 + 1 where every footprint
-// cell of the conjugate is the mirror cell (an even side wider than the kernel):
-// rows N - r are then the conjugates of rows r, added by the same workgroup.
-constexpr int kKbThreads = 512;
+// other workgroup touches them).  n_rows = N, or N / 2 + 1 on an even side wider than
+// the kernel: a cell of a footprint and the mirror cell of the conjugate's are
+// then the conjugates of each other, so rows N - r are those of rows r, added by the
+// same workgroup, except where the position is +-N (cells of an undersampled
+// grid), which are summed apart (`edge` of kb_accumulate).  (A row at +-N is row 0,
+// which is not mirrored.)
+constexpr int kKbThreads = 512, kKbSlabRows = 8;  // (rows: the most)
 template <int kX>
 __global__ void __launch_bounds__(kKbThreads)
 k_grid_kb_slabs(StageGrid g, int n_rows, int rows, int stride, const uint32_t* __restrict__ cells,
@@ -653,6 +676,8 @@ k_grid_kb_slabs(StageGrid g, int n_rows, int rows, int stride, const uint32_t* _
     double* im = re + (size_t)rows * n;                      // [rows][n]
     unsigned* cnt = (unsigned*)(im + (size_t)rows * n);      // [rows][n]
     uint32_t* queues = cnt + (size_t)rows * n;
+    __shared__ double edge[4 * kKbSlabRows];                 // [4][nr]
+    const bool mirror = n_rows < n;
     const int n_slab = (n_rows + rows - 1) / rows;
     const int r0 = (int)(blockIdx.x % (unsigned)n_slab) * rows, nr = min(rows, n_rows - r0);
     const int64_t img = blockIdx.x / (unsigned)n_slab;
@@ -661,10 +686,11 @@ k_grid_kb_slabs(StageGrid g, int n_rows, int rows, int stride, const uint32_t* _
         re[i] = im[i] = 0.0;
         cnt[i] = 0u;
     }
+    if (tid < 4 * kKbSlabRows) edge[tid] = 0.0;
     __syncthreads();
     kb_accumulate<kKbThreads, kX, false>(
         g, wavelength_of(g.freq_hz[img % g.n_ch]), K, kt, cells + (img % g.n_ch) * stride, stride,
-        r0, nr, re, im, queues, [&](int bl) { return stage_value(g, img, bl); },
+        r0, nr, re, im, mirror ? edge : nullptr, queues, [&](int bl) { return stage_value(g, img, bl); },
         [&](int r, int c) { atomicAdd(&cnt[r * n + c], 1u); });
     __syncthreads();
     float2* grid = g.grids + img * (int64_t)n * n;
@@ -679,10 +705,13 @@ k_grid_kb_slabs(StageGrid g, int n_rows, int rows, int stride, const uint32_t* _
     for (int i = tid; i < nr * n; i += kKbThreads) {
         const double x = re[i], y = im[i];
         const unsigned k = cnt[i];
-        const int r = r0 + i / n, c = i % n;
-        add((int64_t)r * n + c, x, y, k);
-        if (n_rows < n && r != 0 && 2 * r != n)
-            add((int64_t)(n - r) * n + (c ? n - c : 0), x, -y, k);
+        const int lr = i / n, r = r0 + lr, c = i % n;
+        const double* e = edge + lr;
+        if (c) add((int64_t)r * n + c, x, y, k);
+        else add((int64_t)r * n, x + e[0], y + e[nr], k);
+        if (!mirror || r == 0 || 2 * r == n) continue;
+        if (c) add((int64_t)(n - r) * n + (n - c), x, -y, k);
+        else add((int64_t)(n - r) * n, x + e[2 * nr], e[3 * nr] - y, k);
     }
 }
 
@@ -692,12 +721,12 @@ static size_t kb_slab_lds(int n, int rows) {
 
 // Rows to accumulate: see k_grid_kb_slabs.
 static int kb_grid_rows(int n, int K) { return n % 2 == 0 && K < n ? n / 2 + 1 : n; }
-// Rows per slab: up to 8 (the wider, the fewer slabs compute a footprint's
+// Rows per slab: up to kKbSlabRows (the wider, the fewer slabs compute a footprint's
 // weights again), fewer while that leaves under four workgroups per CU or
 // fills more than a third of a CU's LDS (16 x 256^2, K 7: 4 rows 147 us, 8 rows 161, 16 rows
 // 321).
 static int kb_slab_rows(int n, int K, int64_t n_img) {
-    int rows = 8;
+    int rows = kKbSlabRows;
     while (rows > 1 && (3 * (int64_t)kb_slab_lds(n, rows) > g_lds_limit ||
                         n_img * ((kb_grid_rows(n, K) + rows - 1) / rows) < 4 * device_cu_count()))
         rows /= 2;
@@ -1661,7 +1690,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     int n_ok = 0;
     const int queued = kb_accumulate<kKbRowThreads, kX, true>(
         sg, wavelength_of(nu), sd.kb_size, sd.kb_table, sd.entries + (int64_t)ch * stride, stride,
-        r0, nr, re, im, queues,
+        r0, nr, re, im, nullptr, queues,
         [&](int bl) {
             float2 v = select_pol2(rec[4 * (size_t)bl + p0],
                                    g.pol >= 2 ? rec[4 * (size_t)bl + p1] : make_float2(0.f, 0.f),

@@ -533,11 +533,15 @@ k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
 // position is +-N only one of a visibility's two footprints has the cell.  Those
 // cells stay out of the planes: edge[0 .. nr), [nr .. 2 nr) sum the real and imaginary
 // parts of position 0 of the rows, and [2 nr .. 4 nr) those of the mirror rows.
+// kHerm (rows 0 .. N / 2 of a plane that is imaged as a Hermitian one, for the real part of
+// its image): the Hermitian part of the plane, so that such a cell counts half, at its
+// place and, conjugated, at the mirror cell.  A footprint takes its share of both: half
+// wherever it or the other one has the cell, nothing where neither has.
 // The planes must be cleared and visible before, and are complete after the next
 // barrier.  Returns the number of footprints that the wavefront queued.
 constexpr int kKbQueue = 64 + 2 * 2 * 64;  // entries of a wavefront: two cells per lane and walk
 constexpr size_t kb_queue_bytes(int nt) { return sizeof(uint32_t) * (size_t)(nt / 64) * kKbQueue; }
-template <int NT, int kX, bool kSwap, class Value, class Count>
+template <int NT, int kX, bool kSwap, bool kHerm, class Value, class Count>
 __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int K,
                                               const double* __restrict__ kt,
                                               const uint32_t* __restrict__ cl, int stride, int r0,
@@ -597,14 +601,26 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
             const double* ck = kSwap ? sp.yk : sp.xk;
             const int rn = wrap_index(s * rp, n) - r0;
             if ((unsigned)rn < (unsigned)nr) count(rn, wrap_index(s * cp, n));
-            // column ce of the footprint lies at -N (this footprint's own) or at +N (the
-            // other sign's); with `edge`, K < N: one of the two at most
-            int ce = -1;
-            bool own = false;
-            if (edge) {
-                const int c_own = -s * n - (cp - mid), c_other = s * n - (cp - mid);
-                own = (unsigned)c_own < (unsigned)K;
-                if (own || (unsigned)c_other < (unsigned)K) ce = own ? c_own : c_other;
+            if ((edge || kHerm) && max(abs(cp), kHerm ? abs(rp) : 0) >= n - mid) {
+                // may reach +-N (few do, if any): cell by cell
+                auto in = [&](int p) { return p >= -n && p < n; };
+                auto wrap = [&](int p) { return p < 0 ? p + n : (p == n ? 0 : p); };
+                for (int j = 0; j < K; j++) {
+                    const int py = s * (rp - mid + j), y = wrap(py) - r0;
+                    if (abs(py) > n || (!kHerm && py == n) || (unsigned)y >= (unsigned)nr) continue;
+                    for (int c = 0; c < K; c++) {
+                        const int px = s * (cp - mid + c);
+                        const bool own = in(px) && in(py), other = in(-px) && (!kHerm || in(-py));
+                        if (!own && !other) continue;
+                        const double w = (kHerm && own != other ? 0.5 : 1.0) * (rk[j] * ck[c]);
+                        const double a = (double)v.x * w, b = (double)s * (double)v.y * w;
+                        const bool plane = kHerm || own == other;
+                        const int i = y * n + wrap(px);
+                        atomicAdd(plane ? &re[i] : &edge[(own ? 0 : 2 * nr) + y], a);
+                        atomicAdd(plane ? &im[i] : &edge[(own ? nr : 3 * nr) + y], plane || own ? b : -b);
+                    }
+                }
+                continue;
             }
             double cw[kX > 0 ? kX : 1];
             int cx[kX > 0 ? kX : 1];
@@ -615,7 +631,7 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
                     if (c >= K) continue;
                     cw[c] = ck[c];
                     int x;
-                    if (c != ce && kb_cell(cp - mid + c, s, n, x)) cx[c] = x;
+                    if (kb_cell(cp - mid + c, s, n, x)) cx[c] = x;
                 }
             }
             unsigned hit = 0;  // rows j of the footprint that are here
@@ -641,14 +657,8 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
                 } else {
                     for (int c = 0; c < K; c++) {
                         int x;
-                        if (c != ce && kb_cell(cp - mid + c, s, n, x)) put(x, ck[c]);
+                        if (kb_cell(cp - mid + c, s, n, x)) put(x, ck[c]);
                     }
-                }
-                if (ce >= 0) {
-                    double* e = edge + (own ? 0 : 2 * nr) + (y - r0);
-                    const double w = wr * ck[ce];
-                    atomicAdd(&e[0], (double)v.x * w);
-                    atomicAdd(&e[nr], (double)(own ? s : -s) * (double)v.y * w);
                 }
             }
         }
@@ -688,7 +698,7 @@ k_grid_kb_slabs(StageGrid g, int n_rows, int rows, int stride, const uint32_t* _
     }
     if (tid < 4 * kKbSlabRows) edge[tid] = 0.0;
     __syncthreads();
-    kb_accumulate<kKbThreads, kX, false>(
+    kb_accumulate<kKbThreads, kX, false, false>(
         g, wavelength_of(g.freq_hz[img % g.n_ch]), K, kt, cells + (img % g.n_ch) * stride, stride,
         r0, nr, re, im, mirror ? edge : nullptr, queues, [&](int bl) { return stage_value(g, img, bl); },
         [&](int r, int c) { atomicAdd(&cnt[r * n + c], 1u); });
@@ -1688,7 +1698,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     const int p1 = g.pol == 3 ? 2 : 3;
     const int stride = kb_cell_stride(g.n_bl);
     int n_ok = 0;
-    const int queued = kb_accumulate<kKbRowThreads, kX, true>(
+    const int queued = kb_accumulate<kKbRowThreads, kX, true, true>(
         sg, wavelength_of(nu), sd.kb_size, sd.kb_table, sd.entries + (int64_t)ch * stride, stride,
         r0, nr, re, im, nullptr, queues,
         [&](int bl) {

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "blink_kernels.hpp"
+#include "blink_scratch.hpp"
 
 using namespace blink;
 
@@ -71,6 +72,7 @@ struct blink_ctx {
     std::map<int, uint16_t*> dft_planes;          // (N, stage, precision) -> split DFT planes
     std::map<std::pair<int, int>, double*> kb_tables;  // (size, mode) -> gridding kernels
     std::map<std::string, DeviceBuffer> scratch;  // named grow-only buffers
+    StageBuffer grid_cells, image_sums;           // of the stage calls
     std::map<std::string, GraphEntry> graphs;     // descriptor bytes -> graph
     uint64_t graph_clock = 0;
     hipStream_t capture_stream = nullptr;
@@ -247,19 +249,47 @@ int ctx_scratch(blink_ctx* ctx, const char* name, size_t bytes, void** out) {
     return BLINK_OK;
 }
 
+// Whether a call on `s` becomes part of a caller's graph.  (The null stream cannot be
+// captured.)
+int capturing(blink_ctx* ctx, hipStream_t s, bool* out) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (s) HIP_TRY(hipStreamIsCapturing(s, &st));
+    *out = st != hipStreamCaptureStatusNone;
+    return BLINK_OK;
+}
+
+void free_stage(void* p) {
+    (void)hipDeviceSynchronize();  // queued work may still use it
+    (void)hipFree(p);
+}
+
+// Scratch of a stage call on `s`.  With `eager_only`, null where a capture would
+// have to allocate it.
+int stage_scratch(blink_ctx* ctx, StageBuffer& b, size_t bytes, hipStream_t s, bool eager_only,
+                  void** out) {
+    bool cap;
+    int rc = capturing(ctx, s, &cap);
+    if (rc) return rc;
+    hipError_t e = hipSuccess;
+    *out = b.take(
+        bytes, cap, !(cap && eager_only),
+        [&](size_t n) -> void* {
+            void* p = nullptr;
+            e = hipMalloc(&p, n);
+            return e == hipSuccess ? p : nullptr;
+        },
+        free_stage);
+    HIP_TRY(e);
+    return BLINK_OK;
+}
+
 // Cells of the stage gridding's slabs.  Null, for the atomics, where a capture
 // would have to allocate them.
 int grid_cells(blink_ctx* ctx, int n_ch, int n_bl, hipStream_t s, uint32_t** out) {
     const size_t bytes = sizeof(uint32_t) * (size_t)n_ch * stage_cell_stride(n_bl);
-    *out = nullptr;
-    if (ctx->scratch["grid_cells"].bytes < bytes) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        HIP_TRY(hipStreamIsCapturing(s, &st));
-        if (st != hipStreamCaptureStatusNone) return BLINK_OK;
-    }
     void* p;
-    const int rc = ctx_scratch(ctx, "grid_cells", bytes, &p);
-    if (!rc) *out = (uint32_t*)p;
+    const int rc = stage_scratch(ctx, ctx->grid_cells, bytes, s, true, &p);
+    *out = (uint32_t*)p;
     return rc;
 }
 
@@ -461,6 +491,8 @@ BLINK_API void blink_destroy(blink_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
     blink_release_cache(ctx);
+    ctx->grid_cells.destroy(free_stage);
+    ctx->image_sums.destroy(free_stage);
     for (auto& kv : ctx->twiddles) (void)hipFree(kv.second);
     for (auto& kv : ctx->dft_planes) (void)hipFree(kv.second);
     for (auto& kv : ctx->kb_tables) (void)hipFree(kv.second);
@@ -482,6 +514,8 @@ BLINK_API int blink_release_cache(blink_ctx* ctx) {
     for (auto& kv : ctx->scratch)
         if (kv.second.ptr) (void)hipFree(kv.second.ptr);
     ctx->scratch.clear();
+    ctx->grid_cells.release(free_stage);
+    ctx->image_sums.release(free_stage);
     return BLINK_OK;
 }
 
@@ -760,7 +794,7 @@ BLINK_API int blink_image(blink_ctx* ctx, float* grids, float* counts, int n_pix
     void* sums;
     // (2 MiB hold a chunk of any side from 128: no growth under a later capture)
     const size_t bytes = std::max<size_t>((sizeof(double) + 1) * rows, 2 << 20);
-    if ((rc = ctx_scratch(ctx, "image_sums", bytes, &sums))) return rc;
+    if ((rc = stage_scratch(ctx, ctx->image_sums, bytes, s, false, &sums))) return rc;
     StageFftArgs a{};
     a.in = a.grids = (float2*)grids;
     a.out = (float2*)images;

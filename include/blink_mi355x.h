@@ -26,6 +26,14 @@
  *     graphs.  Contexts are not thread-safe: use one per host thread.  Calls
  *     on one context share its scratch, so they must not run concurrently on
  *     different streams (order them, or use one context per stream).
+ *     The calls of sections (a) to (d) may be captured into a caller's graph
+ *     once a call of the same shape has run eagerly (tables and scratch are
+ *     then there); a replay counts as a call on the context. The scratch that
+ *     a captured call names stays allocated until blink_destroy. Where gridding
+ *     finds too little scratch under capture, the graph holds the global
+ *     atomics instead of the LDS slabs, for good (16 x 256^2 with 7 x 7
+ *     kernels 4914 instead of 147 us, 32 x 225^2 without 239 instead of 41),
+ *     so run the call once before its capture.
  *     blink_image_batch also uses two streams of the context, forked from
  *     and joined back to `stream` within the call: the second stream for the
  *     visibility compaction of sparse sets on sides up to 2048 (beside the
@@ -91,7 +99,7 @@ enum blink_transform {
 /* Gridding algorithm for blink_gridding. */
 enum blink_grid_algo {
     BLINK_GRID_TILED = 0,  /* slabs of the plane privatised in LDS, or atomics where they are
-                              faster (default) */
+                              faster or a capture finds no scratch (default) */
     BLINK_GRID_ATOMIC = 1  /* one thread per visibility, global atomics (plain path) */
 };
 
@@ -322,7 +330,8 @@ BLINK_API int blink_image_batch(blink_ctx* ctx, const blink_image_set* sets, int
 BLINK_API int blink_image_batch_noalloc(blink_ctx* ctx, const blink_image_set* sets, int n_sets,
                                         void* stream);
 
-/* Releases every captured graph and scratch buffer of the context. */
+/* Releases every captured graph and scratch buffer of the context, except the
+ * scratch that stage calls captured into a caller's graph (see the conventions). */
 BLINK_API int blink_release_cache(blink_ctx* ctx);
 
 /* ------------------------------------------------------- measurement hooks */

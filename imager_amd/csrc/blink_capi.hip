@@ -377,15 +377,20 @@ int stage_chunk(int64_t n, int64_t batch) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(batch, kStageChunkBytes / (8 * n * n)));
 }
 
+// Scratch of blink_image: a partial count sum and a mark for every row of a
+// chunk.  One size whatever the call (it cuts the chunks of sides under 95
+// only), so that a capture finds it once any call has run.
+constexpr int64_t kImageSumBytes = 2 << 20, kImageSumRows = kImageSumBytes / (sizeof(double) + 1);
+static_assert(kImageSumRows >= kMaxPixels, "a chunk is one image at least");
+
 // Rows then columns of `batch` arrays, a chunk of them at a time.
-int fft2d(blink_ctx* ctx, StageFftArgs a, const FftPlan& plan, int batch, int sign,
+int fft2d(blink_ctx* ctx, StageFftArgs a, const FftPlan& plan, int batch, int chunk, int sign,
           hipStream_t stream) {
     const int n = plan.n;
     const float* tw;
     int rc = twiddles(ctx, n, &tw);
     if (rc) return rc;
     const int64_t gs = (int64_t)n * n;
-    const int chunk = stage_chunk(n, batch);
     for (int i0 = 0; i0 < batch; i0 += chunk) {
         const int cnt = std::min(chunk, batch - i0);
         LAUNCH("fft_rows", stream, launch_stage_pass(true, a, plan, cnt, sign, tw, stream));
@@ -745,7 +750,7 @@ BLINK_API int blink_fft2d_c2c(blink_ctx* ctx, const float* in, float* out, int n
     StageFftArgs a{};
     a.in = (const float2*)in;
     a.out = (float2*)out;
-    return fft2d(ctx, a, plan, batch, direction, (hipStream_t)stream);
+    return fft2d(ctx, a, plan, batch, stage_chunk(n_pixels, batch), direction, (hipStream_t)stream);
 }
 
 // ------------------------------------------------------------------ (d)
@@ -788,21 +793,18 @@ BLINK_API int blink_image(blink_ctx* ctx, float* grids, float* counts, int n_pix
     if ((rc = check_fft_size(ctx, n_pixels, plan))) return rc;
     if (n_images == 0) return BLINK_OK;
     hipStream_t s = (hipStream_t)stream;
-    // partial count sums and row marks of a chunk's images (the chunks follow
-    // one another on the stream; at most a partial and a mark per row)
-    const size_t rows = (size_t)n_pixels * stage_chunk(n_pixels, n_images);
+    // (the chunks follow one another on the stream)
+    const int chunk = (int)std::min<int64_t>(stage_chunk(n_pixels, n_images), kImageSumRows / n_pixels);
     void* sums;
-    // (2 MiB hold a chunk of any side from 128: no growth under a later capture)
-    const size_t bytes = std::max<size_t>((sizeof(double) + 1) * rows, 2 << 20);
-    if ((rc = stage_scratch(ctx, ctx->image_sums, bytes, s, false, &sums))) return rc;
+    if ((rc = stage_scratch(ctx, ctx->image_sums, kImageSumBytes, s, false, &sums))) return rc;
     StageFftArgs a{};
     a.in = a.grids = (float2*)grids;
     a.out = (float2*)images;
     a.counts = counts;
     a.part = (double*)sums;
-    a.used = (unsigned char*)sums + sizeof(double) * rows;
+    a.used = (unsigned char*)sums + sizeof(double) * kImageSumRows;
     a.clear = zero_grids;
-    return fft2d(ctx, a, plan, n_images, BLINK_FFT_BACKWARD, s);
+    return fft2d(ctx, a, plan, n_images, chunk, BLINK_FFT_BACKWARD, s);
 }
 
 BLINK_API int blink_image_averaging(blink_ctx* ctx, const float* images, int64_t image_size,

@@ -84,3 +84,34 @@ def test_captured_stage_calls_after_larger_ones(K):
             check(8, *small)
         assert all(int((t != 7).sum()) == 0 for t in others)
         del graph
+
+
+def test_captured_images_of_a_small_side():
+    """A capture of thousands of images of a small side, after images of an ordinary side
+    only: the scratch does not grow with the call."""
+    import torch
+    from imager_amd import capi
+    n, batch = 64, 4000
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    grids = torch.view_as_complex(torch.randn((batch, n, n, 2), device="cuda", generator=gen))
+    counts = torch.randint(1, 4, (batch, n, n), device="cuda", generator=gen).float()
+    images = torch.empty_like(grids)
+    want = torch.fft.fftshift(torch.fft.ifft2(grids.to(torch.complex128), norm="forward"), dim=(1, 2))
+    want /= counts.double().sum(dim=(1, 2))[:, None, None]
+    with capi.Context() as ctx:
+        ordinary = torch.ones((1, 128, 128), dtype=torch.complex64, device="cuda")
+        ctx.image(ordinary, torch.ones((1, 128, 128), device="cuda"), 128, 1, torch.empty_like(ordinary))
+        torch.cuda.synchronize()
+        # (the table of a side that blink_create does not prepare)
+        ctx.fft2d_c2c(grids[:1], images[:1], n, 1)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            ctx.image(grids, counts, n, batch, images, zero_grids=False)
+        for replay in range(3):
+            images.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            err = (images - want).abs().amax(dim=(1, 2)) / want.abs().amax(dim=(1, 2))
+            assert float(err.max()) < 1e-5
+        del graph

@@ -1177,8 +1177,13 @@ hipError_t launch_direct_prep(const SetDesc* sets, int n_sets, int max_work,
     if (n_sets == 0 || max_work <= 0) return hipSuccess;
     // (at most kUvMaxParts blocks: one partial maximum each)
     const unsigned blocks = (unsigned)std::min(kUvMaxParts, (max_work + 255) / 256);
-    hipLaunchKernelGGL(k_direct_prep, dim3(blocks, (unsigned)n_sets), dim3(256), 0, stream, sets);
-    return hipGetLastError();
+    for (int s0 = 0; s0 < n_sets; s0 += kMaxGridZ) {
+        hipLaunchKernelGGL(k_direct_prep, dim3(blocks, (unsigned)std::min(n_sets - s0, kMaxGridZ)),
+                           dim3(256), 0, stream, sets + s0);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t set_batch_kernel_attributes() {

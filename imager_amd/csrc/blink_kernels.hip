@@ -1652,11 +1652,15 @@ k_kb_cells(const SetDesc* __restrict__ sets) {
 hipError_t launch_kb_cells(const SetDesc* sets, int n_sets, int max_bl, int max_ch,
                            hipStream_t stream) {
     if (n_sets == 0 || max_bl == 0 || max_ch == 0) return hipSuccess;
-    if (n_sets > 65535) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k_kb_cells,
-                       dim3(cell_blocks(kb_cell_stride(max_bl)), (unsigned)std::min(max_ch, 65535), (unsigned)n_sets),
-                       dim3(256), 0, stream, sets);
-    return hipGetLastError();
+    for (int s0 = 0; s0 < n_sets; s0 += kMaxGridZ) {
+        hipLaunchKernelGGL(k_kb_cells,
+                           dim3(cell_blocks(kb_cell_stride(max_bl)), (unsigned)std::min(max_ch, 65535),
+                                (unsigned)std::min(n_sets - s0, kMaxGridZ)),
+                           dim3(256), 0, stream, sets + s0);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 // Row pass of convolutional gridding, any side: workgroup (slab, image) owns

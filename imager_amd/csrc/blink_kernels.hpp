@@ -14,6 +14,9 @@ namespace blink {
 constexpr int kMaxPixels = 8192;      // largest grid side (plan entries pack positions in 13 bits)
 constexpr int kMaxBaselines = 1 << 18;  // plan packs the baseline in 18 bits
 constexpr int kTileThreads = 256;
+// Blocks of a launch along y or z: launches with a set per block take the sets
+// of a larger group in turn.
+constexpr int kMaxGridZ = 65535;
 // Columns per block of the register kernels' column-blocked row-pass buffer.
 constexpr int kInterBlockCols = 32;
 constexpr int kMaxTileRows = 16;

@@ -31,14 +31,15 @@ BLINK_HOST_DEVICE inline double div_rn(double a, double b, double y) {
 // each within a few rounding errors of a / (w d): |p - q| <= 5.01 * 2^-53
 // |a / (w d)|, under 3e-7 for |p| < 2^29.  When p lies more than 1e-6 from
 // every half-integer, p and q are therefore on the same side of each
-// half-integer and round to the same integer.  Returns false, leaving `out`,
-// when p is within 1e-6 of a half-integer, not finite, or |p| >= 2^29 (about
-// one cell in a million): the caller then takes the two divisions.
+// half-integer and round to the same integer.  Returns false, with any value in
+// `out`, when p is within 1e-6 of a half-integer, not finite, or |p| >= 2^29
+// (about one cell in a million): the caller then takes the two divisions.
 BLINK_HOST_DEVICE inline bool round_quotient_fast(double a, double k, int& out) {
     const double p = a * k, q = std::rint(p);  // p - q is exact
-    out = (int)q;
     // (false for NaN; no short circuit, which would be a branch)
-    return (int)(std::fabs(p - q) < 0.5 - 1e-6) & (int)(std::fabs(q) < 536870912.0);
+    const bool fits = std::fabs(q) < 536870912.0;
+    out = (int)(fits ? q : 0.0);
+    return (int)(std::fabs(p - q) < 0.5 - 1e-6) & (int)fits;
 }
 
 // |x| in (1e-30, 1e30): no quotient, product or remainder of two such values

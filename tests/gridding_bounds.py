@@ -51,8 +51,10 @@ def footprint_sums(o, n, K, with_sinc, value):
 
 
 def assert_within(got, want, terms, sums):
-    """Both components of every cell within (terms + 2) 2^-24 sums."""
+    """Both components of every cell within (terms + 2) 2^-24 sums, which has to be far below
+    the values themselves."""
     bound = (terms + 2.0) * 2.0 ** -24 * sums
+    assert bound.max() < 1e-2 * np.abs(want).max()
     d = got - want
     assert (np.abs(d.real) - bound).max() <= 0.0
     assert (np.abs(d.imag) - bound).max() <= 0.0

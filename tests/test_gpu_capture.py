@@ -86,6 +86,45 @@ def test_captured_stage_calls_after_larger_ones(K):
         del graph
 
 
+@pytest.mark.parametrize("K", [0, 5])
+def test_capture_without_scratch(K):
+    """A capture that would have to allocate the cells of its channels holds the atomics."""
+    import torch
+    from imager_amd import capi
+    o = synth.small(n_ant=200, n_ch=8, n_t=1, n_pixels=N, seed=23 + K)
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.flags, o.freq)]
+    ref, cref, _ = oracle.gridding(o.vis, o.n_ant, o.u, o.v, o.flags, o.freq, o.delta_u, o.delta_v,
+                                   o.min_uv, N, "XX", precision="f64", kernel_size=K, with_sinc=True)
+    terms, sums = footprint_sums(o, N, K, True, o.vis[0, :, :, 0])
+    grids = torch.zeros((8, N, N), dtype=torch.complex64, device="cuda")
+    counts = torch.zeros((8, N, N), device="cuda")
+
+    def call(ctx, n_ch):
+        args = (d[0], o.n_ant, n_ch, 1, d[1], d[2], d[3], d[4], o.delta_u, o.delta_v, o.min_uv, N, "XX", 0)
+        if K:
+            ctx.gridding_kernel(*args, K, grids, counts)
+        else:
+            ctx.gridding(*args, grids, counts)
+
+    with capi.Context() as ctx:
+        call(ctx, 1)                  # the kernel table, and cells for one channel at most
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            call(ctx, 8)
+        for replay in range(4):
+            grids.zero_()
+            counts.zero_()
+            if replay < 3:
+                graph.replay()
+            else:
+                call(ctx, 8)          # eager: allocates, and takes the slabs
+            torch.cuda.synchronize()
+            assert np.array_equal(counts.cpu().numpy(), cref[0])
+            assert_within(grids.cpu().numpy(), ref[0], terms, sums)
+        del graph
+
+
 def test_captured_images_of_a_small_side():
     """A capture of thousands of images of a small side, after images of an ordinary side
     only: the scratch does not grow with the call."""

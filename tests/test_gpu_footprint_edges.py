@@ -69,3 +69,24 @@ def test_batched_footprints_at_the_far_edge(ctx, n_ant, n_ch, n, K):
     assert (got.imag == 0).all()
     err = np.abs(got.real - want).max(axis=(-2, -1)) / np.abs(want).max(axis=(-2, -1))
     assert err.max() < 1e-5
+
+
+@pytest.mark.parametrize("n", [7392, 7475, 7476, 8192])
+def test_stage_footprints_around_the_largest_slab(ctx, n):
+    """Sides around the largest whose row of cells and queues fit in LDS (7475), with a set
+    dense enough for the slabs there."""
+    import torch
+    K = 31
+    o = undersampled(72, 1, n, seed=n, reach=0.6)
+    d = [_dev(a) for a in (o.vis, o.u, o.v, o.flags, o.freq)]
+    ref, cref, _ = oracle.gridding(o.vis, o.n_ant, o.u, o.v, o.flags, o.freq, 1.0, 1.0, o.min_uv,
+                                   n, "XX", precision="f64", kernel_size=K, with_sinc=True)
+    grids = torch.zeros((1, n, n), dtype=torch.complex64, device="cuda")
+    counts = torch.zeros((1, n, n), device="cuda")
+    print(f"footprints around the largest slab: {n}^2", flush=True)
+    ctx.gridding_kernel(d[0], o.n_ant, 1, 1, d[1], d[2], d[3], d[4], 1.0, 1.0, o.min_uv, n, "XX", 0,
+                        K, grids, counts)
+    torch.cuda.synchronize()
+    assert np.array_equal(counts.cpu().numpy(), cref[0])
+    terms, sums = footprint_sums(o, n, K, True, o.vis[0, :, :, 0])
+    assert_within(grids.cpu().numpy(), ref[0], terms, sums)

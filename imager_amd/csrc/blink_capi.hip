@@ -1947,9 +1947,10 @@ BLINK_API int blink_image_batch(blink_ctx* ctx, const blink_image_set* sets, int
                 if (lru == ctx->graphs.end() || g->second.last_use < lru->second.last_use) lru = g;
             }
         if (variants >= kBufferVariants) {
-            GraphEntry moved = lru->second;
+            // (moved, not copied: a descriptor copy that is still queued reads host_blob)
+            GraphEntry moved = std::move(lru->second);
             ctx->graphs.erase(lru);
-            it = ctx->graphs.emplace(key, moved).first;
+            it = ctx->graphs.emplace(key, std::move(moved)).first;
         }
     }
     if (it != ctx->graphs.end()) {

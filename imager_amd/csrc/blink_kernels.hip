@@ -528,7 +528,7 @@ k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
 // the inner loop would be a gather of 64 cache lines per wavefront.
 // With a queue and barriers for the whole workgroup, chunk by chunk, 64 x 180^2,
 // K = 7 took 335 us (now 313), 32 x 1024^2 284 (270), 4 x 4096^2 846 (568).
-// `edge` (slabs that also write the mirror rows, see k_grid_kb_slabs; otherwise null):
+// `mirror` (slabs that also write the mirror rows, see k_grid_kb_slabs):
 // kb_cell keeps the coordinate -N of a footprint, at cell 0, and drops +N, so where a
 // position is +-N only one of a visibility's two footprints has the cell.  Those
 // cells stay out of the planes: edge[0 .. nr), [nr .. 2 nr) sum the real and imaginary
@@ -546,7 +546,7 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
                                               const double* __restrict__ kt,
                                               const uint32_t* __restrict__ cl, int stride, int r0,
                                               int nr, double* re, double* im, double* edge,
-                                              uint32_t* queues, Value value, Count count) {
+                                              bool mirror, uint32_t* queues, Value value, Count count) {
 #pragma clang fp contract(off)
     const int n = g.n_pixels, mid = K / 2, lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -554,6 +554,7 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
     // rows r0 - reach .. r0 + nr - 1 + reach (kb_cell places the negative rows of
     // an odd side one lower than wrap_index does)
     const int reach = mid + (n & 1), span = nr + 2 * reach;
+    const int far = kHerm || mirror ? n - mid : INT_MAX;  // from here on a footprint may reach +-N
     auto near = [&](uint32_t r) {
         int d = (int)r - (r0 - reach);
         d = d < 0 ? d + n : (d >= n ? d - n : d);
@@ -601,8 +602,8 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
             const double* ck = kSwap ? sp.yk : sp.xk;
             const int rn = wrap_index(s * rp, n) - r0;
             if ((unsigned)rn < (unsigned)nr) count(rn, wrap_index(s * cp, n));
-            if ((edge || kHerm) && max(abs(cp), kHerm ? abs(rp) : 0) >= n - mid) {
-                // may reach +-N (few do, if any): cell by cell
+            if ((kHerm ? max(abs(cp), abs(rp)) : abs(cp)) >= far) {
+                // (few, if any): cell by cell
                 auto in = [&](int p) { return p >= -n && p < n; };
                 auto wrap = [&](int p) { return p < 0 ? p + n : (p == n ? 0 : p); };
                 for (int j = 0; j < K; j++) {
@@ -700,7 +701,7 @@ k_grid_kb_slabs(StageGrid g, int n_rows, int rows, int stride, const uint32_t* _
     __syncthreads();
     kb_accumulate<kKbThreads, kX, false, false>(
         g, wavelength_of(g.freq_hz[img % g.n_ch]), K, kt, cells + (img % g.n_ch) * stride, stride,
-        r0, nr, re, im, mirror ? edge : nullptr, queues, [&](int bl) { return stage_value(g, img, bl); },
+        r0, nr, re, im, edge, mirror, queues, [&](int bl) { return stage_value(g, img, bl); },
         [&](int r, int c) { atomicAdd(&cnt[r * n + c], 1u); });
     __syncthreads();
     float2* grid = g.grids + img * (int64_t)n * n;
@@ -1704,7 +1705,7 @@ k_grid_rows_kb(SetDesc first, const SetDesc* __restrict__ sets, const int* __res
     int n_ok = 0;
     const int queued = kb_accumulate<kKbRowThreads, kX, true, true>(
         sg, wavelength_of(nu), sd.kb_size, sd.kb_table, sd.entries + (int64_t)ch * stride, stride,
-        r0, nr, re, im, nullptr, queues,
+        r0, nr, re, im, nullptr, false, queues,
         [&](int bl) {
             float2 v = select_pol2(rec[4 * (size_t)bl + p0],
                                    g.pol >= 2 ? rec[4 * (size_t)bl + p1] : make_float2(0.f, 0.f),

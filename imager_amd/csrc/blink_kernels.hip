@@ -537,6 +537,8 @@ k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
 // its image): the Hermitian part of the plane, so that such a cell counts half, at its
 // place and, conjugated, at the mirror cell.  A footprint takes its share of both: half
 // wherever it or the other one has the cell, nothing where neither has.
+// Both in a second walk, if the first one met a footprint that may reach +-N: in
+// the first one's loop the cases cost all footprints 1 to 4 %.
 // The planes must be cleared and visible before, and are complete after the next
 // barrier.  Returns the number of footprints that the wavefront queued.
 constexpr int kKbQueue = 64 + 2 * 2 * 64;  // entries of a wavefront: two cells per lane and walk
@@ -564,11 +566,11 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
         const int b = base + 2 * lane;
         return b < stride ? *(const uint2*)&cl[b] : make_uint2(kNoCell, kNoCell);
     };
-    int total = 0, nq = 0;
+    int total = 0, nq = 0, seen_far = 0;
     int base = wave * 128;
     uint2 cur = load(base);
-    for (;; base += 2 * NT) {
-        const bool more = base < stride;
+    for (bool more = true; more; base += 2 * NT) {
+        more = base < stride;
         if (more) {
             const uint2 nxt = load(base + 2 * NT);
             // an entry: baseline * 2, plus 1 for its conjugate's footprint
@@ -603,24 +605,7 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
             const int rn = wrap_index(s * rp, n) - r0;
             if ((unsigned)rn < (unsigned)nr) count(rn, wrap_index(s * cp, n));
             if ((kHerm ? max(abs(cp), abs(rp)) : abs(cp)) >= far) {
-                // (few, if any): cell by cell
-                auto in = [&](int p) { return p >= -n && p < n; };
-                auto wrap = [&](int p) { return p < 0 ? p + n : (p == n ? 0 : p); };
-                for (int j = 0; j < K; j++) {
-                    const int py = s * (rp - mid + j), y = wrap(py) - r0;
-                    if (abs(py) > n || (!kHerm && py == n) || (unsigned)y >= (unsigned)nr) continue;
-                    for (int c = 0; c < K; c++) {
-                        const int px = s * (cp - mid + c);
-                        const bool own = in(px) && in(py), other = in(-px) && (!kHerm || in(-py));
-                        if (!own && !other) continue;
-                        const double w = (kHerm && own != other ? 0.5 : 1.0) * (rk[j] * ck[c]);
-                        const double a = (double)v.x * w, b = (double)s * (double)v.y * w;
-                        const bool plane = kHerm || own == other;
-                        const int i = y * n + wrap(px);
-                        atomicAdd(plane ? &re[i] : &edge[(own ? 0 : 2 * nr) + y], a);
-                        atomicAdd(plane ? &im[i] : &edge[(own ? nr : 3 * nr) + y], plane || own ? b : -b);
-                    }
-                }
+                seen_far = 1;
                 continue;
             }
             double cw[kX > 0 ? kX : 1];
@@ -663,9 +648,42 @@ __device__ __forceinline__ int kb_accumulate(const StageGrid& g, double wl, int 
                 }
             }
         }
-        if (!more) return total;
         team_sync<false>();
     }
+    if (!__any(seen_far)) return total;
+    // the far footprints (few, if any), cell by cell
+    auto in = [&](int p) { return p >= -n && p < n; };
+    auto wrap = [&](int p) { return p < 0 ? p + n : (p == n ? 0 : p); };
+    for (base = wave * 128; base < stride; base += 2 * NT) {
+        cur = load(base);
+        for (int e = 0; e < 4; e++) {
+            const uint32_t cell = e < 2 ? cur.x : cur.y, r = cell >> 16;
+            if (cell == kNoCell || !near((e & 1) && r ? n - r : r)) continue;
+            const int bl = base + 2 * lane + (e >> 1), s = (e & 1) ? -1 : 1;
+            const float2 v = value(bl);
+            KbSpot sp;
+            if (!vis_ok(v) || !kb_spot(g, wl, bl, K, kt, sp)) continue;
+            const int rp = kSwap ? sp.up : sp.vp, cp = kSwap ? sp.vp : sp.up;
+            if ((kHerm ? max(abs(cp), abs(rp)) : abs(cp)) < far) continue;
+            for (int j = 0; j < K; j++) {
+                const int py = s * (rp - mid + j), y = wrap(py) - r0;
+                if (abs(py) > n || (!kHerm && py == n) || (unsigned)y >= (unsigned)nr) continue;
+                for (int c = 0; c < K; c++) {
+                    const int px = s * (cp - mid + c);
+                    const bool own = in(px) && in(py), other = in(-px) && (!kHerm || in(-py));
+                    if (!own && !other) continue;
+                    const double w = (kHerm && own != other ? 0.5 : 1.0) *
+                                     (kSwap ? sp.xk[j] * sp.yk[c] : sp.yk[j] * sp.xk[c]);
+                    const double a = (double)v.x * w, b = (double)s * (double)v.y * w;
+                    const bool plane = kHerm || own == other;
+                    const int i = y * n + wrap(px);
+                    atomicAdd(plane ? &re[i] : &edge[(own ? 0 : 2 * nr) + y], a);
+                    atomicAdd(plane ? &im[i] : &edge[(own ? nr : 3 * nr) + y], plane || own ? b : -b);
+                }
+            }
+        }
+    }
+    return total;
 }
 
 // Stage path: workgroup (slab, image) owns `rows` consecutive grid rows of the

@@ -175,9 +175,9 @@ __device__ __forceinline__ float2 select_pol2(float2 x0, float2 x1, int pol) {
 }
 
 // *p += (x, y) in LDS, atomically, in FP32.  gfx950 executes ds_add_f32 at
-// about 3 clocks per LANE, whatever the addresses (193 clocks per wavefront
-// instruction; ds_add_u32 9, ds_add_f64 21, measured with one 1024-thread
-// workgroup per CU), so two of them cost 389 clocks per wavefront.  A 64-bit
+// about 3 clocks per LANE, at random and at consecutive addresses (193 clocks per
+// wavefront instruction; at random ones ds_add_u32 9, ds_add_f64 21, measured with one
+// 1024-thread workgroup per CU), so two of them cost 388 clocks per wavefront.  A 64-bit
 // compare-and-swap of the whole cell costs 46 (79 with a third of the updates
 // in 128 cells) and rounds the same FP32 sums (768 channels x 256^2, 32896
 // baselines: 426 -> 355 us per batched call; 256 channels with 7 x 7

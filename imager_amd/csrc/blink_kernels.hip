@@ -522,8 +522,9 @@ k_grid_kb(StageGrid g, int64_t n_rec, int K, const double* __restrict__ kt) {
 // updates.  value(bl) gives the visibility; count(row, position) is called once
 // per gridded nearest cell in the rows.
 // The work is the K x K updates of every footprint.  The cells are FP64 planes:
-// ds_add_f64 costs 21 clocks per wavefront instruction whatever collides, where
-// the footprints of a dense core make compare-and-swaps of FP32 cells retry.
+// ds_add_f64 costs 21 clocks per wavefront instruction at random cells, also where a
+// third of them fall in a dense core (9 at consecutive ones), where compare-and-swaps
+// of FP32 cells retry.
 // kX: largest K whose weights along a row stay in registers; each weight read in
 // the inner loop would be a gather of 64 cache lines per wavefront.
 // With a queue and barriers for the whole workgroup, chunk by chunk, 64 x 180^2,

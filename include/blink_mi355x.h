@@ -283,7 +283,9 @@ typedef struct blink_image_set {
                                 convolutional gridding, each visibility and its conjugate
                                 spread over kernel_size x kernel_size cells as
                                 blink_gridding_kernel spreads them (FFT transform, natural
-                                weighting) */
+                                weighting).  Where footprints reach the coordinates +-N (cells
+                                of an undersampled plane) that plane is not Hermitian: the
+                                images are then the real part of its transform */
     int kernel_mode;         /* blink_grid_kernel when kernel_size > 0 */
 } blink_image_set;
 
